@@ -95,14 +95,67 @@ def test_values_that_are_not_finite(shape, value):
         assert e <= 2.0 ** -24 * (x.shape[0] * x.shape[1] * x.shape[2]) ** 0.5, (k, e)
 
 
-@pytest.mark.parametrize("scale", [1e-34, 1e-28, 2.0 ** -82], ids=str)
-def test_tiny_values(scale):
-    """All operands of one side so small that the lower bf16 parts are denormal: fp32 keeps their precision."""
+def _slice_error(got, ref):
+    got, ref = np.asarray(got, np.float64), np.asarray(ref, np.float64)
+    return np.linalg.norm(got - ref) / np.linalg.norm(ref)
+
+
+TINY = [2.0 ** -82, 2.0 ** -112, 2.0 ** -119]       # lower bf16 parts of an unscaled number: normal, lost in part, denormal
+TINY_SHAPES = [(64, 33, 32, 8, 96), (50, 9, 11, 24, 44)]
+
+
+@pytest.mark.parametrize("tiny", TINY, ids=str)
+@pytest.mark.parametrize("shape", TINY_SHAPES, ids=str)
+def test_tiny_values(shape, tiny):
+    """All operands of one side so small that the lower parts of an unscaled split are bf16 denormals: fp32 keeps their bits."""
     geom = _geom()
-    for shape in ((64, 33, 32, 8, 96), (50, 9, 11, 24, 44)):
-        x, w, b, go = _inputs(*shape, geom, 5, scale)
-        got, ref = _run(x, w, b, go, geom), _truth(x, w, b, go, geom)
-        _check(got, ref, {"out": w.shape[0], "dx": 9 * shape[4]})
+    x, w, b, go = _inputs(*shape, geom, 5, tiny)
+    rows = x.shape[0] * x.shape[1] * x.shape[2]
+    _check(_run(x, w, b, go, geom), _truth(x, w, b, go, geom), {"out": w.shape[0], "dx": 9 * shape[4]})
+    got = _run(x, w, b, go / np.float32(tiny), geom)
+    _check(got, _truth(x, w, b, go / np.float32(tiny), geom), {"dw": rows})
+
+
+@pytest.mark.parametrize("tiny", TINY, ids=str)
+@pytest.mark.parametrize("shape", TINY_SHAPES, ids=str)
+def test_tiny_times_huge_values(shape, tiny):
+    """Tiny operands against huge ones, with results of ordinary size."""
+    geom = _geom()
+    x, w, b, go = _inputs(*shape, geom, 8)
+    rows = x.shape[0] * x.shape[1] * x.shape[2]
+    t, huge = np.float32(tiny), np.float32(1 / tiny)
+    got = _run(x * t, w * huge, b, go * t, geom)
+    _check(got, _truth(x * t, w * huge, b, go * t, geom), {"out": w.shape[0], "dx": 9 * shape[4]})
+    _check(_run(x * t, w, b, go * huge, geom), _truth(x * t, w, b, go * huge, geom), {"dw": rows})
+
+
+@pytest.mark.parametrize("tiny", TINY, ids=str)
+@pytest.mark.parametrize("shape", TINY_SHAPES, ids=str)
+def test_tiny_values_among_ordinary_ones(shape, tiny):
+    """One tiny sample, filter and channel among ordinary ones, in the same tiles: each keeps the precision of its own."""
+    N, H, W, C, F = shape
+    geom = _geom()
+    x, w, b, go = _inputs(*shape, geom, 9)
+    b[:] = 0
+    t = np.float32(tiny)
+    rows = N * H * W
+    bound = lambda L: 2.0 ** -24 * max(L, 16) ** 0.5
+
+    xs, gs = x.copy(order="F"), go.copy(order="F")
+    xs[3] *= t
+    gs[3] *= t
+    got, ref = _run(xs, w, b, gs, geom), _truth(xs, w, b, gs, geom)
+    assert _slice_error(got["out"][3], ref["out"][3]) <= bound(9 * C)
+    assert _slice_error(got["dx"][3], ref["dx"][3]) <= bound(9 * F)
+
+    xs, ws, gs = x.copy(order="F"), w.copy(order="F"), go.copy(order="F")
+    xs[..., 2] *= t                     # (rows 18 to 26 of the weights and their gradient)
+    ws[:, 5] *= t
+    gs[..., 5] *= t
+    got, ref = _run(xs, ws, b, gs, geom), _truth(xs, ws, b, gs, geom)
+    assert _slice_error(got["out"][..., 5], ref["out"][..., 5]) <= bound(9 * C)
+    assert _slice_error(got["dw"][18:27, :5], ref["dw"][18:27, :5]) <= bound(rows)
+    assert _slice_error(got["dw"][:18, 5], ref["dw"][:18, 5]) <= bound(rows)
 
 
 def test_values_near_the_largest():
