@@ -77,7 +77,6 @@ struct GatherGeom {
 	 * out_sb b)) + out_M f of `out`. Plain (0, 1, 0, 1, OA, M): out is the M x F matrix itself. Otherwise the rows are
 	 * one residue class of the positions of a larger tensor (a strided input gradient computed class by class). */
 	int out_a0, out_sa, out_b0, out_sb, out_OA, out_M;
-	bool fp32_products;     /* ConvShape::fp32_products */
 };
 
 /* Convolution hyper-parameters in the reference's terms (dilation 0 = dense receptor). */

@@ -42,10 +42,10 @@ __device__ __forceinline__ T lane_group_sum(T v) {
 
 /* D rows are filters (row rr of block i is filter FB*rr + i), D columns are m (column lc of block j is row MB*lc + j of the
  * tile), so a lane owns MB adjacent outputs. `stage`: STAGE elements of LDS that the block is done with; bias_s: the tile's
- * bias values. Returns whether the tile is stored; false (EPI_NONE, EPI_STATS): that is left to the caller. */
+ * bias values; mm: the lane's first row of M; vec_out: whether its rows may be stored as vectors. Returns whether the tile is stored; false (EPI_NONE, EPI_STATS): that is left to the caller. */
 template<typename T, int WAVES_M, int WAVES_F, int WT_M, int WT_F, int VEC, int EPI, int STAGE>
 __device__ __forceinline__ bool gather_epilogue(typename Mfma<T>::acc_t (&acc)[WT_F / Mfma<T>::TL][WT_M / Mfma<T>::TL], const GatherGeom& g,
-		const GatherLaunch& L, const Epilogue<T>& E, T* __restrict__ out, const T* bias_s, T* const stage, int tile, int f0) {
+		const GatherLaunch& L, const Epilogue<T>& E, T* __restrict__ out, const T* bias_s, T* const stage, int tile, int f0, int mm, bool vec_out) {
 	typedef Mfma<T> MF;
 	constexpr int THREADS = 64 * WAVES_M * WAVES_F, BM = WAVES_M * WT_M, BF = WAVES_F * WT_F, TL = MF::TL;
 	constexpr int MB = WT_M / TL, FB = WT_F / TL, VS = MB * (int) sizeof(T) > 16 ? 16 / (int) sizeof(T) : MB;
@@ -208,8 +208,6 @@ __device__ __forceinline__ bool gather_epilogue(typename Mfma<T>::acc_t (&acc)[W
 		});
 		return true;
 	}
-	const bool vec_out = g.M % MB == 0 && (reinterpret_cast<uintptr_t>(out) & (VS * sizeof(T) - 1)) == 0;
-	const int mm = tile_row_m(L, g, tile, BM, wm * WT_M + MB * lc);
 	if constexpr (EPI == EPI_ACT) {
 		act_dispatch(E.kind, [&](auto kc) {
 			constexpr int KIND = decltype(kc)::value;

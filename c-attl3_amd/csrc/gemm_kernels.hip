@@ -431,10 +431,10 @@ __device__ __forceinline__ void gather_gemm_body(const T* __restrict__ src, cons
 				lstm_forward_store_vec<T, LV>(E.lstm, lstm_e[gi], res[gi]);
 		return;
 	}
-	if (gather_epilogue<T, WAVES_M, WAVES_F, WT_M, WT_F, VEC, EPI, 2 * KC * LDA>(acc, g, L, E, out, bias_s, &As[0][0][0], tile, f0))
-		return;
 	const bool vec_out = g.M % MB == 0 && (reinterpret_cast<uintptr_t>(out) & (VS * sizeof(T) - 1)) == 0;
 	const int mm = tile_row_m(L, g, tile, BM, wm * WT_M + MB * lc);
+	if (gather_epilogue<T, WAVES_M, WAVES_F, WT_M, WT_F, VEC, EPI, 2 * KC * LDA>(acc, g, L, E, out, bias_s, &As[0][0][0], tile, f0, mm, vec_out))
+		return;
 	/* (the output map: plain except for the residue classes of a strided input gradient, which have no fused epilogue) */
 	const size_t mm_out = EPI == EPI_NONE ? out_row(g, min(mm, g.M - 1)) : (size_t) mm;
 	#pragma unroll
@@ -2063,6 +2063,11 @@ void launch_wave_split_variant(const T* src, const T* wt, const T* bias, T* out,
 	CATTLE_HIP_CHECK(hipGetLastError());
 }
 
+/* A gathered GEMM and what the host alone asks about it (kernels are given the geometry). */
+struct GatherProblem : GatherGeom {
+	bool fp32_products = false;     /* ConvShape::fp32_products */
+};
+
 /* Which tiles of a launch have their reduction cut into parts, and the memory that the parts' sums take. */
 struct CutReductions {
 	bool few_tiles;         /* far fewer tiles than the chip holds blocks */
@@ -2107,7 +2112,7 @@ CutReductions cut_reductions(const GatherVariant<T>& v, const GatherGeom& g, boo
  * `full` microseconds, one alone in `alone`, and a round of blocks ends with `tail` for the stores that nothing overlaps;
  * the figures are fits to the times of forward and input-gradient launches of 30 layers with each tile (per chunk and
  * block, 256 x 128: 802,816 x 576 x 128 in 650 us is 2.6 us; 256 x 64: 802,816 x 1152 x 64 in 750 us, 1.6 us). */
-const GatherVariant<float>* bf16x3_for(const GatherGeom& g, long M, bool no_split) {
+const GatherVariant<float>* bf16x3_for(const GatherProblem& g, long M, bool no_split) {
 	if (g.fp32_products || g.K < 48 || g.F <= 8 || 2.0 * M * g.K * g.F < 3e7 || tuning().no_bf16x3 || !bf16x3_gather_possible(g))
 		return nullptr;
 	const GatherVariant<float>* const vars = bf16x3_variants();
@@ -2150,7 +2155,7 @@ const GatherVariant<float>* bf16x3_for(const GatherGeom& g, long M, bool no_spli
 }
 
 template<typename T>
-bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const GatherGeom& g, ScratchArena* arena = nullptr,
+bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const GatherProblem& g, ScratchArena* arena = nullptr,
 		int epi = EPI_NONE, const Epilogue<T>* E = nullptr, int* mtiles_out = nullptr, const LstmBackwardStep<T>* then = nullptr,
 		bool* then_done = nullptr, const std::function<void(int bf)>* before_launch = nullptr, WgradRider<T>* rider = nullptr) {
 	const bool vec = g.N % GemmCfg<T>::VEC == 0 && g.NS % GemmCfg<T>::VEC == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
@@ -2423,7 +2428,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
  * with. Returns false, having launched nothing, if there are more problems than the table holds, or if 16-byte loads are
  * not possible (`vec`) and the launch would need them. */
 template<typename T>
-bool launch_gather_classes(const T* src, T* out, const std::vector<GatherGeom>& geoms, const std::vector<const T*>& weights, bool vec) {
+bool launch_gather_classes(const T* src, T* out, const std::vector<GatherProblem>& geoms, const std::vector<const T*>& weights, bool vec) {
 	if (geoms.empty())
 		return true;
 	if ((int) geoms.size() > MAX_GATHER_CLASSES)
@@ -2462,7 +2467,7 @@ bool launch_gather_classes(const T* src, T* out, const std::vector<GatherGeom>& 
 		/* all classes or none: each must have a reduction worth it */
 		long M = 0;
 		bool all = true;
-		for (const GatherGeom& g : geoms) {
+		for (const GatherProblem& g : geoms) {
 			M += g.M;
 			all = all && bf16x3_for(g, g.M, true) != nullptr;
 		}
@@ -2511,8 +2516,8 @@ void plain_output(GatherGeom& g) {
 	g.out_M = g.M;
 }
 
-GatherGeom forward_geom(const ConvShape& s, int N) {
-	GatherGeom g;
+GatherProblem forward_geom(const ConvShape& s, int N) {
+	GatherProblem g;
 	g.N = N; g.NS = N; g.LH = s.H; g.LW = s.W; g.LC = s.C;
 	g.OA = s.OH(); g.OB = s.OW();
 	g.R = s.RH; g.S = s.RW;
@@ -2524,8 +2529,8 @@ GatherGeom forward_geom(const ConvShape& s, int N) {
 	return g;
 }
 
-GatherGeom dgrad_geom(const ConvShape& s, int N) {
-	GatherGeom g;
+GatherProblem dgrad_geom(const ConvShape& s, int N) {
+	GatherProblem g;
 	g.N = N; g.NS = N; g.LH = s.OH(); g.LW = s.OW(); g.LC = s.F;
 	g.OA = s.H; g.OB = s.W;
 	g.R = s.RH; g.S = s.RW;
@@ -2822,7 +2827,7 @@ WgradPlan wgrad_plan(int M, int K, int F, int N, bool vec) {
 /* The plan of wgrad_bf16x3_kernel, or false where it does not apply. Of its tile shapes the one with the least padding
  * (the larger on ties, which reads the operands less often) that gives half of the CUs a block of at least four chunks;
  * then as many slices of M as fill the chip once. A function of the problem alone, like wgrad_plan. */
-bool bf16x3_wgrad_plan(const GatherGeom& g, Bf16x3WgradPlan* plan) {
+bool bf16x3_wgrad_plan(const GatherProblem& g, Bf16x3WgradPlan* plan) {
 	if (g.fp32_products || g.F <= 8 || g.K < 48 || 2.0 * g.M * g.K * g.F < 3e8 || tuning().no_bf16x3 || !bf16x3_wgrad_possible(g))
 		return false;
 	const int chunks = (g.M + BF16X3_KC - 1) / BF16X3_KC, positions = g.M / g.N;
@@ -2893,7 +2898,7 @@ ConvWorkspace conv_workspace(const ConvShape& s, int N) {
 template<typename T>
 void conv_forward(const ConvShape& s, int N, const T* x, const T* w, const T* b, T* out, T* wt, bool wt_ready, int x_batch) {
 	check_sizes(s, std::max(N, x_batch));
-	GatherGeom g = forward_geom(s, N);
+	GatherProblem g = forward_geom(s, N);
 	if (x_batch > 0)
 		g.NS = x_batch;
 	if (!wt_ready) {
@@ -2909,7 +2914,7 @@ template<typename T>
 bool conv_forward_lstm(const ConvShape& s, int N, const T* x, int x_batch, const T* w, const T* b, T* wt, bool wt_ready,
 		const LstmForwardStep<T>& step) {
 	check_sizes(s, std::max(N, x_batch));
-	GatherGeom g = forward_geom(s, N);
+	GatherProblem g = forward_geom(s, N);
 	if (x_batch > 0)
 		g.NS = x_batch;
 	Epilogue<T> E = { 0, (T) 0, nullptr, nullptr, 1, 1, 1, 1, nullptr, step };
@@ -2929,7 +2934,7 @@ template<typename T>
 bool conv_forward_fused(const ConvShape& s, int N, const T* x, const T* w, const T* b, T* out, T* wt, bool wt_ready, int epi,
 		const Epilogue<T>& E, int* mtiles) {
 	check_sizes(s, N);
-	const GatherGeom g = forward_geom(s, N);
+	const GatherProblem g = forward_geom(s, N);
 	if (epi == EPI_POOL) {
 		CATTLE_HIP_REQUIRE(E.prh > 0 && E.prw > 0 && g.OA % E.prh == 0 && g.OB % E.prw == 0 && E.OHp == g.OA / E.prh &&
 				E.OWp == g.OB / E.prw && (E.inds != nullptr || E.pool_mean), "the pooling epilogue needs windows that tile the output");
@@ -2979,7 +2984,7 @@ void conv_forward_static(const ConvShape& s, int N, const T* x, const T* w, cons
 	CATTLE_HIP_CHECK(hipGetDevice(&dev));
 	CATTLE_HIP_REQUIRE(dev >= 0 && dev < MAX_DEVICES && g_scratch_ptr[dev] != nullptr, "the static scratch buffer of this device is not set up");
 	ScratchArena arena = { static_cast<char*>(g_scratch_ptr[dev]), STATIC_SCRATCH_BYTES, 0 };
-	const GatherGeom g = forward_geom(s, N);
+	const GatherProblem g = forward_geom(s, N);
 	const int Kp = round_up(g.K, WT_ROW_PAD);
 	const size_t count = (size_t) Kp * g.ldw;
 	T* wt = static_cast<T*>(arena.take(count * sizeof(T), "prepared weights"));
@@ -3009,7 +3014,7 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 	check_sizes(s, N);
 	if (deferred)
 		deferred->count = 0;
-	const GatherGeom g = forward_geom(s, N);
+	const GatherProblem g = forward_geom(s, N);
 	/* split-M partials, then a fixed-order reduction that accumulates */
 	const bool vec = N % GemmCfg<T>::VEC == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
 			(reinterpret_cast<uintptr_t>(out_grad) & 15) == 0 &&
@@ -3139,7 +3144,7 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 			empty_class = empty_class || (c.Rc * c.Sc == 0 && c.OAc * c.OBc > 0);
 		if (empty_class)        /* positions that no tap reaches (a receptor narrower than the stride) */
 			device_zero_fill(in_grad, (size_t) N * s.H * s.W * s.C * sizeof(T));
-		std::vector<GatherGeom> geoms;
+		std::vector<GatherProblem> geoms;
 		std::vector<const T*> weights;
 		for (const StridedClass& c : classes) {
 			if (c.OAc * c.OBc == 0 || c.Rc * c.Sc == 0)
@@ -3152,7 +3157,7 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 						c.r0, s.sv, c.Rc, c.s0, s.sh, c.Sc, Kp, ldw);
 				CATTLE_HIP_CHECK(hipGetLastError());
 			}
-			GatherGeom g;
+			GatherProblem g;
 			g.N = N; g.NS = og_batch > 0 ? og_batch : N; g.LH = s.OH(); g.LW = s.OW(); g.LC = s.F;
 			g.OA = c.OAc; g.OB = c.OBc;
 			g.R = c.Rc; g.S = c.Sc;
@@ -3169,7 +3174,7 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 		for (size_t i = 0; i < order.size(); ++i)
 			order[i] = i;
 		std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return geoms[x].K > geoms[y].K; });
-		std::vector<GatherGeom> sorted_geoms;
+		std::vector<GatherProblem> sorted_geoms;
 		std::vector<const T*> sorted_weights;
 		for (size_t i : order) {
 			sorted_geoms.push_back(geoms[i]);
@@ -3185,7 +3190,7 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 				launch_gather<T>(out_grad, weights[i], (const T*) nullptr, in_grad, geoms[i]);
 		return false;
 	}
-	GatherGeom d = dgrad_geom(s, N);
+	GatherProblem d = dgrad_geom(s, N);
 	if (og_batch > 0)
 		d.NS = og_batch;
 	if (!wt_ready) {
