@@ -82,10 +82,8 @@ struct GatherGeom {
 /* Convolution hyper-parameters in the reference's terms (dilation 0 = dense receptor). */
 struct ConvShape {
 	int H, W, C, F, RH, RW, pv, ph, sv, sh, dv, dh;
-	/* The fp32 matrix instructions for all products, also where the bf16 ones would serve: for a kernel layer that is grouped
-	 * with a max pool. Which of nearly equal values a max pool picks, and so where the gradient goes, turns on the last bits
-	 * of the layer's results: with other roundings, if smaller ones, parameters trained for four batches came out 3e-3 (2-norm)
-	 * away from where the fp32 instructions had taken them (from the 64-bit result: 2e-5 and 7e-4). */
+	/* The fp32 matrix instructions for all products of a call, also where the bf16 ones would serve (FusedLayer::shape says
+	 * who asks for them, and why). */
 	bool fp32_products = false;
 	int OH() const { return (H - RH - (RH - 1) * dv + 2 * pv) / sv + 1; }
 	int OW() const { return (W - RW - (RW - 1) * dh + 2 * ph) / sh + 1; }

@@ -2598,7 +2598,8 @@ bool strided_classes(const ConvShape& s, std::vector<StridedClass>* out, size_t*
 template<typename T>
 bool use_strided_classes(const ConvShape& s, int N) {
 	/* a lane's neighbouring rows (up to four in fp64, two in fp32) have to be samples of one position */
-	if (s.C <= FEW_COLUMNS || N % (std::is_same<T, float>::value ? 2 : 4) != 0 || !strided_classes(s, nullptr, nullptr))
+	const int together = std::is_same<T, float>::value && !s.fp32_products ? 2 : 4;
+	if (s.C <= FEW_COLUMNS || N % together != 0 || !strided_classes(s, nullptr, nullptr))
 		return false;
 	const double useful = 2.0 * N * s.OH() * s.OW() * (double) s.K() * s.F;
 	return useful >= 2e8 * s.sv * s.sh;

@@ -487,34 +487,38 @@ struct ConvLayer : LayerBase {
 		return new ConvLayer(*this, share);
 	}
 	void forward(const void* in, size_t N, bool, void* out) override {
+		forward_as(shape, in, N, out);
+	}
+	void backward(const void* out_grad, size_t N, void* in_grad) override {
+		backward_as(shape, out_grad, N, in_grad, nullptr);
+	}
+	/* The passes of this layer's problem `s`: its shape, as the caller wants it run (ConvShape::fp32_products). */
+	void forward_as(const ConvShape& s, const void* in, size_t N, void* out) {
 		const int n = checked_int(N, "batch size");
-		const ConvWorkspace ws = conv_workspace<T>(shape, n);
+		const ConvWorkspace ws = conv_workspace<T>(s, n);
 		Param& w = *params[0];
 		T* wt = (T*) w.derived[0].ensure(ws.wt_fwd * sizeof(T));
 		const bool ready = w.derived_version[0] == w.version;
-		conv_forward<T>(shape, n, (const T*) in, (const T*) w.values.p, (const T*) params[1]->values.p, (T*) out, wt, ready);
+		conv_forward<T>(s, n, (const T*) in, (const T*) w.values.p, (const T*) params[1]->values.p, (T*) out, wt, ready);
 		w.derived_version[0] = w.version;
 		x_cache = (const T*) in;       /* the reference caches the patch matrix (ConvKernelLayer.hpp:127); the input suffices */
 	}
-	void backward(const void* out_grad, size_t N, void* in_grad) override {
-		backward_through(out_grad, N, in_grad, nullptr);
-	}
 	/* `act`: out_grad is the gradient behind an element-wise activation whose derivative the weight-gradient launch
 	 * applies on its way (WgradAct) */
-	void backward_through(const void* out_grad, size_t N, void* in_grad, const WgradAct<T>* act) {
+	void backward_as(const ConvShape& s, const void* out_grad, size_t N, void* in_grad, const WgradAct<T>* act) {
 		CATTLE_HIP_REQUIRE(x_cache != nullptr, "pass_back without a cached forward input");
 		const int n = checked_int(N, "batch size");
-		const ConvWorkspace ws = conv_workspace<T>(shape, n);
 		Param& w = *params[0];
+		const ConvWorkspace ws = conv_workspace<T>(s, n);
 		T* wt = (T*) w.derived[1].ensure(ws.wt_dgrad * sizeof(T));
-		const int layout = dgrad_weight_layout<T>(shape, n);
+		const int layout = dgrad_weight_layout<T>(s, n);
 		const bool ready = w.derived_version[1] == w.version && w.dgrad_layout == layout;
 		/* the partial sums of the launch before, if they still wait, would be overwritten */
 		if (w.pending)
 			g_deferred.settle();
 		T* part = (T*) w.partials.ensure(ws.partials * sizeof(T));
 		ReduceBatch<T> later;
-		conv_backward<T>(shape, n, x_cache, (const T*) w.values.p, (const T*) out_grad, (T*) w.grad.p, (T*) params[1]->grad.p,
+		conv_backward<T>(s, n, x_cache, (const T*) w.values.p, (const T*) out_grad, (T*) w.grad.p, (T*) params[1]->grad.p,
 				(T*) in_grad, wt, ready, part, act, &later);
 		g_deferred.add<T>(&w, later);
 		if (in_grad) {
@@ -1051,8 +1055,6 @@ struct FusedLayer : LayerBase {
 		CATTLE_HIP_REQUIRE(at == layers.size(), "members must be: kernel layer, then optionally batch norm, activation, pool, in this order");
 		for (size_t i = 0; i + 1 < layers.size(); ++i)
 			CATTLE_HIP_REQUIRE(layers[i]->out_volume() == layers[i + 1]->in_volume(), "member dimensions do not chain");
-		if (pool && pool->kind == CATTLE_HIP_POOL_MAX)
-			conv->shape.fp32_products = true;
 		std::memcpy(in_dims, conv->in_dims, sizeof(in_dims));
 		std::memcpy(out_dims, layers.back()->out_dims, sizeof(out_dims));
 		input_layer = conv->input_layer;
@@ -1074,6 +1076,19 @@ struct FusedLayer : LayerBase {
 		return f;
 	}
 
+	/* The kernel layer's problem as this group runs it. With a max pool: on the fp32 matrix instructions, as these groups always
+	 * have. Which of nearly equal values the pool picks turns on the last bits of the kernel layer's results, and where the
+	 * gradient goes turns on that: any other rounding, of the forward products or (a step later, through the weights) of the
+	 * gradients, moves some picks and a trained network with them. Over four batches of a small image classifier (128 x 32 x
+	 * 32 x 3, Adam) the parameters of the two kinds of instruction come out up to 1e-2 (2-norm) apart. Not because the fp32
+	 * ones were the more accurate: over 20 seeds they are 1.7e-4 from 64 bits in the median, the bf16 ones 1.4e-5, and 1.1e-2
+	 * at the worst with either. It leaves trained results where they were; a large layer pays for it in time.
+	 * The member layer itself is not touched: called alone it chooses like any other. */
+	ConvShape shape() const {
+		ConvShape s = conv->shape;
+		s.fp32_products = pool && pool->kind == CATTLE_HIP_POOL_MAX;
+		return s;
+	}
 	int OH() const { return conv->shape.OH(); }
 	int OW() const { return conv->shape.OW(); }
 	int F() const { return conv->shape.F; }
@@ -1101,7 +1116,7 @@ struct FusedLayer : LayerBase {
 		return cs;
 	}
 	T* prepared_weights(int n, bool& ready) {
-		const ConvWorkspace ws = conv_workspace<T>(conv->shape, n);
+		const ConvWorkspace ws = conv_workspace<T>(shape(), n);
 		Param& w = *conv->params[0];
 		ready = w.derived_version[0] == w.version;
 		return (T*) w.derived[0].ensure(ws.wt_fwd * sizeof(T));
@@ -1137,7 +1152,7 @@ struct FusedLayer : LayerBase {
 			bool ok = true;
 			if (training) {
 				E.stats = (T*) stats_buf.ensure(conv_stats_rows(conv->shape, n) * F() * 3 * sizeof(T));
-				ok = conv_forward_fused<T>(conv->shape, n, x, wv, bv, z, wt, ready, EPI_STATS, E, &mtiles);
+				ok = conv_forward_fused<T>(shape(), n, x, wv, bv, z, wt, ready, EPI_STATS, E, &mtiles);
 				weights_prepared();
 			}
 			if (!ok) {
@@ -1145,7 +1160,7 @@ struct FusedLayer : LayerBase {
 				return;
 			}
 			if (!training) {
-				conv_forward<T>(conv->shape, n, x, wv, bv, z, wt, ready);
+				conv_forward<T>(shape(), n, x, wv, bv, z, wt, ready);
 				weights_prepared();
 			}
 			pool_in_chain = pool_tiles();
@@ -1194,7 +1209,7 @@ struct FusedLayer : LayerBase {
 				E.inds = (unsigned*) pool->inds.ensure(pcount * sizeof(unsigned));
 				E.pre = needs_pre ? (T*) pre_buf.ensure(pcount * sizeof(T)) : nullptr;
 			}
-			const bool ok = conv_forward_fused<T>(conv->shape, n, x, wv, bv, (T*) out, wt, ready, EPI_POOL, E, nullptr);
+			const bool ok = conv_forward_fused<T>(shape(), n, x, wv, bv, (T*) out, wt, ready, EPI_POOL, E, nullptr);
 			weights_prepared();
 			ready = true;
 			if (ok) {
@@ -1216,7 +1231,7 @@ struct FusedLayer : LayerBase {
 		if (act) {
 			T* y = pool ? (T*) z_buf.ensure(zcount * sizeof(T)) : (T*) out;
 			E.pre = needs_pre ? (T*) pre_buf.ensure(zcount * sizeof(T)) : nullptr;
-			const bool ok = conv_forward_fused<T>(conv->shape, n, x, wv, bv, y, wt, ready, EPI_ACT, E, nullptr);
+			const bool ok = conv_forward_fused<T>(shape(), n, x, wv, bv, y, wt, ready, EPI_ACT, E, nullptr);
 			weights_prepared();
 			if (ok) {
 				if (pool)
@@ -1237,7 +1252,10 @@ struct FusedLayer : LayerBase {
 		for (size_t i = 0; i < members.size(); ++i) {
 			LayerBase* l = members[i];
 			void* dst = i + 1 == members.size() ? out : mid[i]->ensure(N * l->out_volume() * esize());
-			l->forward(cur, N, training, dst);
+			if (i == 0)
+				conv->forward_as(shape(), cur, N, dst);
+			else
+				l->forward(cur, N, training, dst);
 			cur = dst;
 		}
 		mode = MODE_UNFUSED;
@@ -1254,7 +1272,10 @@ struct FusedLayer : LayerBase {
 				void* dst = in_grad;
 				if (i > 0)
 					dst = ((members.size() - i) % 2 ? grad_a : grad_b).ensure(N * l->in_volume() * esize());
-				l->backward(g, N, dst);
+				if (i == 0)
+					conv->backward_as(shape(), g, N, dst, nullptr);
+				else
+					l->backward(g, N, dst);
 				g = dst;
 			}
 			return;
@@ -1293,12 +1314,12 @@ struct FusedLayer : LayerBase {
 				 * launch while it loads the gradient, which also leaves dz behind for the input-gradient launch - no
 				 * pass of its own */
 				const WgradAct<T> through = { y_cache, in_grad ? dz : nullptr, act->kind, (T) act->p, nullptr, 0, 0 };
-				conv->backward_through(g, N, in_grad, &through);
+				conv->backward_as(shape(), g, N, in_grad, &through);
 				return;
 			}
 			chain_backward<T>(chain_shape(false), n, g, nullptr, y_cache, needs_pre() ? (const T*) pre_buf.p : nullptr, dz);
 		}
-		conv->backward(dz, N, in_grad);
+		conv->backward_as(shape(), dz, N, in_grad, nullptr);
 	}
 	bool needs_pre() const {
 		return act && !act_backward_from_output(act->kind, (double) act->p);
@@ -1324,7 +1345,7 @@ struct FusedLayer : LayerBase {
 		if (act && !(act_sign_coded(act->kind) && act->p >= 0))
 			return false;
 		const WgradAct<T> through = { y_cache, nullptr, act ? act->kind : -1, act ? (T) act->p : (T) 0, (const unsigned*) pool->inds.p, sh_a, sh_b };
-		conv->backward_through(g, (size_t) n, nullptr, &through);
+		conv->backward_as(shape(), g, (size_t) n, nullptr, &through);
 		return true;
 	}
 	void empty_cache() override {

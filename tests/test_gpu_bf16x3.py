@@ -223,3 +223,64 @@ def test_fused_epilogues(shape, behind):
         if k in one:
             e = np.linalg.norm(one[k].astype(np.float64) - many[k]) / np.linalg.norm(many[k].astype(np.float64))
             assert e <= (2 if k == "out" else 200 if "batch" in behind or "relu" in behind else 2) * 2.0 ** -24 * L ** 0.5, (k, e)
+
+
+def _pooled_layers(shape, w, b):
+    H, W, C, F = shape
+    layers = [ch.ConvKernelLayer(np.float32, (H, W, C), F), ch.ActivationLayer(np.float32, "relu", (H, W, F)), ch.MaxPoolLayer(np.float32, (H, W, F))]
+    layers[0].get_params()[0].set_values(w)
+    layers[0].get_params()[1].set_values(b)
+    return layers
+
+
+@pytest.mark.parametrize("N", [32, 30, 33])
+def test_max_pool_group_leaves_its_kernel_layer_as_it_was(N):
+    """A kernel layer grouped with a max pool runs on the fp32 instructions there; called by itself, before or after the
+    group, it gives the bits of a layer that was never grouped."""
+    H, W, C, F = 16, 16, 24, 100
+    x, w, b, go = _inputs(N, H, W, C, F, _geom(), 13)
+    pooled = go[:, ::2, ::2]
+
+    def alone(conv):
+        out = conv.pass_forward(x, True)
+        dx = conv.pass_back(go)
+        dw = conv.get_params()[0].get_grad()
+        for p in conv.get_params():
+            p.reset_grad()
+        return out, dx, dw
+
+    plain, members = _pooled_layers((H, W, C, F), w, b), _pooled_layers((H, W, C, F), w, b)
+    expected = alone(plain[0])
+    group = ch.fuse_layers(members)
+    assert len(group) == 1
+    for _ in range(2):
+        for got, ref in zip(alone(members[0]), expected):
+            assert np.array_equal(got, ref)
+        group[0].pass_forward(x, True)
+        group[0].pass_back(pooled)
+        for p in members[0].get_params():
+            p.reset_grad()
+
+
+@pytest.mark.parametrize("N", [32, 30, 33])
+def test_max_pool_group_against_its_layers(N):
+    """Values whose products and sums are exact on either kind of instruction (small whole numbers): the group and the layers one
+    by one agree to the last bit, ties between equal values included."""
+    H, W, C, F = 16, 16, 24, 100
+    g = hp.rng(17)
+    x = np.asfortranarray(g.integers(-3, 4, (N, H, W, C)).astype(np.float32))
+    w = np.asfortranarray(g.integers(-2, 3, (9 * C, F)).astype(np.float32))
+    b = np.asfortranarray(g.integers(-2, 3, (1, F)).astype(np.float32))
+    go = np.asfortranarray(g.integers(-3, 4, (N, H // 2, W // 2, F)).astype(np.float32))
+
+    def run(layers, conv):
+        a, d = x, go
+        for l in layers:
+            a = l.pass_forward(a, True)
+        for l in reversed(layers):
+            d = l.pass_back(d)
+        return a, d, conv.get_params()[0].get_grad(), conv.get_params()[1].get_grad()
+
+    plain, members = _pooled_layers((H, W, C, F), w, b), _pooled_layers((H, W, C, F), w, b)
+    for got, ref in zip(run(ch.fuse_layers(members), members[0]), run(plain, plain[0])):
+        assert np.array_equal(np.asarray(got), np.asarray(ref))
