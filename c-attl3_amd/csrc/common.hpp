@@ -82,8 +82,8 @@ struct GatherGeom {
 /* Convolution hyper-parameters in the reference's terms (dilation 0 = dense receptor). */
 struct ConvShape {
 	int H, W, C, F, RH, RW, pv, ph, sv, sh, dv, dh;
-	/* The fp32 matrix instructions for all products of a call, also where the bf16 ones would serve (FusedLayer::shape says
-	 * who asks for them, and why). */
+	/* The fp32 matrix instructions for all products of a call, also where the bf16 ones would serve (FusedLayer::shape and
+	 * weight_gradient_workspace say who asks for them, and why). */
 	bool fp32_products = false;
 	int OH() const { return (H - RH - (RH - 1) * dv + 2 * pv) / sv + 1; }
 	int OW() const { return (W - RW - (RW - 1) * dh + 2 * ph) / sh + 1; }

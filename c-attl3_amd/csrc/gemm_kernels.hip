@@ -1029,10 +1029,20 @@ const DeviceShape& device_shape() {
 
 /* Grow-only device scratch for split reductions. Calls into the library are serialised and issued on
  * one stream, so a later call may reuse (or, after hipFree's implicit synchronisation, replace) it. */
-void* split_workspace(size_t bytes) {
-	static void* ptr = nullptr;
-	static size_t cap = 0;
-	static uint64_t born = 0;
+struct SplitWorkspace {
+	void* ptr = nullptr;
+	size_t cap = 0;
+	uint64_t born = 0;
+	bool may_grow() const { return !capturing() && !(ptr && pinned_by_graph(born)); }
+};
+SplitWorkspace g_split_workspace;
+/* `bytes` of it; where it may grow, at least `reserve` */
+void* split_workspace(size_t bytes, size_t reserve = 0) {
+	void*& ptr = g_split_workspace.ptr;
+	size_t& cap = g_split_workspace.cap;
+	uint64_t& born = g_split_workspace.born;
+	if (reserve > bytes && g_split_workspace.may_grow())
+		bytes = reserve;
 	if (bytes > cap) {
 		forbid_while_capturing("growing the scratch buffer of the split reductions (run the step once before recording it)");
 		/* every layer shares this buffer: a living graph recorded since it was allocated may point into it */
@@ -2309,14 +2319,20 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 	if constexpr (std::is_same<T, float>::value)
 		if (epi != EPI_LSTM && !divs && then == nullptr && !(rider && chosen->launch_with_wgrad))
 			if (const GatherVariant<float>* b = bf16x3_for(g, g.M, no_split)) {
-				/* a pooling epilogue: only with whole windows in that tile; a caller's scratch range: only where the fp32 launch
-				 * would fit it (or be refused), and this one does */
+				/* A pooling epilogue: only with whole windows in that tile. A caller's scratch range: only where the fp32 launch
+				 * would fit it (or be refused), and this one does. The library's own scratch: where a graph that is being
+				 * recorded, or a living one, keeps it from growing, only if this launch's parts fit it; and it grows to what
+				 * the fp32 launch would take, so that no problem finds less room than if all launches were of that kind. */
 				const RowBlocks windows = pooled ? plan_row_blocks<T>(g, b->bm, E->prh, E->prw, true) : rb;
-				const size_t room = arena ? arena->cap - arena->used : 0;
-				if ((!pooled || windows.ok) && (!arena || (cut_reductions(*chosen, g, no_split, vec, divs, epi, 0).partial_bytes <= room &&
-						cut_reductions(*b, g, no_split, vec, divs, epi, 0).partial_bytes <= room))) {
+				const size_t fp32_bytes = cut_reductions(*chosen, g, no_split, vec, divs, epi, 0).partial_bytes;
+				const size_t bytes = cut_reductions(*b, g, no_split, vec, divs, epi, 0).partial_bytes;
+				const bool fits = arena ? std::max(bytes, fp32_bytes) <= arena->cap - arena->used :
+						bytes <= g_split_workspace.cap || g_split_workspace.may_grow();
+				if ((!pooled || windows.ok) && fits) {
 					chosen = b;
 					rb = windows;
+					if (!arena)
+						(void) split_workspace(0, fp32_bytes);
 				}
 			}
 	const GatherVariant<T>& v = *chosen;

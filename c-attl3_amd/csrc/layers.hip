@@ -462,6 +462,18 @@ int checked_int(size_t v, const char* what) {
 	return (int) v;
 }
 
+/* The scratch sizes of a layer's backward pass whose partial weight gradients go to `partials`. Where a graph that is being
+ * recorded, or a living one, keeps that buffer from growing and the plan does not fit it, `s` is given to the fp32
+ * instructions, whose plan may: a batch that ran when all plans were of that kind is not refused. */
+template<typename T>
+ConvWorkspace weight_gradient_workspace(ConvShape& s, int n, const DevBuf& partials) {
+	const ConvWorkspace ws = conv_workspace<T>(s, n);
+	if (ws.partials * sizeof(T) <= partials.cap || s.fp32_products || !(capturing() || partials.pinned()))
+		return ws;
+	s.fp32_products = true;
+	return conv_workspace<T>(s, n);
+}
+
 /* ConvKernelLayer and DenseKernelLayer (a dense layer is the 1x1 case on a 1x1 image whose
  * channels are the input volume: X = Map(in.data(), N, volume), DenseKernelLayer.hpp:98). */
 template<typename T>
@@ -505,11 +517,11 @@ struct ConvLayer : LayerBase {
 	}
 	/* `act`: out_grad is the gradient behind an element-wise activation whose derivative the weight-gradient launch
 	 * applies on its way (WgradAct) */
-	void backward_as(const ConvShape& s, const void* out_grad, size_t N, void* in_grad, const WgradAct<T>* act) {
+	void backward_as(ConvShape s, const void* out_grad, size_t N, void* in_grad, const WgradAct<T>* act) {
 		CATTLE_HIP_REQUIRE(x_cache != nullptr, "pass_back without a cached forward input");
 		const int n = checked_int(N, "batch size");
 		Param& w = *params[0];
-		const ConvWorkspace ws = conv_workspace<T>(s, n);
+		const ConvWorkspace ws = weight_gradient_workspace<T>(s, n, w.partials);
 		T* wt = (T*) w.derived[1].ensure(ws.wt_dgrad * sizeof(T));
 		const int layout = dgrad_weight_layout<T>(s, n);
 		const bool ready = w.derived_version[1] == w.version && w.dgrad_layout == layout;
@@ -586,14 +598,15 @@ struct TransConvLayer : LayerBase {
 	void backward(const void* out_grad, size_t N, void* in_grad) override {
 		CATTLE_HIP_REQUIRE(x_cache != nullptr, "pass_back without a cached forward input");
 		const int n = checked_int(N, "batch size");
-		const ConvWorkspace ws = conv_workspace<T>(conv, n);
+		ConvShape s = conv;
+		const ConvWorkspace ws = weight_gradient_workspace<T>(s, n, partials);
 		Param& w = *params[0];
 		accumulate_column_sums<T>(n, out_volume(), (const T*) out_grad, (T*) params[1]->grad.p);      /* :184-185 */
 		/* in_mat^T * patches(out_grad) (:208) is the transpose of the convolution's weight gradient */
 		T* part = (T*) partials.ensure(ws.partials * sizeof(T));
 		T* gt = (T*) wgrad_t.ensure(w.bytes());
 		fill_zero(gt, w.bytes());
-		conv_weight_gradient<T>(conv, n, (const T*) out_grad, x_cache, gt, (T*) nullptr, part);
+		conv_weight_gradient<T>(s, n, (const T*) out_grad, x_cache, gt, (T*) nullptr, part);
 		transpose_matrix<T>((int) w.cols, (int) w.rows, gt, (T*) w.grad.p, true);
 		if (!in_grad)
 			return;
@@ -792,14 +805,16 @@ struct ConvLstm : LayerBase {
 			g_deferred.settle();
 		ReduceBatch<T> later;
 		if (total > 1) {
-			const ConvWorkspace ws = conv_workspace<T>(sh, (int) (N * total));
-			conv_weight_gradient<T>(sh, (int) (N * total), (const T*) hprev_all.p, (const T*) dzh_all.p, (T*) wh.grad.p,
+			ConvShape s = sh;
+			const ConvWorkspace ws = weight_gradient_workspace<T>(s, (int) (N * total), wh.partials);
+			conv_weight_gradient<T>(s, (int) (N * total), (const T*) hprev_all.p, (const T*) dzh_all.p, (T*) wh.grad.p,
 					(T*) params[3]->grad.p, (T*) wh.partials.ensure(ws.partials * e), nullptr, &later);
 			g_deferred.add<T>(&wh, later);
 		}
 		{
-			const ConvWorkspace ws = conv_workspace<T>(sx, (int) (N * T_in));
-			conv_weight_gradient<T>(sx, (int) (N * T_in), x_cache, (const T*) dzx_all.p, (T*) wx.grad.p, (T*) params[1]->grad.p,
+			ConvShape s = sx;
+			const ConvWorkspace ws = weight_gradient_workspace<T>(s, (int) (N * T_in), wx.partials);
+			conv_weight_gradient<T>(s, (int) (N * T_in), x_cache, (const T*) dzx_all.p, (T*) wx.grad.p, (T*) params[1]->grad.p,
 					(T*) wx.partials.ensure(ws.partials * e), nullptr, &later);
 			g_deferred.add<T>(&wx, later);
 			if (in_grad) {

@@ -284,3 +284,33 @@ def test_max_pool_group_against_its_layers(N):
     plain, members = _pooled_layers((H, W, C, F), w, b), _pooled_layers((H, W, C, F), w, b)
     for got, ref in zip(run(ch.fuse_layers(members), members[0]), run(plain, plain[0])):
         assert np.array_equal(np.asarray(got), np.asarray(ref))
+
+
+def test_smaller_batches_run_while_a_graph_lives():
+    """Scratch buffers that were grown at the largest batch stay where they are while a graph lives. A smaller batch whose slices
+    on the bf16 instructions would need more than that takes the fp32 plan instead of being refused."""
+    H, W, C, F = 10, 10, 87, 239
+    geom = _geom()
+    tiny = ch.DenseKernelLayer(np.float32, (4,), 3)
+    tx, ty = ch.DeviceTensor.from_host(np.ones((4, 4), np.float32, order="F")), ch.DeviceTensor((4, 3), np.float32)
+    tiny.forward_into(tx, ty, False)
+    layer = ch.ConvKernelLayer(np.float32, (H, W, C), F)
+    x, w, b, go = _inputs(61, H, W, C, F, geom, 21)
+    layer.get_params()[0].set_values(w)
+    layer.get_params()[1].set_values(b)
+    layer.pass_forward(x, True)
+    layer.pass_back(go)
+    graph = ch.Graph()
+    with graph:
+        tiny.forward_into(tx, ty, False)
+    try:
+        for N in (60, 53, 45, 38, 30, 24):
+            for p in layer.get_params():
+                p.reset_grad()
+            xs, gs = np.asfortranarray(x[:N]), np.asfortranarray(go[:N])
+            layer.pass_forward(xs, True)
+            dx = layer.pass_back(gs)
+            ref = _truth(xs, w, b, gs, geom)
+            _check({"dx": dx, "dw": layer.get_params()[0].get_grad()}, ref, {"dx": 9 * F, "dw": N * H * W})
+    finally:
+        graph.destroy()
