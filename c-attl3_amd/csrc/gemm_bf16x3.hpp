@@ -21,7 +21,8 @@ bool bf16x3_gather_possible(const GatherGeom& g);
  * batch is a multiple of four and src and out lie on 16-byte boundaries. */
 void bf16x3_gather(int shape, const float* src, const float* wt, const float* bias, float* out, const GatherGeom& g,
 		const GatherLaunch& L, float* partials, int wt_rows, int epi, const Epilogue<float>& E);
-/* the problems of a table in one launch: 16-byte rows (N a multiple of four), no bias, weights padded to wt_row_pad rows */
+/* the problems of a table in one launch: N even, src on an 8-byte boundary (pairs of samples), no bias, weights padded to
+ * wt_row_pad rows */
 void bf16x3_gather_classes(int shape, int classes_used, const float* src, float* out, const GatherClasses<float>& classes, int wt_row_pad);
 int bf16x3_gather_blocks_per_cu(int shape);
 
@@ -30,7 +31,7 @@ constexpr int BF16X3_WGRAD_TILES = 4;
 struct Bf16x3WgradPlan {
 	int shape;
 	int ktiles, tiles, splits, chunks_per_split;
-	int pixels;             /* slices are ranges of output positions (needs N % 32 == 0), else of chunks of 32 rows */
+	int pixels;             /* slices are ranges of output positions (N % 32 == 0 and 16-byte boundaries), else of chunks of 32 rows */
 	int direct;             /* one slice: the block adds its tile to the gradient itself */
 };
 void bf16x3_wgrad_tile(int shape, int* bk, int* bf);

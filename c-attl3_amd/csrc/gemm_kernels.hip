@@ -2841,10 +2841,11 @@ WgradPlan wgrad_plan(int M, int K, int F, int N, bool vec) {
 	return p;
 }
 
-/* The plan of wgrad_bf16x3_kernel, or false where it does not apply. Of its tile shapes the one with the least padding
- * (the larger on ties, which reads the operands less often) that gives half of the CUs a block of at least four chunks;
- * then as many slices of M as fill the chip once. A function of the problem alone, like wgrad_plan. */
-bool bf16x3_wgrad_plan(const GatherProblem& g, Bf16x3WgradPlan* plan) {
+/* The plan of wgrad_bf16x3_kernel, or false where it does not apply. Every tile shape is given as many slices of M as fill
+ * the chip once, of four chunks or more, and the shape of least estimated time is taken: the larger tiles read the operands
+ * less often, the smaller ones pad less. A function of the problem and of whether both operands lie on 16-byte boundaries
+ * (`aligned`: the walk by positions takes 16 bytes at a time). */
+bool bf16x3_wgrad_plan(const GatherProblem& g, bool aligned, Bf16x3WgradPlan* plan) {
 	if (g.fp32_products || g.F <= 8 || g.K < 48 || 2.0 * g.M * g.K * g.F < 3e8 || tuning().no_bf16x3 || !bf16x3_wgrad_possible(g))
 		return false;
 	const int chunks = (g.M + BF16X3_KC - 1) / BF16X3_KC, positions = g.M / g.N;
@@ -2863,7 +2864,7 @@ bool bf16x3_wgrad_plan(const GatherProblem& g, Bf16x3WgradPlan* plan) {
 		int want = std::max(1, std::min(slots / p.tiles, chunks / min_chunks));
 		p.chunks_per_split = (chunks + want - 1) / want;
 		p.splits = (chunks + p.chunks_per_split - 1) / p.chunks_per_split;
-		p.pixels = g.N % BF16X3_KC == 0 && positions >= 2;
+		p.pixels = aligned && g.N % BF16X3_KC == 0 && positions >= 2;
 		if (p.pixels)
 			p.splits = std::max(1, std::min(want, positions));
 		p.direct = p.splits == 1;
@@ -2904,9 +2905,11 @@ ConvWorkspace conv_workspace(const ConvShape& s, int N) {
 	const WgradPlan p = wgrad_plan<T>(M, s.K(), s.F, N, true), q = wgrad_plan<T>(M, s.K(), s.F, N, false);
 	int splits = std::max(p.splits, q.splits);
 	if (std::is_same<T, float>::value) {
+		const GatherProblem g = forward_geom(s, N);
 		Bf16x3WgradPlan b;
-		if (bf16x3_wgrad_plan(forward_geom(s, N), &b))
-			splits = std::max(splits, b.splits);
+		for (const bool aligned : { true, false })
+			if (bf16x3_wgrad_plan(g, aligned, &b))
+				splits = std::max(splits, b.splits);
 	}
 	ws.partials = (size_t) splits * ((size_t) s.K() * s.F + (size_t) s.F);
 	return ws;
@@ -3051,18 +3054,9 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 	}
 	/* fp32 with the gradient as it is: on the bf16 matrix instructions */
 	Bf16x3WgradPlan b3;
-	const bool bf16x3 = std::is_same<T, float>::value && !act && !few_filters && bf16x3_wgrad_plan(g, &b3);
-	if (bf16x3) {
-		if (b3.pixels && !vec) {
-			/* (a plan does not know the alignment: the same number of slices as ranges of chunks) */
-			const int chunks = (g.M + BF16X3_KC - 1) / BF16X3_KC;
-			b3.pixels = 0;
-			b3.chunks_per_split = (chunks + b3.splits - 1) / b3.splits;
-			b3.splits = (chunks + b3.chunks_per_split - 1) / b3.chunks_per_split;
-			b3.direct = b3.splits == 1;
-		}
+	const bool bf16x3 = std::is_same<T, float>::value && !act && !few_filters && bf16x3_wgrad_plan(g, vec, &b3);
+	if (bf16x3)
 		p.splits = b3.splits;
-	}
 	T* bias_partials = partials + (size_t) p.splits * count;
 	static_assert(WGRAD_MC == 32, "the chunk length gather_with_wgrad_kernel is built with");
 	const bool can_ride = elsewhere != nullptr && !bf16x3 && std::is_same<T, float>::value && !act && vec && v.bk == 32 && v.bf == 32 &&

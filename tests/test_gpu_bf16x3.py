@@ -4,6 +4,7 @@ for an fp32 number - infinities, NaNs, values near the largest and near the smal
 
 The bound on the 2-norm error is that of fp32 sums: L roundings of relative size 2^-24 that add up like a random walk,
 sqrt(L) 2^-24, for reductions of length L."""
+import ctypes
 import importlib
 
 import numpy as np
@@ -93,6 +94,41 @@ def test_values_that_are_not_finite(shape, value):
         assert bad.any() and np.array_equal(np.isnan(a), np.isnan(r)) and np.array_equal(a[np.isinf(r)], r[np.isinf(r)]), k
         e = np.linalg.norm((a - r)[~bad]) / np.linalg.norm(r[~bad]) if (~bad).any() else 0.0
         assert e <= 2.0 ** -24 * (x.shape[0] * x.shape[1] * x.shape[2]) ** 0.5, (k, e)
+
+
+class _Offset(object):
+    """A device tensor that begins `elements` fp32 elements behind a 256-byte boundary."""
+
+    def __init__(self, shape, elements, values=None):
+        self.shape = shape
+        self._block = ch.DeviceTensor((int(np.prod(shape)) + 4,), np.float32)
+        self.ptr = ctypes.c_void_p(self._block.ptr.value + 4 * elements)
+        if values is not None:
+            values = np.asfortranarray(values)
+            ch.binding._check(ch.lib().cattle_hip_upload(self.ptr, ctypes.c_void_p(values.ctypes.data), ctypes.c_size_t(values.nbytes)))
+
+    def to_host(self):
+        a = np.empty(self.shape, np.float32, order="F")
+        ch.binding._check(ch.lib().cattle_hip_download(ctypes.c_void_p(a.ctypes.data), self.ptr, ctypes.c_size_t(a.nbytes)))
+        return a
+
+
+@pytest.mark.parametrize("offset", [1, 2])
+@pytest.mark.parametrize("shape", [(64, 33, 32, 8, 96), (32, 20, 21, 24, 130), (66, 24, 24, 16, 48)], ids=str)
+def test_unaligned_tensors(shape, offset):
+    """Caller's tensors on 4- and 8-byte boundaries only: no 16-byte loads, and so no walk of the weight gradient by positions."""
+    geom = _geom()
+    x, w, b, go = _inputs(*shape, geom, 19)
+    layer = ch.ConvKernelLayer(np.float32, x.shape[1:], shape[4])
+    wp, bp = layer.get_params()
+    wp.set_values(w)
+    bp.set_values(b)
+    xd, gd, out, dx = _Offset(x.shape, offset, x), _Offset(go.shape, offset, go), _Offset(go.shape, offset), _Offset(x.shape, offset)
+    layer.forward_into(xd, out)
+    layer.backward_into(gd, dx)
+    rows = shape[0] * shape[1] * shape[2]
+    _check({"out": out.to_host(), "dx": dx.to_host(), "dw": wp.get_grad(), "db": bp.get_grad()}, _truth(x, w, b, go, geom),
+           {"out": w.shape[0], "dx": 9 * shape[4], "dw": rows, "db": rows})
 
 
 def _slice_error(got, ref):
