@@ -2114,54 +2114,86 @@ CutReductions cut_reductions(const GatherVariant<T>& v, const GatherGeom& g, boo
 	return c;
 }
 
+/* Microseconds of a round-by-round walk: a CU that holds `resident` blocks of a tile steps them all by one chunk of the
+ * reduction in `full`, one alone in `alone`, and a round of blocks ends with `tail` for what nothing overlaps (prologue, stores). */
+struct StepTimes { double full, alone, tail; };
+double rounds_time(double blocks_per_cu, int resident, int chunks, bool tail_is_cut, const StepTimes& s) {
+	const double rounds = blocks_per_cu / resident, last = rounds - std::floor(rounds);
+	const double t = std::floor(rounds) * (chunks * s.full + s.tail);
+	if (last == 0)
+		return t;
+	const double step = tail_is_cut ? s.full * last : std::max(s.alone, s.full * std::min(1.0, std::ceil(last * resident) / resident));
+	return t + chunks * step + s.tail;
+}
+template<typename T>
+double gather_time(const GatherVariant<T>& v, const GatherGeom& g, const CutReductions& cut, int resident, const StepTimes& s, double launch) {
+	const int mtiles = (g.M + v.bm - 1) / v.bm, ftiles = (g.F + v.bf - 1) / v.bf;
+	const double per_cu = (double) mtiles * ftiles / device_shape().cus;
+	const bool cuts = cut.main_count < mtiles;
+	double t;
+	if (cuts && cut.main_count == 0)
+		t = cut.chunks_per_part * std::max(s.alone, s.full * std::min(1.0, std::ceil(per_cu * cut.ksplit) / resident)) + s.tail;
+	else
+		t = rounds_time(per_cu, resident, (g.K + v.kc - 1) / v.kc, cuts, s);
+	return cuts ? t + launch + (double) cut.partial_bytes * 2 / 4e6 : t;    /* another launch; the parts written and read at 4 TB/s */
+}
+/* fp32 tiles: a chunk's products and its staging, by the tile's area and its edges; `vec`: 16-byte loads */
+template<typename T>
+StepTimes fp32_step_times(const GatherVariant<T>& v, int resident, bool vec) {
+	const double chunk = v.kc / 32.0, area = (double) v.bm * v.bf / 8192, edges = (v.bm + v.bf) / 128.0;
+	if (vec)
+		return { resident * chunk * (1.05 * area + 0.16 * edges), 0.91 * chunk, 3.7 + 0.10 * area * resident };
+	return { resident * chunk * (0.74 * area + 0.62 * edges), 1.63 * chunk, 3.3 + 0.31 * area * resident };
+}
+
 /* The tile of gather_gemm_bf16x3_kernel for a problem (of M rows in all: the classes of a strided gradient count together,
- * and cut no reductions), or null where the fp32 kernels stay: reductions of a chunk or two; problems of a few microseconds,
- * which launches and waits make up (364 x 61 x 110 took 6.0 us there, 6.5 here; 13,294 x 80 x 55, 9.4 against 7.9); and what
- * the kernel cannot address.
- * The tile is the one of least estimated time. A CU that holds `resident` blocks of a tile steps them all by one chunk in
- * `full` microseconds, one alone in `alone`, and a round of blocks ends with `tail` for the stores that nothing overlaps;
- * the figures are fits to the times of forward and input-gradient launches of 30 layers with each tile (per chunk and
- * block, 256 x 128: 802,816 x 576 x 128 in 650 us is 2.6 us; 256 x 64: 802,816 x 1152 x 64 in 750 us, 1.6 us). */
-const GatherVariant<float>* bf16x3_for(const GatherProblem& g, long M, bool no_split) {
+ * and cut no reductions), or null where the fp32 launch stays: what the kernel cannot address; problems of a few microseconds,
+ * which launches and waits make up (364 x 61 x 110 took 6.0 us there, 6.5 here); and reductions of up to four chunks where
+ * `fp32_time` microseconds, the estimate for the launch it would replace (0: none), are a tenth less than its own: few columns
+ * over many rows, whose stores and splits so few products do not cover (131,440 x 63 x 31: 13.4 us there, 22.5 here).
+ * The tile is the one of least estimated time. Up to eight chunks the launch's ends weigh as much as its chunks: step times of
+ * their own, and whether reductions are cut (`cuts`) is a choice too, since cutting a few chunks costs a launch to save less
+ * (15,678 x 125 x 21: 16.4 us cut, 9.2 whole). Longer ones, which the whole chip steps at a lower clock, are cut by the rule
+ * of cut_reductions alone (per chunk and block, 256 x 128: 802,816 x 576 x 128 in 650 us is 2.6 us; 256 x 64: 802,816 x 1152 x
+ * 64 in 750 us, 1.6 us).
+ * The step times are fits to the forward launches of 460 layers, with each tile, whole and cut, and on the fp32 instructions;
+ * for four fifths of the layers they are within 20 %. Of the 460, ten run more than 5 % slower than their fp32 launch, by up to 18 %
+ * (43, by up to 67 %, with one table of step times, without the choice of cuts and without the comparison); of 280 others 15, by
+ * up to 27 % (22, up to 67 %). */
+struct Bf16x3Choice { const GatherVariant<float>* v; bool cuts; };
+Bf16x3Choice bf16x3_for(const GatherProblem& g, long M, bool no_split, double fp32_time) {
 	if (g.fp32_products || g.K < 48 || g.F <= 8 || 2.0 * M * g.K * g.F < 3e7 || tuning().no_bf16x3 || !bf16x3_gather_possible(g))
-		return nullptr;
+		return { nullptr, false };
 	const GatherVariant<float>* const vars = bf16x3_variants();
 	if (tuning().bf16x3_tile >= 0)
-		return &vars[tuning().bf16x3_tile];
-	static const struct { double full, alone, tail; } step[BF16X3_TILES] = {
+		return { &vars[tuning().bf16x3_tile], true };
+	static const StepTimes up_to_eight[BF16X3_TILES] = {
+		{ 1.74, 1.58, 9.2 }, { 1.26, 1.26, 7.0 }, { 1.71, 0.65, 5.7 }, { 1.39, 0.71, 4.8 }, { 1.21, 0.85, 5.2 }
+	}, longer[BF16X3_TILES] = {
 		{ 2.6, 2.6, 5.0 }, { 1.6, 1.6, 4.5 }, { 2.08, 1.2, 2.5 }, { 1.56, 0.75, 2.5 }, { 1.5, 1.2, 5.0 }
 	};
+	const int chunks = (g.K + BF16X3_KC - 1) / BF16X3_KC;
+	const bool is_short = chunks <= 8;
 	GatherGeom whole = g;
 	whole.M = (int) std::min<long>(M, 2147483647);
-	int best = -1;
+	Bf16x3Choice best = { nullptr, false };
 	double least = 0;
 	for (int i = 0; i < BF16X3_TILES; ++i) {
-		const GatherVariant<float>& v = vars[i];
-		const int resident = v.blocks_per_cu(0, true, false, EPI_NONE), cus = device_shape().cus;
-		const int mtiles = (whole.M + v.bm - 1) / v.bm, ftiles = (g.F + v.bf - 1) / v.bf;
-		const CutReductions cut = cut_reductions(v, whole, no_split, true, false, EPI_NONE, 0);
-		const double per_chunk = (double) mtiles * ftiles / cus;
-		/* time per chunk and round with n blocks on a CU */
-		const auto chunk = [&](double n) { return std::max(step[i].alone, step[i].full * std::min(1.0, std::ceil(n) / resident)); };
-		double t;
-		if (cut.few_tiles) {
-			t = cut.chunks_per_part * chunk(per_chunk * cut.ksplit) + step[i].tail;
-		} else {
-			const double rounds = (double) mtiles * ftiles / ((double) cus * resident);
-			const double last = rounds - std::floor(rounds);
-			const int chunks = (g.K + BF16X3_KC - 1) / BF16X3_KC;
-			t = std::floor(rounds) * (chunks * step[i].full + step[i].tail);
-			if (last > 0)
-				t += cut.main_count < mtiles ? chunks * step[i].full * last + step[i].tail : chunks * chunk(last * resident) + step[i].tail;
-		}
-		if (cut.main_count < mtiles)
-			t += 5.0 + (double) cut.partial_bytes * 2 / 4e6;         /* another launch; the parts written and read at 4 TB/s */
-		if (best < 0 || t < least) {
-			best = i;
-			least = t;
+		const int resident = vars[i].blocks_per_cu(0, true, false, EPI_NONE);
+		for (const bool cuts : { true, false }) {
+			if (cuts ? no_split : !no_split && !is_short)
+				continue;
+			const CutReductions cut = cut_reductions(vars[i], whole, !cuts, true, false, EPI_NONE, 0);
+			const double t = gather_time(vars[i], whole, cut, resident, is_short ? up_to_eight[i] : longer[i], is_short ? 3.0 : 5.0);
+			if (best.v == nullptr || t < least) {
+				best = { &vars[i], cuts };
+				least = t;
+			}
 		}
 	}
-	return &vars[best];
+	if (chunks <= 4 && fp32_time > 0 && least > 1.1 * fp32_time)
+		return { nullptr, false };
+	return best;
 }
 
 template<typename T>
@@ -2316,25 +2348,34 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 	const bool mapped = g.out_sa != 1 || g.out_sb != 1 || g.out_a0 != 0 || g.out_b0 != 0 || g.out_OA != g.OA;
 	const bool no_split = tune.no_split || epi == EPI_POOL || epi == EPI_STATS || epi == EPI_LSTM || (mapped && g.N % 4 != 0);
 	const GatherVariant<T>* chosen = &vars[best_v];
+	bool cuts = true;
 	if constexpr (std::is_same<T, float>::value)
-		if (epi != EPI_LSTM && !divs && then == nullptr && !(rider && chosen->launch_with_wgrad))
-			if (const GatherVariant<float>* b = bf16x3_for(g, g.M, no_split)) {
+		if (epi != EPI_LSTM && !divs && then == nullptr && !(rider && chosen->launch_with_wgrad)) {
+			const CutReductions fp32_cut = cut_reductions(*chosen, g, no_split, vec, divs, epi, 0);
+			const int resident = chosen->blocks_per_cu(0, vec, divs, epi);
+			/* (few tiles whose reductions the wavefronts of a block share are that launch either way) */
+			const double fp32_time = fp32_cut.few_tiles && wave_split_waves<T>(g) > 0 ? 0.0 :
+					gather_time(*chosen, g, fp32_cut, resident, fp32_step_times(*chosen, resident, vec), 5.0);
+			const Bf16x3Choice choice = bf16x3_for(g, g.M, no_split, fp32_time);
+			if (const GatherVariant<float>* b = choice.v) {
 				/* A pooling epilogue: only with whole windows in that tile. A caller's scratch range: only where the fp32 launch
 				 * would fit it (or be refused), and this one does. The library's own scratch: where a graph that is being
 				 * recorded, or a living one, keeps it from growing, only if this launch's parts fit it; and it grows to what
 				 * the fp32 launch would take, so that no problem finds less room than if all launches were of that kind. */
 				const RowBlocks windows = pooled ? plan_row_blocks<T>(g, b->bm, E->prh, E->prw, true) : rb;
-				const size_t fp32_bytes = cut_reductions(*chosen, g, no_split, vec, divs, epi, 0).partial_bytes;
-				const size_t bytes = cut_reductions(*b, g, no_split, vec, divs, epi, 0).partial_bytes;
+				const size_t fp32_bytes = fp32_cut.partial_bytes;
+				const size_t bytes = cut_reductions(*b, g, no_split || !choice.cuts, vec, divs, epi, 0).partial_bytes;
 				const bool fits = arena ? std::max(bytes, fp32_bytes) <= arena->cap - arena->used :
 						bytes <= g_split_workspace.cap || g_split_workspace.may_grow();
 				if ((!pooled || windows.ok) && fits) {
 					chosen = b;
 					rb = windows;
+					cuts = choice.cuts;
 					if (!arena)
 						(void) split_workspace(0, fp32_bytes);
 				}
 			}
+		}
 	const GatherVariant<T>& v = *chosen;
 	if (epi == EPI_LSTM) {
 		/* a short tile (it stages itself whole) whose column groups are whole gate groups of the hidden channels */
@@ -2374,7 +2415,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 	}
 	if (mtiles_out)
 		*mtiles_out = mtiles;
-	const CutReductions cut = cut_reductions(v, g, no_split, vec, divs, epi, dyn);
+	const CutReductions cut = cut_reductions(v, g, no_split || !cuts, vec, divs, epi, dyn);
 	const Epilogue<T> none = { 0, (T) 0, nullptr, nullptr, 1, 1, 1, 1, nullptr, {} };
 	const Epilogue<T>& epi_args = E ? *E : none;
 
@@ -2403,7 +2444,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 		}
 	};
 
-	if (cut.few_tiles) {
+	if (cuts ? cut.few_tiles : cut_reductions(v, g, no_split, vec, divs, epi, dyn).few_tiles) {
 		/* far fewer tiles than the chip holds blocks: the reduction of every tile is dealt to the wavefronts of one block
 		 * where it is short enough for that (wave_split_gemm_kernel: one launch, no partial sums in memory), else cut into
 		 * parts, one block each, which a second launch adds up */
@@ -2485,10 +2526,10 @@ bool launch_gather_classes(const T* src, T* out, const std::vector<GatherProblem
 		bool all = true;
 		for (const GatherProblem& g : geoms) {
 			M += g.M;
-			all = all && bf16x3_for(g, g.M, true) != nullptr;
+			all = all && bf16x3_for(g, g.M, true, 0).v != nullptr;
 		}
 		if (all && (reinterpret_cast<uintptr_t>(src) & 7) == 0 && geoms[0].N % 2 == 0 && geoms[0].NS % 2 == 0) {
-			chosen = bf16x3_for(geoms[0], M, true);
+			chosen = bf16x3_for(geoms[0], M, true, 0).v;
 			vec = true;             /* pairs of samples are all it needs */
 		}
 	}
