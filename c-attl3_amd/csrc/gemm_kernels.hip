@@ -2882,15 +2882,33 @@ WgradPlan wgrad_plan(int M, int K, int F, int N, bool vec) {
 	return p;
 }
 
+/* Microseconds of a weight gradient of `tiles` tiles of bk x bf and their slices of `chunks` chunks of mc rows each: rounds of
+ * blocks, then the sum of the slices (another launch, and the slices written and read at 4 TB/s) or the gradient's own update. */
+double wgrad_time(const GatherGeom& g, int bk, int bf, int mc, int tiles, int splits, int chunks, int resident, const double (&fit)[5]) {
+	const double chunk = mc / 32.0, gradient = 4.0 * g.K * g.F / 4e6;
+	const StepTimes s = { resident * chunk * (fit[0] * bk * bf / 4096 + fit[1] * (bk + bf) / 64), fit[2] * chunk, fit[3] };
+	return rounds_time((double) tiles * splits / device_shape().cus, resident, chunks, false, s) +
+			(splits > 1 ? fit[4] + 2.0 * splits * gradient : 2.0 * gradient);
+}
+
 /* The plan of wgrad_bf16x3_kernel, or false where it does not apply. Every tile shape is given as many slices of M as fill
  * the chip once, of four chunks or more, and the shape of least estimated time is taken: the larger tiles read the operands
- * less often, the smaller ones pad less. A function of the problem and of whether both operands lie on 16-byte boundaries
- * (`aligned`: the walk by positions takes 16 bytes at a time). */
-bool bf16x3_wgrad_plan(const GatherProblem& g, bool aligned, Bf16x3WgradPlan* plan) {
-	if (g.fp32_products || g.F <= 8 || g.K < 48 || 2.0 * g.M * g.K * g.F < 3e8 || tuning().no_bf16x3 || !bf16x3_wgrad_possible(g))
+ * less often, the smaller ones pad less. A function of the problem and of whether both operands allow 16-byte loads (`vec`:
+ * the walk by positions takes 16 bytes at a time).
+ * Up to sixteen chunks in all (a dense layer, whose M is the batch) the time is that of the launches' ends and of the slices'
+ * sum: it is estimated in microseconds (fits to 410 layers, within 20 % for four fifths of them). Up to ten, either kind of
+ * instruction may be the faster (229 x 5146 x 381: 21.4 us on the fp32 ones, 38 here with any tile but one; 338 x 3979 x 829:
+ * 62.7 there, 29.6 here), and the fp32 plan stays where it is estimated a tenth better. Above sixteen the cost counts
+ * products and staging only. */
+constexpr double BF16X3_WGRAD_FLOPS = 3e8;
+bool bf16x3_wgrad_plan(const GatherProblem& g, bool vec, Bf16x3WgradPlan* plan) {
+	if (g.fp32_products || g.F <= 8 || g.K < 48 || 2.0 * g.M * g.K * g.F < BF16X3_WGRAD_FLOPS || tuning().no_bf16x3 || !bf16x3_wgrad_possible(g))
 		return false;
 	const int chunks = (g.M + BF16X3_KC - 1) / BF16X3_KC, positions = g.M / g.N;
 	const int min_chunks = tuning().wgrad_min_chunks > 0 ? tuning().wgrad_min_chunks : 4;
+	static const double fit[5] = { 0.122, 0.243, 0.6, 2.9, 10.5 }, fp32_vec[5] = { 0.514, 0.047, 1.32, 1.4, 10.5 },
+			fp32_scalar[5] = { 0.344, 0.216, 0.24, 4.6, 9.9 };
+	const bool short_m = chunks <= 16;
 	double best = 0;
 	for (int i = 0; i < BF16X3_WGRAD_TILES; ++i) {
 		if (tuning().bf16x3_wtile >= 0 && i != tuning().bf16x3_wtile)
@@ -2905,7 +2923,7 @@ bool bf16x3_wgrad_plan(const GatherProblem& g, bool aligned, Bf16x3WgradPlan* pl
 		int want = std::max(1, std::min(slots / p.tiles, chunks / min_chunks));
 		p.chunks_per_split = (chunks + want - 1) / want;
 		p.splits = (chunks + p.chunks_per_split - 1) / p.chunks_per_split;
-		p.pixels = aligned && g.N % BF16X3_KC == 0 && positions >= 2;
+		p.pixels = vec && g.N % BF16X3_KC == 0 && positions >= 2;
 		if (p.pixels)
 			p.splits = std::max(1, std::min(want, positions));
 		p.direct = p.splits == 1;
@@ -2913,13 +2931,20 @@ bool bf16x3_wgrad_plan(const GatherProblem& g, bool aligned, Bf16x3WgradPlan* pl
 		 * of a column of products each */
 		const double blocks = (double) p.tiles * p.splits;
 		const double rounds = std::max(1.0, std::ceil(blocks / slots));
-		const double cost = rounds * bf16x3_wgrad_blocks_per_cu(i) * ((double) bk * bf + 24.0 * (bk + bf)) * ((double) chunks / p.splits + 4);
+		const double cost = short_m ?
+				wgrad_time(g, bk, bf, BF16X3_KC, p.tiles, p.splits, (chunks + p.splits - 1) / p.splits, bf16x3_wgrad_blocks_per_cu(i), fit) :
+				rounds * bf16x3_wgrad_blocks_per_cu(i) * ((double) bk * bf + 24.0 * (bk + bf)) * ((double) chunks / p.splits + 4);
 		if (best == 0 || cost < best) {
 			best = cost;
 			*plan = p;
 		}
 	}
-	return true;
+	if (chunks > 10 || tuning().bf16x3_wtile >= 0)
+		return true;
+	const WgradPlan q = wgrad_plan<float>(g.M, g.K, g.F, g.N, vec);
+	const WgradVariant<float>& v = WgradVariants<float>::get()[q.variant];
+	const int resident = std::max(1, std::min(v.blocks_per_cu(), std::max(3, 16 / v.waves)));
+	return best <= 1.1 * wgrad_time(g, v.bk, v.bf, v.mc, q.ktiles * q.ftiles, q.splits, q.chunks_per_split, resident, vec ? fp32_vec : fp32_scalar);
 }
 
 } /* namespace */
@@ -2948,8 +2973,8 @@ ConvWorkspace conv_workspace(const ConvShape& s, int N) {
 	if (std::is_same<T, float>::value) {
 		const GatherProblem g = forward_geom(s, N);
 		Bf16x3WgradPlan b;
-		for (const bool aligned : { true, false })
-			if (bf16x3_wgrad_plan(g, aligned, &b))
+		for (const bool vec : { true, false })
+			if (bf16x3_wgrad_plan(g, vec, &b))
 				splits = std::max(splits, b.splits);
 	}
 	ws.partials = (size_t) splits * ((size_t) s.K() * s.F + (size_t) s.F);
@@ -3100,7 +3125,10 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 		p.splits = b3.splits;
 	T* bias_partials = partials + (size_t) p.splits * count;
 	static_assert(WGRAD_MC == 32, "the chunk length gather_with_wgrad_kernel is built with");
-	const bool can_ride = elsewhere != nullptr && !bf16x3 && std::is_same<T, float>::value && !act && vec && v.bk == 32 && v.bf == 32 &&
+	/* (a larger one that stays on the fp32 instructions does not ride: it would hold the input gradient there too, 368 x 1549 x 442
+	 * backward 60 us against 36) */
+	const bool can_ride = elsewhere != nullptr && !bf16x3 && (g.fp32_products || 2.0 * g.M * g.K * g.F < BF16X3_WGRAD_FLOPS) &&
+			std::is_same<T, float>::value && !act && vec && v.bk == 32 && v.bf == 32 &&
 			v.waves == 1 && v.mc == WGRAD_MC;
 	auto run = [&](T* to_w, T* to_b, const WgradSplit& how) {
 		if (few_filters) {
