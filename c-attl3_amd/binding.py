@@ -31,7 +31,7 @@ EXPORTS = [
     "cattle_hip_timer_destroy", "cattle_hip_timer_start", "cattle_hip_timer_stop", "cattle_hip_conv_create",
     "cattle_hip_transconv_create", "cattle_hip_dense_create", "cattle_hip_batchnorm_create", "cattle_hip_batchnorm_get_stats_initialized",
     "cattle_hip_batchnorm_set_stats_initialized", "cattle_hip_activation_create", "cattle_hip_pool_create",
-    "cattle_hip_convlstm_set_multiplicative_integration", "cattle_hip_convlstm_fused_steps", "cattle_hip_layer_param_set_regularization",
+    "cattle_hip_convlstm_set_multiplicative_integration", "cattle_hip_convlstm_fused_steps", "cattle_hip_last_products", "cattle_hip_layer_param_set_regularization",
     "cattle_hip_layer_param_regularization_penalty", "cattle_hip_dropout_create", "cattle_hip_reshape_create", "cattle_hip_broadcast_create",
     "cattle_hip_layer_clone", "cattle_hip_layer_destroy", "cattle_hip_layer_input_dims",
     "cattle_hip_layer_output_dims", "cattle_hip_layer_is_input_layer", "cattle_hip_layer_set_input_layer",
@@ -188,6 +188,14 @@ def conv_forward_noalloc(x, weights, bias, out, receptor_height=3, receptor_widt
         _dtype_code(x.dtype), _sz(N), _sz(H), _sz(W), _sz(C), _sz(F), _sz(receptor_height), _sz(receptor_width),
         _sz(vertical_padding), _sz(horizontal_padding), _sz(vertical_stride), _sz(horizontal_stride), _sz(vertical_dilation),
         _sz(horizontal_dilation), x.ptr, weights.ptr, None if bias is None else bias.ptr, out.ptr))
+
+
+def last_products():
+    """(product, weight gradient): rows * 1000 + columns of the tile that the last forward or input-gradient product and the
+    last weight gradient of a kernel layer took on the bf16 matrix instructions, 0 where they ran on others."""
+    p, w = ctypes.c_int(), ctypes.c_int()
+    _check(lib().cattle_hip_last_products(ctypes.byref(p), ctypes.byref(w)))
+    return int(p.value), int(w.value)
 
 
 class Timer(object):

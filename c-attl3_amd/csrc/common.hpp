@@ -90,6 +90,11 @@ struct ConvShape {
 	int K() const { return RH * RW * C; }
 };
 
+/* What the last launches of a kernel layer ran on (cattle_hip_last_products): rows * 1000 + columns of the tile on the bf16
+ * instructions, 0 on others. */
+struct LastProducts { int product = 0, weight_gradient = 0; };
+extern LastProducts g_last_products;
+
 /* Sizes of the scratch buffers the GEMM launchers need for a batch of N (in elements of T). */
 struct ConvWorkspace {
 	size_t wt_fwd;      /* prepared forward weights  */

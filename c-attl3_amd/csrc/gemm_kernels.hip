@@ -35,6 +35,8 @@
 
 namespace cattle_hip {
 
+LastProducts g_last_products;
+
 namespace {
 
 /* Where gathered loads that fall into the zero padding are pointed at. */
@@ -2146,6 +2148,16 @@ StepTimes fp32_step_times(const GatherVariant<T>& v, int resident, bool vec) {
 	return { resident * chunk * (0.74 * area + 0.62 * edges), 1.63 * chunk, 3.3 + 0.31 * area * resident };
 }
 
+/* Of the bf16 variants, which have their own table: rows * 1000 + columns, else 0 */
+template<typename T>
+int bf16x3_label(const GatherVariant<T>& v) {
+	if constexpr (std::is_same<T, float>::value)
+		for (int i = 0; i < BF16X3_TILES; ++i)
+			if (&v == &bf16x3_variants()[i])
+				return v.bm * 1000 + v.bf;
+	return 0;
+}
+
 /* The tile of gather_gemm_bf16x3_kernel for a problem (of M rows in all: the classes of a strided gradient count together,
  * and cut no reductions), or null where the fp32 launch stays: what the kernel cannot address; problems of a few microseconds,
  * which launches and waits make up (364 x 61 x 110 took 6.0 us there, 6.5 here); and reductions of up to four chunks where
@@ -2200,6 +2212,7 @@ template<typename T>
 bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const GatherProblem& g, ScratchArena* arena = nullptr,
 		int epi = EPI_NONE, const Epilogue<T>* E = nullptr, int* mtiles_out = nullptr, const LstmBackwardStep<T>* then = nullptr,
 		bool* then_done = nullptr, const std::function<void(int bf)>* before_launch = nullptr, WgradRider<T>* rider = nullptr) {
+	g_last_products.product = 0;
 	const bool vec = g.N % GemmCfg<T>::VEC == 0 && g.NS % GemmCfg<T>::VEC == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
 	const bool divs = g.DA != 1 || g.DB != 1;
 	if (epi != EPI_NONE && (!vec || divs || (reinterpret_cast<uintptr_t>(out) & 15) != 0))
@@ -2429,6 +2442,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 			partials = static_cast<T*>(arena ? arena->take(cut.partial_bytes, "partial sums of the split reduction") : split_workspace(cut.partial_bytes));
 		dim3 grid((unsigned) (L.main_blocks + L.split_count * L.ksplit), (unsigned) ftiles);
 		v.launch(grid, dyn, src, wt, bias, out, g, L, partials, vec, divs, epi, epi_args);
+		g_last_products.product = bf16x3_label<T>(v);
 		if (L.split_count > 0) {
 			const int groups = v.bm * v.bf / (256 * (16 / (int) sizeof(T)));
 			const dim3 rgrid((unsigned) (L.split_count * ftiles * groups));
@@ -2562,6 +2576,7 @@ bool launch_gather_classes(const T* src, T* out, const std::vector<GatherProblem
 		table.L[i] = table.L[0];
 		table.wt[i] = weights[0];
 	}
+	g_last_products.product = bf16x3_label<T>(v);
 	v.launch_classes(dim3(blocks, (unsigned) ((F + v.bf - 1) / v.bf), (unsigned) geoms.size()), src, out, table);
 	return true;
 }
@@ -3121,8 +3136,13 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 	/* fp32 with the gradient as it is: on the bf16 matrix instructions */
 	Bf16x3WgradPlan b3;
 	const bool bf16x3 = std::is_same<T, float>::value && !act && !few_filters && bf16x3_wgrad_plan(g, vec, &b3);
-	if (bf16x3)
+	g_last_products.weight_gradient = 0;
+	if (bf16x3) {
+		int bk, bf;
+		bf16x3_wgrad_tile(b3.shape, &bk, &bf);
+		g_last_products.weight_gradient = bk * 1000 + bf;
 		p.splits = b3.splits;
+	}
 	T* bias_partials = partials + (size_t) p.splits * count;
 	static_assert(WGRAD_MC == 32, "the chunk length gather_with_wgrad_kernel is built with");
 	/* (a larger one that stays on the fp32 instructions does not ride: it would hold the input gradient there too, 368 x 1549 x 442

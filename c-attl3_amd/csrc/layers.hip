@@ -2254,6 +2254,14 @@ int cattle_hip_convlstm_fused_steps(cattle_hip_layer_t lstm, int* forward_steps,
 	});
 }
 
+int cattle_hip_last_products(int* product, int* weight_gradient) {
+	return guarded([&] {
+		CATTLE_HIP_REQUIRE(product != nullptr && weight_gradient != nullptr, "null output pointer");
+		*product = g_last_products.product;
+		*weight_gradient = g_last_products.weight_gradient;
+	});
+}
+
 int cattle_hip_dense_create(cattle_hip_dtype dtype, size_t input_volume, size_t output_size, cattle_hip_layer_t* layer) {
 	return guarded([&] {
 		check_dtype(dtype);

@@ -439,6 +439,10 @@ int cattle_hip_convlstm_set_multiplicative_integration(cattle_hip_layer_t lstm, 
  * multiples of 8 or 16, no multiplicative integration for the forward step); results are the same either way to
  * rounding. */
 int cattle_hip_convlstm_fused_steps(cattle_hip_layer_t lstm, int* forward_steps, int* backward_steps);
+/* Which matrix instructions the last kernel layer's launches ran on (no counterpart in the reference; for tests and profiles):
+ * *product for the last forward or input-gradient product, *weight_gradient for the last weight gradient - the tile's rows *
+ * 1000 + its columns where it multiplied on the bf16 instructions, 0 where on others. */
+int cattle_hip_last_products(int* product, int* weight_gradient);
 
 #ifdef __cplusplus
 }
