@@ -28,9 +28,15 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
-# MI355X dense matrix peaks (no sparsity). f32: fp32 products as six bf16 products each at the bf16 instructions' 2500 (the
-# fp32 instructions' peak, which smaller problems run on, is 157.3)
-PEAK_TFLOPS = {"f32": 416.7, "f64": 78.6}
+# MI355X dense matrix peaks (no sparsity). bf16x3: fp32 products as six bf16 products each, at the bf16 instructions' 2500
+PEAK_TFLOPS = {"f32": 157.3, "bf16x3": 416.7, "f64": 78.6}
+
+
+def product_peak(dtype, tile):
+    """The peak in TFLOP/s of the matrix instructions that a product ran on (`tile`: its entry of last_products)."""
+    return PEAK_TFLOPS["f64" if np.dtype(dtype) == np.float64 else "bf16x3" if tile else "f32"]
+
+
 SHAPE = dict(H=56, W=56, C=64, F=128, RH=3, RW=3)
 
 # HBM bytes per launch (read + written) of the three GEMM kernels come from rocprofv3 FETCH_SIZE and WRITE_SIZE readings
@@ -39,9 +45,9 @@ SHAPE = dict(H=56, W=56, C=64, F=128, RH=3, RW=3)
 # rewrites from the counter runs, together with a hash of the kernel sources they were measured on; a build from other
 # sources reports null.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "conv_cfg4_hbm_traffic.json")
-KERNEL_SOURCES = ("c-attl3_amd/csrc/gemm_kernels.hip", "c-attl3_amd/csrc/gemm_bf16x3.hip", "c-attl3_amd/csrc/gemm_tiles.hpp",
-                  "c-attl3_amd/csrc/gather_epilogue.hpp", "c-attl3_amd/csrc/common.hpp", "c-attl3_amd/csrc/act_math.hpp",
-                  "c-attl3_amd/csrc/lstm_math.hpp")
+KERNEL_SOURCES = ("c-attl3_amd/csrc/gemm_kernels.hip", "c-attl3_amd/csrc/gemm_bf16x3.hip", "c-attl3_amd/csrc/gemm_bf16x3.hpp",
+                  "c-attl3_amd/csrc/gemm_tiles.hpp", "c-attl3_amd/csrc/gather_epilogue.hpp", "c-attl3_amd/csrc/common.hpp",
+                  "c-attl3_amd/csrc/act_math.hpp", "c-attl3_amd/csrc/lstm_math.hpp")
 
 
 def kernel_sources_hash():
@@ -122,7 +128,9 @@ def gpu_run(args, dtype):
         return float(np.median(groups))
 
     t_fwd = timed(lambda: layer.forward_into(x, out, True))
+    tiles = (ch.last_products()[0],)
     t_bwd = timed(lambda: layer.backward_into(go, dx))
+    tiles += ch.last_products()
     layer.set_input_layer(True)
     t_wgrad = timed(lambda: layer.backward_into(go, None))         # weight + bias gradient only
     layer.set_input_layer(False)
@@ -133,6 +141,8 @@ def gpu_run(args, dtype):
         "weight gradient (+ reduce, bias column sums)": t_wgrad,
         "gather GEMM (input gradient)": t_dgrad,
     }
+    peaks = dict(zip(("gather GEMM (forward)", "gather GEMM (input gradient)", "weight gradient (+ reduce, bias column sums)"),
+                     (product_peak(dtype, t) for t in tiles)))
     es = np.dtype(dtype).itemsize
     in_b, out_b, w_b = N * H * W * C * es, N * H * W * F * es, K * F * es
     nbytes = {
@@ -149,7 +159,7 @@ def gpu_run(args, dtype):
         ch.synchronize()
     for t in (x, go, out, dx):
         t.free()
-    return dict(wall_ms=wall_ms, walls=walls, M=M, K=K, F=F, gemm_flop=gemm_flop, kernels=kernels, bytes=nbytes)
+    return dict(wall_ms=wall_ms, walls=walls, M=M, K=K, F=F, gemm_flop=gemm_flop, kernels=kernels, bytes=nbytes, peaks=peaks)
 
 
 def host_tensor_run(args, dtype):
@@ -200,7 +210,6 @@ def small_convs_run(args, dtype):
     ch = importlib.import_module("c-attl3_amd")
     ch.init(0)
     es = np.dtype(dtype).itemsize
-    peak = PEAK_TFLOPS[args.dtype] * 1e12
     shapes = [
         ("configs[0] conv 64x32x32x3 -> 16", 64, 32, 32, 3, 16),
         ("configs[2] conv1 128x32x32x3 -> 32", 128, 32, 32, 3, 32),
@@ -232,21 +241,24 @@ def small_convs_run(args, dtype):
             return timer.stop() / reps
 
         t_fwd = timed(lambda: layer.forward_into(x, out, True)) if args.passes in ("both", "fwd") else float("nan")
+        fwd_tiles = (ch.last_products()[0],)
         if args.passes in ("both", "bwd"):
             layer.forward_into(x, out, True)
             t_bwd = timed(lambda: layer.backward_into(go, dx))
         else:
             t_bwd = float("nan")
+        bwd_tiles = ch.last_products()
         in_b, out_b, w_b = M * C * es, M * F * es, K * F * es
         flop = 2.0 * M * K * F
-        for pass_name, t_ms, launches, nbytes in (("forward", t_fwd, 1, in_b + w_b + out_b),
-                                                  ("backward (weight, bias and input gradients)", t_bwd, 2, 2 * (in_b + out_b + w_b))):
+        for pass_name, t_ms, tiles, nbytes in (("forward", t_fwd, fwd_tiles, in_b + w_b + out_b),
+                                               ("backward (weight, bias and input gradients)", t_bwd, bwd_tiles, 2 * (in_b + out_b + w_b))):
             if t_ms != t_ms:
                 continue
-            roof_s = max(launches * flop / peak, nbytes / 8e12)
+            launches, mfma_s = len(tiles), sum(flop / (product_peak(dtype, t) * 1e12) for t in tiles)
+            roof_s = max(mfma_s, nbytes / 8e12)
             rows.append({"layer": name, "pass": pass_name, "M": M, "K": K, "F": F, "ms": round(t_ms, 4),
                          "gflops": round(launches * flop / (t_ms * 1e-3) / 1e9, 1), "GB/s": round(nbytes / (t_ms * 1e-3) / 1e9, 1),
-                         "bound": "mfma" if launches * flop / peak >= nbytes / 8e12 else "hbm",
+                         "bound": "mfma" if mfma_s >= nbytes / 8e12 else "hbm",
                          "roofline_us": round(roof_s * 1e6, 2), "frac_of_roofline": round(roof_s / (t_ms * 1e-3), 4)})
         for t in (x, go, out, dx):
             t.free()
@@ -295,7 +307,7 @@ def conv_shapes_run(args, dtype):
     rows = []
     for name, kind, N, H, W, C, F, RH, RW, pv, ph, sv, sh, dv, dh, fp64 in shapes:
         dt = np.float64 if (fp64 or args.dtype == "f64") else np.float32
-        es, peak = np.dtype(dt).itemsize, PEAK_TFLOPS["f64" if dt == np.float64 else "f32"] * 1e12
+        es = np.dtype(dt).itemsize
         if kind == "dense":
             layer = ch.DenseKernelLayer(dt, (C,), F)
             in_shape, K = (N, C), C
@@ -325,19 +337,22 @@ def conv_shapes_run(args, dtype):
             return timer.stop() / reps
 
         t_fwd = timed(lambda: layer.forward_into(x, out, True)) if args.passes in ("both", "fwd") else None
+        fwd_tiles = (ch.last_products()[0],)
         t_bwd = None
         if args.passes in ("both", "bwd"):
             layer.forward_into(x, out, True)
             t_bwd = timed(lambda: layer.backward_into(go, dx))
         in_b, out_b, w_b = int(np.prod(in_shape)) * es, int(np.prod(out_shape)) * es, wp.get_rows() * wp.get_cols() * es
         flop = 2.0 * M * K * cols
-        for pass_name, t_ms, launches, nbytes in (("fwd", t_fwd, 1, in_b + w_b + out_b), ("bwd", t_bwd, 2, 2 * (in_b + out_b + w_b))):
+        bwd_tiles = ch.last_products()
+        for pass_name, t_ms, tiles, nbytes in (("fwd", t_fwd, fwd_tiles, in_b + w_b + out_b), ("bwd", t_bwd, bwd_tiles, 2 * (in_b + out_b + w_b))):
             if t_ms is None:
                 continue
-            roof_s = max(launches * flop / peak, nbytes / 8e12)
+            launches, mfma_s = len(tiles), sum(flop / (product_peak(dt, t) * 1e12) for t in tiles)
+            roof_s = max(mfma_s, nbytes / 8e12)
             rows.append({"layer": name, "pass": pass_name, "M": M, "K": K, "F": cols, "dtype": np.dtype(dt).name,
                          "us": round(t_ms * 1e3, 2), "tflops": round(launches * flop / (t_ms * 1e-3) / 1e12, 2),
-                         "bound": "mfma" if launches * flop / peak >= nbytes / 8e12 else "hbm",
+                         "bound": "mfma" if mfma_s >= nbytes / 8e12 else "hbm",
                          "roofline_us": round(roof_s * 1e6, 2), "frac_of_roofline": round(roof_s / (t_ms * 1e-3), 4)})
         for t in (x, go, out, dx):
             t.free()
@@ -837,7 +852,7 @@ def main():
     r = gpu_run(args, dtype)
     step_flop = 3.0 * r["gemm_flop"]
     gflops = step_flop / (r["wall_ms"] * 1e-3) / 1e9
-    peak = PEAK_TFLOPS[args.dtype]
+    peak = 3.0 / sum(1.0 / p for p in r["peaks"].values())           # of the three products together
     name, t_ms = max(r["kernels"].items(), key=lambda kv: kv[1])
     achieved = r["gemm_flop"] / (t_ms * 1e-3) / 1e12
     line = {
@@ -849,8 +864,8 @@ def main():
                    "M": r["M"], "K": r["K"], "F": r["F"], "flop_per_step": step_flop},
         "samples_per_s": round(args.batch / (r["wall_ms"] * 1e-3), 1),
         "frac_of_mfma_peak": round(gflops / 1e3 / peak, 4),
-        "roofline": {"bound": "mfma", "kernel": name, "achieved": round(achieved, 2), "peak": peak, "unit": "TFLOP/s",
-                     "frac": round(achieved / peak, 4),
+        "roofline": {"bound": "mfma", "kernel": name, "achieved": round(achieved, 2), "peak": r["peaks"][name], "unit": "TFLOP/s",
+                     "frac": round(achieved / r["peaks"][name], 4),
                      "traffic": None,
                      "algorithmic_bytes": r["bytes"][name],
                      "flop_per_launch": r["gemm_flop"], "ms_per_launch": round(t_ms, 4)},
