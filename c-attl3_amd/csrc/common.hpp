@@ -285,11 +285,11 @@ size_t conv_stats_rows(const ConvShape& s, int N);
 /* The output-side kernels of an LSTM cell step (s.F = 4 * hidden filters: forget | write | candidate | read) on the
  * previous hidden output x (the first N of x_batch samples per position if x_batch > 0), followed in the same kernel
  * by the element-wise part of the step: the weighted previous outputs never reach memory. `wt` (conv_workspace().wt_fwd
- * elements) is a prepared layout of its own, not the one conv_forward builds. Returns false, having launched nothing
- * and leaving wt alone, when the problem does not allow it (no 16-byte accesses, too many rows for the short tiles
+ * elements) is a prepared layout of its own, not the one conv_forward builds; *gate_block is the gate block (lstm_gate_column)
+ * of the layout that it holds, 0 for none that is current. Returns false, having launched nothing and leaving both alone, when the problem does not allow it (no 16-byte accesses, too many rows for the short tiles
  * that can stage a whole tile, a hidden size that does not fill tiles with whole gate groups). */
 template<typename T> bool conv_forward_lstm(const ConvShape& s, int N, const T* x, int x_batch, const T* w, const T* b, T* wt,
-		bool wt_ready, const LstmForwardStep<T>& step);
+		int* gate_block, const LstmForwardStep<T>& step);
 /* The layers behind the kernel layer, on its output z (N, H, W, C): element-wise activation `kind` (argument p) and a
  * pool (0 none, 1 max, 2 mean) whose prh x prw windows tile z exactly. */
 struct ChainShape {

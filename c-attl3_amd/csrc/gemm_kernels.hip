@@ -19,6 +19,7 @@
 #include "common.hpp"
 #include "gather_epilogue.hpp"
 #include "gemm_bf16x3.hpp"
+#include "lstm_steps.hpp"
 #include "gemm_tiles.hpp"
 #include "act_math.hpp"
 #include "lstm_math.hpp"
@@ -3012,7 +3013,7 @@ void conv_forward(const ConvShape& s, int N, const T* x, const T* w, const T* b,
 }
 
 template<typename T>
-bool conv_forward_lstm(const ConvShape& s, int N, const T* x, int x_batch, const T* w, const T* b, T* wt, bool wt_ready,
+bool conv_forward_lstm(const ConvShape& s, int N, const T* x, int x_batch, const T* w, const T* b, T* wt, int* gate_block,
 		const LstmForwardStep<T>& step) {
 	check_sizes(s, std::max(N, x_batch));
 	GatherProblem g = forward_geom(s, N);
@@ -3021,13 +3022,20 @@ bool conv_forward_lstm(const ConvShape& s, int N, const T* x, int x_batch, const
 	Epilogue<T> E = { 0, (T) 0, nullptr, nullptr, 1, 1, 1, 1, nullptr, step };
 	/* the prepared columns depend on the tile width, which the launcher chooses */
 	const std::function<void(int)> prepare = [&](int bf) {
-		if (wt_ready)
+		if (*gate_block == bf / 4)
 			return;
 		const int Kp = round_up(g.K, WT_ROW_PAD);
 		const size_t count = (size_t) Kp * g.ldw;
 		prep_fwd_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, g.K, g.F, Kp, g.ldw, bf / 4);
 		CATTLE_HIP_CHECK(hipGetLastError());
+		*gate_block = bf / 4;
 	};
+	if constexpr (std::is_same<T, float>::value)
+		if (lstm_step_forward_possible(g, step, device_shape().cus)) {
+			prepare(4 * LSTM_STEP_GATE_BLOCK);
+			lstm_step_forward(x, wt, b, g, step);
+			return true;
+		}
 	return launch_gather<T>(x, wt, b, (T*) nullptr, g, nullptr, EPI_LSTM, &E, nullptr, nullptr, nullptr, &prepare);
 }
 
@@ -3300,6 +3308,11 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 				Kp, d.ldw);
 		CATTLE_HIP_CHECK(hipGetLastError());
 	}
+	if constexpr (std::is_same<T, float>::value)
+		if (then != nullptr && lstm_step_backward_possible(d, *then, device_shape().cus)) {
+			lstm_step_backward(out_grad, wt_dgrad, d, *then);
+			return true;
+		}
 	bool then_done = false;
 	launch_gather<T>(out_grad, wt_dgrad, (const T*) nullptr, in_grad, d, nullptr, EPI_NONE, nullptr, nullptr, then, &then_done, nullptr, rider);
 	return then_done;
@@ -3330,9 +3343,9 @@ template bool conv_forward_fused<float>(const ConvShape&, int, const float*, con
 		const Epilogue<float>&, int*);
 template bool conv_forward_fused<double>(const ConvShape&, int, const double*, const double*, const double*, double*, double*, bool, int,
 		const Epilogue<double>&, int*);
-template bool conv_forward_lstm<float>(const ConvShape&, int, const float*, int, const float*, const float*, float*, bool,
+template bool conv_forward_lstm<float>(const ConvShape&, int, const float*, int, const float*, const float*, float*, int*,
 		const LstmForwardStep<float>&);
-template bool conv_forward_lstm<double>(const ConvShape&, int, const double*, int, const double*, const double*, double*, bool,
+template bool conv_forward_lstm<double>(const ConvShape&, int, const double*, int, const double*, const double*, double*, int*,
 		const LstmForwardStep<double>&);
 template void conv_forward_static<float>(const ConvShape&, int, const float*, const float*, const float*, float*);
 template void conv_forward_static<double>(const ConvShape&, int, const double*, const double*, const double*, double*);

@@ -261,6 +261,7 @@ struct Param {
 	DevBuf derived[3];
 	uint64_t derived_version[3] = { 0, 0, 0 };
 	int dgrad_layout = 0;              /* which layout derived[1] holds (dgrad_weight_layout) */
+	int gate_block = 0;                /* and derived[2] of a recurrent kernel (conv_forward_lstm) */
 	/* A weight matrix: the partial sums of the last weight-gradient launch that was cut into slices (its own and, behind
 	 * them, those of the bias gradient). They are added to the gradients when a gradient is first needed - by the
 	 * optimizer step as a rule, in one launch for all layers - and until then `pending` lists them (see Deferred). */
@@ -738,8 +739,10 @@ struct ConvLstm : LayerBase {
 				 * the backward pass reads it, so it has to be stored) */
 				if (!wth_gates)
 					wth_gates = (T*) wh.derived[2].ensure(wsh.wt_fwd * e);
+				int block = wh.derived_version[2] == wh.version ? wh.gate_block : 0;
 				if (conv_forward_lstm<T>(sh, n, hprev, (int) (N * total), (const T*) wh.values.p, (const T*) params[3]->values.p,
-						wth_gates, wh.derived_version[2] == wh.version, fs)) {
+						wth_gates, &block, fs)) {
+					wh.gate_block = block;
 					wh.derived_version[2] = wh.version;
 					++fused_forward_steps;
 					continue;

@@ -103,16 +103,21 @@ __host__ __device__ __forceinline__ int lstm_gate_column(int f, int cb, int hidd
 /* What the forward step of an element reads besides the weighted previous output. */
 template<typename T> struct LstmForwardInputs { T zx[4]; T prev; };
 
+/* (n, rest: e = n + N rest, and slab_rows = P / N, for a kernel that has them at hand: two 32-bit divisions otherwise) */
 template<typename T>
-__device__ __forceinline__ LstmForwardInputs<T> lstm_forward_load(const LstmForwardStep<T>& A, unsigned e) {
-	const unsigned N = (unsigned) A.N, slab_rows = (unsigned) A.P / N;
-	const unsigned rest = e / N, n = e - rest * N;
+__device__ __forceinline__ LstmForwardInputs<T> lstm_forward_load_at(const LstmForwardStep<T>& A, unsigned e, unsigned n, unsigned rest,
+		unsigned slab_rows) {
 	LstmForwardInputs<T> in;
 	#pragma unroll
 	for (int g = 0; g < 4; ++g)
 		in.zx[g] = A.zx ? lstm_ld<T>(A.zx, seq_offset(n, rest + g * slab_rows, A.N, A.zx_T, A.zx_t)) : (T) 0;
 	in.prev = A.prev_state ? lstm_ld<T>(A.prev_state, e) : (T) 0;
 	return in;
+}
+template<typename T>
+__device__ __forceinline__ LstmForwardInputs<T> lstm_forward_load(const LstmForwardStep<T>& A, unsigned e) {
+	const unsigned N = (unsigned) A.N, rest = e / N;
+	return lstm_forward_load_at<T>(A, e, e - rest * N, rest, (unsigned) A.P / N);
 }
 
 /* What the forward step of an element writes: the gates' pre-activation values and values, the state, the activated
@@ -147,9 +152,9 @@ __device__ __forceinline__ LstmForwardOutputs<T> lstm_forward_compute(const Lstm
 }
 
 template<typename T>
-__device__ __forceinline__ void lstm_forward_store(const LstmForwardStep<T>& A, unsigned e, const LstmForwardOutputs<T>& o) {
-	const unsigned N = (unsigned) A.N, P = (unsigned) A.P;
-	const unsigned rest = e / N, n = e - rest * N;
+__device__ __forceinline__ void lstm_forward_store_at(const LstmForwardStep<T>& A, unsigned e, unsigned n, unsigned rest,
+		const LstmForwardOutputs<T>& o) {
+	const unsigned P = (unsigned) A.P;
 	#pragma unroll
 	for (int g = 0; g < 4; ++g) {
 		if (A.z)
@@ -166,6 +171,11 @@ __device__ __forceinline__ void lstm_forward_store(const LstmForwardStep<T>& A, 
 	}
 	if (A.out)
 		lstm_st<T>(A.out, seq_offset(n, rest, A.N, A.out_T, A.out_t), o.h);
+}
+template<typename T>
+__device__ __forceinline__ void lstm_forward_store(const LstmForwardStep<T>& A, unsigned e, const LstmForwardOutputs<T>& o) {
+	const unsigned N = (unsigned) A.N, rest = e / N;
+	lstm_forward_store_at<T>(A, e, e - rest * N, rest, o);
 }
 
 /* The same for V consecutive elements e0 .. e0 + V - 1 (e0 and N multiples of V, so they are V consecutive samples of
@@ -289,9 +299,9 @@ __device__ __forceinline__ bool lstm_backward_can_preload(const LstmBackwardStep
 	return A.z == nullptr && A.zx_fwd == nullptr;
 }
 template<typename T>
-__device__ __forceinline__ LstmBackwardInputs<T> lstm_backward_load(const LstmBackwardStep<T>& A, unsigned e, bool has_dh) {
-	const unsigned N = (unsigned) A.N, P = (unsigned) A.P;
-	const unsigned rest = e / N, n = e - rest * N;
+__device__ __forceinline__ LstmBackwardInputs<T> lstm_backward_load_at(const LstmBackwardStep<T>& A, unsigned e, unsigned n, unsigned rest,
+		bool has_dh) {
+	const unsigned P = (unsigned) A.P;
 	LstmBackwardInputs<T> in;
 	in.og = A.out_grad ? lstm_ld<T>(A.out_grad, seq_offset(n, rest, A.N, A.og_T, A.og_t)) : (T) 0;
 	#pragma unroll
@@ -303,13 +313,15 @@ __device__ __forceinline__ LstmBackwardInputs<T> lstm_backward_load(const LstmBa
 	in.prev = A.prev_state ? lstm_ld<T>(A.prev_state, e) : (T) 0;
 	return in;
 }
+template<typename T>
+__device__ __forceinline__ LstmBackwardInputs<T> lstm_backward_load(const LstmBackwardStep<T>& A, unsigned e, bool has_dh) {
+	const unsigned N = (unsigned) A.N, rest = e / N;
+	return lstm_backward_load_at<T>(A, e, e - rest * N, rest, has_dh);
+}
 /* The step itself on preloaded inputs: the same arithmetic, in the same order, as lstm_backward_element below. */
 template<typename T, bool STD = false>
-__device__ __forceinline__ void lstm_backward_finish(const LstmBackwardStep<T>& A, unsigned e, bool has_dh, T dh,
-		const LstmBackwardInputs<T>& in) {
-	const unsigned N = (unsigned) A.N, P = (unsigned) A.P;
-	const unsigned slab_rows = P / N;
-	const unsigned rest = e / N, n = e - rest * N;
+__device__ __forceinline__ void lstm_backward_finish_at(const LstmBackwardStep<T>& A, unsigned e, unsigned n, unsigned rest, unsigned slab_rows,
+		bool has_dh, T dh, const LstmBackwardInputs<T>& in) {
 	T hg = has_dh ? dh : (T) 0;
 	if (A.out_grad)
 		hg += in.og;
@@ -329,6 +341,12 @@ __device__ __forceinline__ void lstm_backward_finish(const LstmBackwardStep<T>& 
 		if (A.dzh_all)
 			lstm_st<T>(A.dzh_all, seq_offset(n, rest + g * slab_rows, A.N, A.h_T, A.h_t), A.prev_state ? d[g] : (T) 0);
 	}
+}
+template<typename T, bool STD = false>
+__device__ __forceinline__ void lstm_backward_finish(const LstmBackwardStep<T>& A, unsigned e, bool has_dh, T dh,
+		const LstmBackwardInputs<T>& in) {
+	const unsigned N = (unsigned) A.N, rest = e / N;
+	lstm_backward_finish_at<T, STD>(A, e, e - rest * N, rest, (unsigned) A.P / N, has_dh, dh, in);
 }
 
 /* Backward step of element e. dh: the gradient of the element's hidden output that came back through the next

@@ -215,3 +215,14 @@ def test_a_network_reused_with_another_sequence_length():
     assert np.array_equal(used.backpropagate(go), fresh.backpropagate(go))
     for a, b in zip(used.get_params(), fresh.get_params()):
         assert np.array_equal(a.get_grad(), b.get_grad())
+
+
+@pytest.mark.parametrize("hidden", [8, 16, 24, 32, 40, 48])
+@pytest.mark.parametrize("N,dims,conv_kw", [(4, (3, 3, 1), {}), (12, (7, 5, 2), {}), (8, (9, 8, 3), dict(RH=3, RW=3, pv=2, ph=3, dv=1, dh=2))],
+                         ids=["36 rows", "420 rows", "dilated"])
+def test_steps_of_a_three_by_three_cell(N, dims, conv_kw, hidden):
+    """The kernels of a whole time step (fp32, 3 x 3 receptor, hidden channels in eights up to 48): every count of channels
+    per wavefront, last tiles of rows that are not full, column tiles and groups of gates that are not, positions whose
+    receptor lies mostly in the padding."""
+    net, _, _ = _check(np.float32, N, 3, dims, hidden, SMOOTH, False, lambda T: (T, 0), conv_kw=conv_kw)
+    assert net.fused_steps() == (2, 2)
