@@ -85,6 +85,8 @@ struct ConvShape {
 	/* The fp32 matrix instructions for all products of a call, also where the bf16 ones would serve (FusedLayer::shape and
 	 * weight_gradient_workspace say who asks for them, and why). */
 	bool fp32_products = false;
+	/* The sums of the forward product in the order that the tiled launches take them (FusedLayer::shape says who asks for it). */
+	bool keeps_sums = false;
 	int OH() const { return (H - RH - (RH - 1) * dv + 2 * pv) / sv + 1; }
 	int OW() const { return (W - RW - (RW - 1) * dh + 2 * ph) / sh + 1; }
 	int K() const { return RH * RW * C; }

@@ -20,6 +20,7 @@
 #include "gather_epilogue.hpp"
 #include "gemm_bf16x3.hpp"
 #include "lstm_steps.hpp"
+#include "small_dense.hpp"
 #include "gemm_tiles.hpp"
 #include "act_math.hpp"
 #include "lstm_math.hpp"
@@ -2079,6 +2080,7 @@ void launch_wave_split_variant(const T* src, const T* wt, const T* bias, T* out,
 /* A gathered GEMM and what the host alone asks about it (kernels are given the geometry). */
 struct GatherProblem : GatherGeom {
 	bool fp32_products = false;     /* ConvShape::fp32_products */
+	bool keeps_sums = false;        /* ConvShape::keeps_sums */
 };
 
 /* Which tiles of a launch have their reduction cut into parts, and the memory that the parts' sums take. */
@@ -2216,6 +2218,17 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 	g_last_products.product = 0;
 	const bool vec = g.N % GemmCfg<T>::VEC == 0 && g.NS % GemmCfg<T>::VEC == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
 	const bool divs = g.DA != 1 || g.DB != 1;
+	/* a dense layer's product with few tiles; where a weight gradient would ride in the launch only if it cannot (below) */
+	const auto small_dense_product = [&]() {
+		if constexpr (std::is_same<T, float>::value)
+			if ((epi == EPI_NONE || epi == EPI_ACT) && then == nullptr && !g.keeps_sums && small_product_possible(g, device_shape().cus)) {
+				small_product(src, wt, bias, out, g, round_up(g.K, WT_ROW_PAD), epi == EPI_ACT ? E : nullptr, device_shape().cus);
+				return true;
+			}
+		return false;
+	};
+	if (!rider && small_dense_product())
+		return true;
 	if (epi != EPI_NONE && (!vec || divs || (reinterpret_cast<uintptr_t>(out) & 15) != 0))
 		return false;
 	/* 16-byte loads wherever alignment allows, even where they leave a SIMD a wave or two: measured, a quarter of
@@ -2463,10 +2476,17 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 		/* far fewer tiles than the chip holds blocks: the reduction of every tile is dealt to the wavefronts of one block
 		 * where it is short enough for that (wave_split_gemm_kernel: one launch, no partial sums in memory), else cut into
 		 * parts, one block each, which a second launch adds up */
+		if (small_dense_product())
+			return true;
 		const bool lstm_tail = then != nullptr && epi == EPI_NONE && bias == nullptr && (size_t) g.M * g.F == then->P;
 		const int tail = lstm_tail ? WS_LSTM_BACKWARD : epi == EPI_ACT ? WS_ACT : WS_PLAIN;
 		const int waves = ((divs && tail != WS_PLAIN) || tune.no_wave_split) ? 0 : wave_split_waves<T>(g);
 		if (waves > 0) {
+			if constexpr (std::is_same<T, float>::value)
+				if (tail != WS_LSTM_BACKWARD && addressable_product(g)) {
+					small_product_ordered(src, wt, bias, out, g, round_up(g.K, WT_ROW_PAD), epi == EPI_ACT ? E : nullptr, waves);
+					return true;
+				}
 			if (waves == 16)
 				launch_wave_split_variant<T, 16>(src, wt, bias, out, g, divs, tail, epi_args, then);
 			else if (waves == 8)
@@ -2598,6 +2618,7 @@ GatherProblem forward_geom(const ConvShape& s, int N) {
 	g.M = N * g.OA * g.OB; g.K = s.K(); g.F = s.F;
 	g.ldw = round_up(s.F, WT_COL_PAD);
 	g.fp32_products = s.fp32_products;
+	g.keeps_sums = s.keeps_sums;
 	plain_output(g);
 	return g;
 }
@@ -2703,20 +2724,26 @@ struct WgradVariant {
 	int (*blocks_per_cu)();         /* what the runtime says fits on a CU (registers and LDS) */
 };
 
+/* The derivative on the negative side, p0 + p1 * y, that a weight-gradient launch applies to the gradient it loads. */
+template<typename T>
+void negative_side(const WgradAct<T>* act, T* p0, T* p1) {
+	*p0 = *p1 = (T) 0;
+	if (act && act->pool_inds && act->kind < 0) {
+		*p0 = (T) 1;            /* no activation behind the pool: slope one on either side */
+	} else if (act) {
+		CATTLE_HIP_REQUIRE(act_sign_coded(act->kind) && act->p >= (T) 0, "only a rectifier can be undone while the gradient is loaded");
+		*p0 = act->kind == ACT_RELU ? (T) 0 : act->p;
+		*p1 = act->kind == ACT_ELU ? (T) 1 : (T) 0;
+	}
+}
+
 template<typename T, int WK, int WF, int TK, int TF, int MINW = 1, int MC = WGRAD_MC>
 void launch_wgrad_variant(const T* x, const T* og, T* partials, T* bias_partials, const GatherGeom& g, const WgradSplit& plan,
 		bool vec, const WgradAct<T>* act) {
 	constexpr int VEC = GemmCfg<T>::VEC;
 	dim3 block(64 * WK * WF), grid((unsigned) round_up(plan.tiles * plan.splits, 8));
-	/* derivative on the negative side: p0 + p1 * y */
-	T p0 = (T) 0, p1 = (T) 0;
-	if (act && act->pool_inds && act->kind < 0) {
-		p0 = (T) 1;             /* no activation behind the pool: slope one on either side */
-	} else if (act) {
-		CATTLE_HIP_REQUIRE(act_sign_coded(act->kind) && act->p >= (T) 0, "only a rectifier can be undone while the gradient is loaded");
-		p0 = act->kind == ACT_RELU ? (T) 0 : act->p;
-		p1 = act->kind == ACT_ELU ? (T) 1 : (T) 0;
-	}
+	T p0, p1;
+	negative_side(act, &p0, &p1);
 	if (act && act->pool_inds) {
 		CATTLE_HIP_REQUIRE(vec && act->dz == nullptr, "the weight gradient from a pooled gradient needs 16-byte loads and forms no full-size gradient");
 		wgrad_pooled_kernel<T, WK, WF, TK, TF, MC, VEC><<<grid, block, 0, stream()>>>(x, og, partials, bias_partials, g, plan, act->y, p0, p1,
@@ -3158,6 +3185,13 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 	const bool can_ride = elsewhere != nullptr && !bf16x3 && (g.fp32_products || 2.0 * g.M * g.K * g.F < BF16X3_WGRAD_FLOPS) &&
 			std::is_same<T, float>::value && !act && vec && v.bk == 32 && v.bf == 32 &&
 			v.waves == 1 && v.mc == WGRAD_MC;
+	if constexpr (std::is_same<T, float>::value)
+		if (!can_ride && !bf16x3 && small_weight_gradient_possible(g, vec, act)) {
+			T p0, p1;
+			negative_side(act, &p0, &p1);
+			small_weight_gradient(x, out_grad, wgrad, bgrad, g, act, p0, p1);
+			return;
+		}
 	auto run = [&](T* to_w, T* to_b, const WgradSplit& how) {
 		if (few_filters) {
 			const dim3 grid((unsigned) ((g.LC + 3) / 4), (unsigned) how.splits);

@@ -1101,10 +1101,15 @@ struct FusedLayer : LayerBase {
 	 * 32 x 3, Adam) the parameters of the two kinds of instruction come out up to 1e-2 (2-norm) apart. Not because the fp32
 	 * ones were the more accurate: over 20 seeds they are 1.7e-4 from 64 bits in the median, the bf16 ones 1.4e-5, and 1.1e-2
 	 * at the worst with either. It leaves trained results where they were; a large layer pays for it in time.
+	 * A rectifier in a training pass asks for less: its forward products keep the order of their sums. Which side of zero a
+	 * value falls on decides whether its gradient passes, and of the million values of a few batches of an MLP (784-512-256-10, eight
+	 * batches of 256) another order of the sums moves one across now and then: the trained parameters are then 1.5e-4 from where
+	 * they were (2e-7 without such a value), with neither side the more accurate.
 	 * The member layer itself is not touched: called alone it chooses like any other. */
-	ConvShape shape() const {
+	ConvShape shape(bool training = false) const {
 		ConvShape s = conv->shape;
 		s.fp32_products = pool && pool->kind == CATTLE_HIP_POOL_MAX;
+		s.keeps_sums = s.fp32_products || (training && act && (act_sign_coded(act->kind) || act->kind == CATTLE_HIP_ACT_BINARY_STEP));
 		return s;
 	}
 	int OH() const { return conv->shape.OH(); }
@@ -1170,7 +1175,7 @@ struct FusedLayer : LayerBase {
 			bool ok = true;
 			if (training) {
 				E.stats = (T*) stats_buf.ensure(conv_stats_rows(conv->shape, n) * F() * 3 * sizeof(T));
-				ok = conv_forward_fused<T>(shape(), n, x, wv, bv, z, wt, ready, EPI_STATS, E, &mtiles);
+				ok = conv_forward_fused<T>(shape(training), n, x, wv, bv, z, wt, ready, EPI_STATS, E, &mtiles);
 				weights_prepared();
 			}
 			if (!ok) {
@@ -1178,7 +1183,7 @@ struct FusedLayer : LayerBase {
 				return;
 			}
 			if (!training) {
-				conv_forward<T>(shape(), n, x, wv, bv, z, wt, ready);
+				conv_forward<T>(shape(training), n, x, wv, bv, z, wt, ready);
 				weights_prepared();
 			}
 			pool_in_chain = pool_tiles();
@@ -1227,7 +1232,7 @@ struct FusedLayer : LayerBase {
 				E.inds = (unsigned*) pool->inds.ensure(pcount * sizeof(unsigned));
 				E.pre = needs_pre ? (T*) pre_buf.ensure(pcount * sizeof(T)) : nullptr;
 			}
-			const bool ok = conv_forward_fused<T>(shape(), n, x, wv, bv, (T*) out, wt, ready, EPI_POOL, E, nullptr);
+			const bool ok = conv_forward_fused<T>(shape(training), n, x, wv, bv, (T*) out, wt, ready, EPI_POOL, E, nullptr);
 			weights_prepared();
 			ready = true;
 			if (ok) {
@@ -1249,7 +1254,7 @@ struct FusedLayer : LayerBase {
 		if (act) {
 			T* y = pool ? (T*) z_buf.ensure(zcount * sizeof(T)) : (T*) out;
 			E.pre = needs_pre ? (T*) pre_buf.ensure(zcount * sizeof(T)) : nullptr;
-			const bool ok = conv_forward_fused<T>(shape(), n, x, wv, bv, y, wt, ready, EPI_ACT, E, nullptr);
+			const bool ok = conv_forward_fused<T>(shape(training), n, x, wv, bv, y, wt, ready, EPI_ACT, E, nullptr);
 			weights_prepared();
 			if (ok) {
 				if (pool)
@@ -1271,7 +1276,7 @@ struct FusedLayer : LayerBase {
 			LayerBase* l = members[i];
 			void* dst = i + 1 == members.size() ? out : mid[i]->ensure(N * l->out_volume() * esize());
 			if (i == 0)
-				conv->forward_as(shape(), cur, N, dst);
+				conv->forward_as(shape(training), cur, N, dst);
 			else
 				l->forward(cur, N, training, dst);
 			cur = dst;
