@@ -44,6 +44,9 @@ __device__ __forceinline__ T row_combine(T v, T* lds) {
 	return acc;
 }
 
+__device__ __forceinline__ float dev_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double dev_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 template<typename T> struct MachineEps;
 template<> struct MachineEps<float> { static constexpr float value = 1.1920928955078125e-07f; };
 template<> struct MachineEps<double> { static constexpr double value = 2.220446049250313e-16; };
@@ -229,6 +232,41 @@ void softmax_ce_kernel(int N, int T_steps, int V, T eps, T scale, const T* __res
 	const bool live = n < N;
 	const size_t cs = (size_t) N * T_steps;
 	T total = (T) 0;
+	/* the gradient of up to a few dozen classes: a thread's outputs and objectives are fetched once, all at the same time, instead of
+	 * in three passes, each a round trip to memory or to a cache (256 x 10: 4.2 -> 3.6 us). The same operations in the same order. */
+	constexpr int HELD = 4;
+	if (GRAD && V <= HELD * PARTS) {
+		for (int t = 0; t < T_steps; ++t) {
+			const size_t base = (size_t) (live ? n : 0) + (size_t) N * t;
+			T mx = out[base], o[HELD], want[HELD];
+			#pragma unroll
+			for (int i = 0; i < HELD; ++i) {
+				const int j = threadIdx.y + i * PARTS;
+				o[i] = j < V ? out[base + cs * j] : mx;
+				want[i] = j < V ? obj[base + cs * j] : (T) 0;
+			}
+			if (live) {
+				#pragma unroll
+				for (int i = 0; i < HELD; ++i)
+					if (threadIdx.y + i * PARTS < V)
+						mx = o[i] > mx ? o[i] : mx;
+			}
+			mx = row_combine<T, true>(mx, lds);
+			T s = (T) 0;
+			#pragma unroll
+			for (int i = 0; i < HELD; ++i) {
+				o[i] = dev_exp(o[i] - mx);
+				if (live && threadIdx.y + i * PARTS < V)
+					s += o[i];
+			}
+			const T denom = row_combine<T, false>(s, lds) + eps;
+			#pragma unroll
+			for (int i = 0; i < HELD; ++i)
+				if (live && threadIdx.y + i * PARTS < V)
+					dst[base + cs * (threadIdx.y + i * PARTS)] = scale * (o[i] / denom - want[i]);
+		}
+		return;
+	}
 	for (int t = 0; t < T_steps; ++t) {
 		const size_t base = (size_t) (live ? n : 0) + (size_t) N * t;
 		T mx = out[base];
@@ -277,51 +315,71 @@ void softmax_ce_kernel(int N, int T_steps, int V, T eps, T scale, const T* __res
  *   OPT_NADAM         optimizer/NadamOptimizer.hpp:44-65             k: d1, d2, lr, l2_corr, eps, d1 * l1_corr, (1 - d1) * l1_next_corr
  *   OPT_AMSGRAD       optimizer/AMSGradOptimizer.hpp:48-66           k: d1, d2, lr, -, eps */
 template<typename T, int RULE>
-__device__ __forceinline__ T optimizer_element(const OptCoef<T>& k, T g, T v, T* __restrict__ s0, T* __restrict__ s1,
-		T* __restrict__ s2, size_t i) {
+__device__ __forceinline__ T optimizer_value(const OptCoef<T>& k, T g, T v, T& s0, T& s1, T& s2) {
+	/* Which products are fused into the sum that follows is written out, so that an update is the same to the last bit in every
+	 * kernel that it is compiled into. */
+#pragma clang fp contract(off)
 	const T one = (T) 1;
 	if (RULE == OPT_VANILLA_SGD) {
-		return v - g * k.c[0];
+		return dev_fma(-g, k.c[0], v);
 	} else if (RULE == OPT_MOMENTUM_SGD) {
-		const T s = s0[i] * k.c[1] + g * k.c[0];
-		s0[i] = s;
-		return v - s;
+		s0 = dev_fma(g, k.c[0], s0 * k.c[1]);
+		return v - s0;
 	} else if (RULE == OPT_NESTEROV) {
-		const T old = s0[i];
-		const T s = old * k.c[1] - g * k.c[0];
-		s0[i] = s;
-		return v + old * -k.c[1] + s * (one + k.c[1]);
+		const T old = s0;
+		s0 = dev_fma(old, k.c[1], -(g * k.c[0]));
+		return dev_fma(s0, one + k.c[1], dev_fma(old, -k.c[1], v));
 	} else if (RULE == OPT_ADAGRAD || RULE == OPT_RMSPROP) {
-		const T a = RULE == OPT_ADAGRAD ? s0[i] + g * g : s0[i] * (one - k.c[2]) + g * g * k.c[2];
-		s0[i] = a;
-		return v - g * k.c[0] / (dev_sqrt(a) + k.c[1]);
+		s0 = RULE == OPT_ADAGRAD ? dev_fma(g, g, s0) : dev_fma(g * g, k.c[2], s0 * (one - k.c[2]));
+		return v - g * k.c[0] / (dev_sqrt(s0) + k.c[1]);
 	} else if (RULE == OPT_ADADELTA) {
-		const T a = s0[i] * (one - k.c[0]) + g * g * k.c[0];
-		const T upd = -g * dev_sqrt(s1[i] + k.c[1]) / dev_sqrt(a + k.c[1]);
-		s0[i] = a;
-		s1[i] = s1[i] * (one - k.c[0]) + upd * upd * k.c[0];
+		s0 = dev_fma(g * g, k.c[0], s0 * (one - k.c[0]));
+		const T upd = -g * dev_sqrt(s1 + k.c[1]) / dev_sqrt(s0 + k.c[1]);
+		s1 = dev_fma(upd * upd, k.c[0], s1 * (one - k.c[0]));
 		return v + upd;
 	} else {
-		const T m = s0[i] * (one - k.c[0]) + g * k.c[0];
-		s0[i] = m;
+		const T m = dev_fma(g, k.c[0], s0 * (one - k.c[0]));
+		s0 = m;
 		if (RULE == OPT_ADAMAX) {
-			const T decayed = s1[i] * (one - k.c[1]), ag = g < (T) 0 ? -g : g;
+			const T decayed = s1 * (one - k.c[1]), ag = g < (T) 0 ? -g : g;
 			const T u = decayed > ag ? decayed : ag;
-			s1[i] = u;
+			s1 = u;
 			return v - (m * k.c[2]) / (u + k.c[4]);
 		}
-		const T sq = s1[i] * (one - k.c[1]) + g * g * k.c[1];
-		s1[i] = sq;
+		const T sq = dev_fma(g * g, k.c[1], s1 * (one - k.c[1]));
+		s1 = sq;
 		if (RULE == OPT_ADAM)
-			return v - (m * k.c[2]) / dev_sqrt(sq * k.c[3] + k.c[4]);
+			return v - (m * k.c[2]) / dev_sqrt(dev_fma(sq, k.c[3], k.c[4]));
 		if (RULE == OPT_NADAM)
-			return v - ((g * k.c[5] + m * k.c[6]) * k.c[2]) / dev_sqrt(sq * k.c[3] + k.c[4]);
+			return v - (dev_fma(g, k.c[5], m * k.c[6]) * k.c[2]) / dev_sqrt(dev_fma(sq, k.c[3], k.c[4]));
 		/* OPT_AMSGRAD */
-		const T prev = s2[i];
+		const T prev = s2;
 		const T mx = sq > prev ? sq : prev;
-		s2[i] = mx;
+		s2 = mx;
 		return v - (m * k.c[2]) / dev_sqrt(mx + k.c[4]);
 	}
+}
+
+/* how many state matrices a rule reads and writes */
+constexpr int states_of(int rule) {
+	return rule == OPT_VANILLA_SGD ? 0 : rule == OPT_AMSGRAD ? 3 :
+			rule == OPT_MOMENTUM_SGD || rule == OPT_NESTEROV || rule == OPT_ADAGRAD || rule == OPT_RMSPROP ? 1 : 2;
+}
+
+/* the value of element i, its state read and written in place */
+template<typename T, int RULE>
+__device__ __forceinline__ T optimizer_element(const OptCoef<T>& k, T g, T v, T* __restrict__ s0, T* __restrict__ s1,
+		T* __restrict__ s2, size_t i) {
+	constexpr int S = states_of(RULE);
+	T a = S > 0 ? s0[i] : (T) 0, b = S > 1 ? s1[i] : (T) 0, c = S > 2 ? s2[i] : (T) 0;
+	const T r = optimizer_value<T, RULE>(k, g, v, a, b, c);
+	if (S > 0)
+		s0[i] = a;
+	if (S > 1)
+		s1[i] = b;
+	if (S > 2)
+		s2[i] = c;
+	return r;
 }
 
 /* Parameters::regularize before the update (optimizer/SGDOptimizer.hpp:59-63, parameters/StandardParameters.hpp:133-136):
@@ -330,6 +388,7 @@ __device__ __forceinline__ T optimizer_element(const OptCoef<T>& k, T g, T v, T*
  * or both (ElasticNetParameterRegularization.hpp:40-42). Both lambdas zero: no regularization, the gradient as it is. */
 template<typename T>
 __device__ __forceinline__ T regularized_gradient(T g, T v, T l1, T l2) {
+#pragma clang fp contract(off)
 	if (l1 == (T) 0 && l2 == (T) 0)
 		return g;
 	const T sign_term = v >= (T) 0 ? l1 : -l1;
@@ -438,42 +497,81 @@ void add_regularization_kernel(size_t n, const T* __restrict__ values, T* __rest
 		grad[i] = regularized_gradient(grad[i], values[i], l1, l2);
 }
 
+/* Four elements of a parameter, all their loads issued before the first is used: the stores of one would otherwise hold back
+ * the loads of the next (nothing says that the tensors do not overlap), four round trips to memory instead of one. A step of SGD on
+ * 784 x 512, 512 x 256 and 256 x 10 weights, both prepared layouts rewritten, 7.8 -> 7.2 us; Adam on the 70 thousand parameters of a
+ * small image classifier 5.8 -> 5.3, Nadam on 63 thousand with up to eight partial sums each 10.0 -> 6.2.
+ * An element's gradient is what has been accumulated plus the partial sums that still wait, these added up first, in ascending
+ * order from zero (the order and grouping of reduce_partials_many for so few of them). Writes the new value, state and a
+ * gradient of zero, and returns the values. */
+template<typename T, int RULE>
+__device__ __forceinline__ void step_of_four(const OptParam<T>& q, const OptCoef<T>& k, const size_t (&at)[4], const bool (&in)[4], T (&values)[4]) {
+	constexpr int S = states_of(RULE);
+	T g[4], v[4], s0[4], s1[4], s2[4], parts[4][OPT_MAX_PARTS];
+	#pragma unroll
+	for (int j = 0; j < 4; ++j) {
+		const size_t i = in[j] ? at[j] : 0;
+		g[j] = q.grad[i];
+		v[j] = q.values[i];
+		s0[j] = S > 0 ? q.s0[i] : (T) 0;
+		s1[j] = S > 1 ? q.s1[i] : (T) 0;
+		s2[j] = S > 2 ? q.s2[i] : (T) 0;
+	}
+	const int splits = q.parts != nullptr ? q.splits : 0;
+	#pragma unroll
+	for (int s = 0; s < OPT_MAX_PARTS; ++s)
+		#pragma unroll
+		for (int j = 0; j < 4; ++j)
+			parts[j][s] = s < splits ? q.parts[(size_t) s * q.n + (in[j] ? at[j] : 0)] : (T) 0;
+	#pragma unroll
+	for (int j = 0; j < 4; ++j) {
+		if (splits > 0) {
+			T t = (T) 0;
+			#pragma unroll
+			for (int s = 0; s < OPT_MAX_PARTS; ++s)
+				t += parts[j][s];               /* (a sum that started at zero is never -0: adding zero keeps it) */
+			g[j] += t;
+		}
+		values[j] = optimizer_value<T, RULE>(k, regularized_gradient(g[j], v[j], q.l1, q.l2), v[j], s0[j], s1[j], s2[j]);
+	}
+	#pragma unroll
+	for (int j = 0; j < 4; ++j)
+		if (in[j]) {
+			q.values[at[j]] = values[j];
+			q.grad[at[j]] = (T) 0;
+			if (S > 0)
+				q.s0[at[j]] = s0[j];
+			if (S > 1)
+				q.s1[at[j]] = s1[j];
+			if (S > 2)
+				q.s2[at[j]] = s2[j];
+		}
+}
+
 /* The update and gradient reset of up to OPT_BATCH parameters in one launch (blockIdx.y picks the parameter,
  * blockIdx.x a run of 1024 elements, or a 32 x 32 tile of the matrix). A convolution or dense weight matrix may
  * bring its prepared layouts along (the forward layout wt[k][f] and the input-gradient layout wd[tap + RHW * f][c],
  * both zero-padded when they were first built): the new values are written there as well, which saves the two
  * re-layout launches of the next pass. The matrix is column-major (k fastest) and wt is f fastest, so a tile goes
  * through LDS and both sides are accessed along their contiguous index. */
-/* the gradient of element i: what has been accumulated plus the partial sums that still wait, these added up first, in
- * ascending order from zero (the order and grouping of reduce_partials_many for so few of them) */
-template<typename T>
-__device__ __forceinline__ T whole_gradient(const OptParam<T>& q, size_t i) {
-	T g = q.grad[i];
-	if (q.parts != nullptr) {
-		T t = (T) 0;
-		for (int s = 0; s < q.splits; ++s)
-			t += q.parts[(size_t) s * q.n + i];
-		g += t;
-	}
-	return g;
-}
-
 template<typename T, int RULE>
 __global__ __launch_bounds__(256)
 void optimizer_step_many_kernel(OptBatch<T> batch, OptCoef<T> k) {
 	__shared__ T tile[32][33];
 	const OptParam<T>& q = batch.p[blockIdx.y];
 	const int tid = threadIdx.x;
+	size_t at[4];
+	bool in[4];
+	T v[4];
 	if (!q.wt_fwd && !q.wt_dgrad) {
+		if ((size_t) blockIdx.x * 1024 >= q.n)
+			return;
 		#pragma unroll
 		for (int j = 0; j < 4; ++j) {
-			const size_t i = (size_t) blockIdx.x * 1024 + tid + 256 * j;
-			if (i < q.n) {
-				q.values[i] = optimizer_element<T, RULE>(k, regularized_gradient(whole_gradient(q, i), q.values[i], q.l1, q.l2), q.values[i], q.s0, q.s1,
-						q.s2, i);
-				q.grad[i] = (T) 0;
-			}
+			at[j] = (size_t) blockIdx.x * 1024 + tid + 256 * j;
+			in[j] = at[j] < q.n;
 		}
+		step_of_four<T, RULE>(q, k, at, in, v);
 		return;
 	}
 	const int F = (int) (q.n / (size_t) q.K);
@@ -482,22 +580,21 @@ void optimizer_step_many_kernel(OptBatch<T> batch, OptCoef<T> k) {
 		return;
 	const int k0 = ((int) blockIdx.x % tiles_k) * 32, f0 = ((int) blockIdx.x / tiles_k) * 32;
 	const int a = tid % 32, b = tid / 32;
+	const int row = k0 + a;
 	#pragma unroll
 	for (int j = 0; j < 4; ++j) {
-		const int row = k0 + a, f = f0 + b + 8 * j;
-		if (row < q.K && f < F) {
-			const size_t i = (size_t) row + (size_t) q.K * f;
-			const T v = optimizer_element<T, RULE>(k, regularized_gradient(whole_gradient(q, i), q.values[i], q.l1, q.l2), q.values[i], q.s0, q.s1,
-					q.s2, i);
-			q.values[i] = v;
-			q.grad[i] = (T) 0;
-			tile[b + 8 * j][a] = v;
-			if (q.wt_dgrad) {
-				const unsigned tap = (unsigned) row % (unsigned) q.RHW, c = (unsigned) row / (unsigned) q.RHW;
-				q.wt_dgrad[(size_t) (tap + (unsigned) q.RHW * f) * q.ldw_dgrad + c] = v;
-			}
-		}
+		at[j] = (size_t) row + (size_t) q.K * (f0 + b + 8 * j);
+		in[j] = row < q.K && f0 + b + 8 * j < F;
 	}
+	step_of_four<T, RULE>(q, k, at, in, v);
+	const unsigned tap = (unsigned) row % (unsigned) q.RHW, c = (unsigned) row / (unsigned) q.RHW;
+	#pragma unroll
+	for (int j = 0; j < 4; ++j)
+		if (in[j]) {
+			tile[b + 8 * j][a] = v[j];
+			if (q.wt_dgrad)
+				q.wt_dgrad[(size_t) (tap + (unsigned) q.RHW * (unsigned) (f0 + b + 8 * j)) * q.ldw_dgrad + c] = v[j];
+		}
 	if (!q.wt_fwd)
 		return;
 	__syncthreads();
