@@ -7,6 +7,7 @@ the reference's column-major Eigen buffers; DeviceTensor keeps a tensor resident
 layers. There is no host fallback: without the built library or without an MI355X every call raises.
 """
 import ctypes
+import math
 import os
 import subprocess
 
@@ -61,6 +62,32 @@ def build():
 
 _lib = None
 
+# The calls of a training or inference step, with their argument types declared: ctypes then converts Python integers itself, in
+# a third of the time that it takes to make an object of each argument first. Function objects of their own (those that lib()
+# hands out take whatever they are given, as ever), bound by lib(). A step of an MLP (three layers forward and back, loss and
+# optimizer, eight calls) on a library that does nothing took 101 us of Python on one machine, and takes 28 this way; a good part
+# of the rest was numpy's product of a few integers.
+_P, _SZ, _I, _D = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_double
+_STEP_CALLS = {
+    "cattle_hip_alloc": (_P, _SZ), "cattle_hip_free": (_P,), "cattle_hip_layer_forward": (_P, _P, _I, _SZ, _I, _P, _I),
+    "cattle_hip_layer_backward": (_P, _P, _I, _SZ, _P, _I), "cattle_hip_layer_is_input_layer": (_P, _P),
+    "cattle_hip_loss_d_function": (_I, _I, _P, _I, _P, _I, _SZ, _SZ, _SZ, _D, _D, _P, _I),
+    "cattle_hip_optimizer_step_many": (_P, _P, _SZ, _I, _P, _SZ, _SZ), "cattle_hip_layer_reset_param_grad": (_P, _SZ),
+}
+
+
+class _Step(object):
+    """The bound functions of _STEP_CALLS; the first use loads the library."""
+
+    def __getattr__(self, name):
+        if "cattle_hip_" + name not in _STEP_CALLS:
+            raise AttributeError(name)
+        lib()
+        return self.__dict__[name]
+
+
+_step = _Step()
+
 
 def lib():
     """Loads the built library; raises if it has not been built (there is no other code path)."""
@@ -68,11 +95,16 @@ def lib():
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise CattleHipError(-1, "libcattle_hip.so is not built: run __graft_entry__.build() or make -C c-attl3_amd")
-        _lib = ctypes.CDLL(LIB_PATH)
-        _lib.cattle_hip_last_error.restype = ctypes.c_char_p
+        loaded = ctypes.CDLL(LIB_PATH)
+        loaded.cattle_hip_last_error.restype = ctypes.c_char_p
         for name in EXPORTS:
             if name != "cattle_hip_last_error":
-                getattr(_lib, name).restype = ctypes.c_int
+                getattr(loaded, name).restype = ctypes.c_int
+        for name, types in _STEP_CALLS.items():
+            fn = loaded[name]
+            fn.argtypes, fn.restype = types, ctypes.c_int
+            setattr(_step, name[len("cattle_hip_"):], fn)
+        _lib = loaded           # last: another thread that sees it finds everything bound
     return _lib
 
 
@@ -101,11 +133,14 @@ def synchronize():
     _check(lib().cattle_hip_synchronize())
 
 
+_FLOAT32, _FLOAT64 = np.dtype(np.float32), np.dtype(np.float64)
+
+
 def _dtype_code(dtype):
     dtype = np.dtype(dtype)
-    if dtype == np.float32:
+    if dtype == _FLOAT32:
         return F32
-    if dtype == np.float64:
+    if dtype == _FLOAT64:
         return F64
     raise TypeError("Scalar must be float32 or float64")
 
@@ -118,12 +153,24 @@ class DeviceTensor(object):
     """A tensor resident in device memory, in the reference's column-major layout."""
 
     def __init__(self, shape, dtype):
-        self.shape = tuple(int(s) for s in shape)
-        self.dtype = np.dtype(dtype)
-        self.nbytes = int(np.prod(self.shape)) * self.dtype.itemsize
+        self._allocate(tuple(int(s) for s in shape), np.dtype(dtype))
+
+    def _allocate(self, shape, dtype):
+        """`shape` a tuple of ints, `dtype` a numpy dtype."""
+        self.shape = shape
+        self.dtype = dtype
+        self.nbytes = math.prod(shape) * dtype.itemsize
         p = ctypes.c_void_p()
-        _check(lib().cattle_hip_alloc(ctypes.byref(p), _sz(self.nbytes)))
+        rc = _step.alloc(ctypes.byref(p), self.nbytes)
+        if rc:
+            _check(rc)
         self.ptr = p
+
+    @staticmethod
+    def _of(shape, dtype):
+        t = DeviceTensor.__new__(DeviceTensor)
+        t._allocate(shape, dtype)
+        return t
 
     @staticmethod
     def from_host(a):
@@ -139,7 +186,9 @@ class DeviceTensor(object):
 
     def free(self):
         if self.ptr is not None and self.ptr.value:
-            _check(lib().cattle_hip_free(self.ptr))
+            rc = _step.free(self.ptr)
+            if rc:
+                _check(rc)
         self.ptr = None
 
     def __del__(self):
@@ -253,7 +302,9 @@ class Parameters(object):
         return a
 
     def reset_grad(self):
-        _check(lib().cattle_hip_layer_reset_param_grad(self._layer._h, _sz(self._index)))
+        rc = _step.layer_reset_param_grad(self._layer._h, self._index)
+        if rc:
+            _check(rc)
 
     def optimizer_update(self, optimizer, hyper, epoch=0, timestep=0):
         """<Name>Optimizer::_update_params on the device; optimizer is a key of OPTIMIZERS, hyper the reference
@@ -322,9 +373,10 @@ class ParameterList(object):
         return len(self._params)
 
     def optimizer_step(self, optimizer, hyper, epoch=0, timestep=0):
-        _check(lib().cattle_hip_optimizer_step_many(self._layers, self._indices, _sz(len(self._params)),
-                                                    ctypes.c_int(OPTIMIZERS[optimizer]), _hyper_array(tuple(hyper)),
-                                                    _sz(epoch), _sz(timestep)))
+        rc = _step.optimizer_step_many(self._layers, self._indices, len(self._params), OPTIMIZERS[optimizer],
+                                       _hyper_array(tuple(hyper)), int(epoch), int(timestep))
+        if rc:
+            _check(rc)
 
 
 def _hyper_array(hyper):
@@ -347,7 +399,7 @@ def _loss_args(out, obj, sequential):
         raise ValueError("out and obj dimensions differ")          # assert(out.dimensions() == obj.dimensions())
     batch = out.shape[0]
     steps = out.shape[1] if sequential else 1
-    size = int(np.prod(out.shape[1:])) // steps
+    size = math.prod(out.shape[1:]) // steps
     dev = isinstance(out, DeviceTensor)
     ptr = (lambda t: t.ptr) if dev else (lambda a: ctypes.c_void_p(a.ctypes.data))
     return out, obj, batch, steps, size, (DEVICE if dev else HOST), ptr
@@ -374,12 +426,13 @@ def loss_d_function(kind, out, obj, epsilon=1e-5, scale=1.0, sequential=False, n
     (numpy array or DeviceTensor) in the shape of out."""
     out, obj, batch, steps, size, space, ptr = _loss_args(out, obj, sequential)
     if space == DEVICE:
-        grad = DeviceTensor(out.shape, out.dtype)
+        grad = DeviceTensor._of(out.shape, out.dtype)
     else:
         grad = np.empty(out.shape, dtype=out.dtype, order="F")
-    _check(lib().cattle_hip_loss_d_function(_dtype_code(out.dtype), _loss_kind(kind, negated), ptr(out), space, ptr(obj), space,
-                                            _sz(batch), _sz(steps), _sz(size), ctypes.c_double(epsilon),
-                                            ctypes.c_double(scale), ptr(grad), space))
+    rc = _step.loss_d_function(_dtype_code(out.dtype), LOSS[kind] | (LOSS_NEGATED if negated else 0), ptr(out), space, ptr(obj), space,
+                               batch, steps, size, float(epsilon), float(scale), ptr(grad), space)
+    if rc:
+        _check(rc)
     return grad
 
 
@@ -389,8 +442,8 @@ class Layer(object):
     def __init__(self, handle, dtype, in_shape, out_shape):
         self._h = handle
         self.dtype = np.dtype(dtype)
-        self._in_shape = tuple(in_shape)        # per-sample shapes as the caller sees them
-        self._out_shape = tuple(out_shape)
+        self._in_shape = tuple(int(d) for d in in_shape)        # per-sample shapes as the caller sees them
+        self._out_shape = tuple(int(d) for d in out_shape)
 
     # -- cattle::Layer ------------------------------------------------------------------------
     def get_input_dims(self):
@@ -401,7 +454,9 @@ class Layer(object):
 
     def is_input_layer(self):
         v = ctypes.c_int()
-        _check(lib().cattle_hip_layer_is_input_layer(self._h, ctypes.byref(v)))
+        rc = _step.layer_is_input_layer(self._h, ctypes.byref(v))
+        if rc:
+            _check(rc)
         return bool(v.value)
 
     def set_input_layer(self, flag):
@@ -433,9 +488,12 @@ class Layer(object):
         """x: numpy array (host path, returns numpy) or DeviceTensor (device path, returns DeviceTensor)."""
         if isinstance(x, DeviceTensor):
             batch = x.shape[0]
-            self._expect(x.shape[1:], self._in_shape, "input")
-            out = DeviceTensor((batch,) + self._out_shape, self.dtype)
-            _check(lib().cattle_hip_layer_forward(self._h, x.ptr, DEVICE, _sz(batch), ctypes.c_int(int(training)), out.ptr, DEVICE))
+            if x.shape[1:] != self._in_shape:
+                self._expect(x.shape[1:], self._in_shape, "input")
+            out = DeviceTensor._of((batch,) + self._out_shape, self.dtype)
+            rc = _step.layer_forward(self._h, x.ptr, DEVICE, batch, int(training), out.ptr, DEVICE)
+            if rc:
+                _check(rc)
             self._keep = (x, out)                 # borrowed by the layer until pass_back
             return out
         x = np.asfortranarray(x, dtype=self.dtype)
@@ -448,22 +506,27 @@ class Layer(object):
 
     def forward_into(self, x, out, training=True):
         """Device path without allocation: x and out are DeviceTensors owned by the caller."""
-        _check(lib().cattle_hip_layer_forward(self._h, x.ptr, DEVICE, _sz(x.shape[0]), ctypes.c_int(int(training)), out.ptr,
-                                              DEVICE))
+        rc = _step.layer_forward(self._h, x.ptr, DEVICE, x.shape[0], int(training), out.ptr, DEVICE)
+        if rc:
+            _check(rc)
 
     def backward_into(self, out_grad, in_grad):
         """Device path without allocation; in_grad may be None for an input layer."""
-        _check(lib().cattle_hip_layer_backward(self._h, out_grad.ptr, DEVICE, _sz(out_grad.shape[0]),
-                                               None if in_grad is None else in_grad.ptr, DEVICE))
+        rc = _step.layer_backward(self._h, out_grad.ptr, DEVICE, out_grad.shape[0], None if in_grad is None else in_grad.ptr, DEVICE)
+        if rc:
+            _check(rc)
 
     def pass_back(self, out_grad):
         """Returns the input gradient, or None for an input layer (the reference's null tensor)."""
         skip = self.is_input_layer() and not getattr(self, "_always_backprop", False)
         if isinstance(out_grad, DeviceTensor):
             batch = out_grad.shape[0]
-            self._expect(out_grad.shape[1:], self._out_shape, "output gradient")
-            dx = None if skip else DeviceTensor((batch,) + self._in_shape, self.dtype)
-            _check(lib().cattle_hip_layer_backward(self._h, out_grad.ptr, DEVICE, _sz(batch), None if skip else dx.ptr, DEVICE))
+            if out_grad.shape[1:] != self._out_shape:
+                self._expect(out_grad.shape[1:], self._out_shape, "output gradient")
+            dx = None if skip else DeviceTensor._of((batch,) + self._in_shape, self.dtype)
+            rc = _step.layer_backward(self._h, out_grad.ptr, DEVICE, batch, None if skip else dx.ptr, DEVICE)
+            if rc:
+                _check(rc)
             return dx
         g = np.asfortranarray(out_grad, dtype=self.dtype)
         batch = g.shape[0]
