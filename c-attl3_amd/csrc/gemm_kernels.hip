@@ -474,7 +474,8 @@ __device__ __forceinline__ void gather_gemm_body(const T* __restrict__ src, cons
 /* How the weight-gradient launch is cut: tiles = ktiles * ftiles blocks per slice, `splits` slices. */
 struct WgradSplit {
 	int ktiles, tiles, splits, chunks_per_split, pixel_mode;
-	int direct;     /* one slice only: the block adds its tile to the gradient itself, `partials` and `bias_partials` are the gradients */
+	int direct;     /* one slice only: the block adds its tile to the gradient itself, `partials` and `bias_partials` are the gradients
+	                 * (as they are where 0 is given for gradients that are to be overwritten) */
 };
 
 /* ------------------------------------------------------------------------------------------------
@@ -878,7 +879,7 @@ void gather_with_wgrad_kernel(const T* __restrict__ src, const T* __restrict__ w
  * are reproducible. For V > 1 the count is a multiple of V and the partials are 16-byte aligned. */
 template<typename T, int V>
 __device__ __forceinline__ void reduce_partials_block(const T* __restrict__ partials, T* __restrict__ dst, size_t count, int blk,
-		int splits, T (&lds)[16][64]) {
+		int splits, bool fresh, T* __restrict__ copy, T (&lds)[16][64]) {
 	constexpr int OV = 64 / V, GR = 256 / OV;
 	static_assert(GR <= 16, "group sums fit the staging array");
 	const int ox = (threadIdx.x % OV) * V, grp = threadIdx.x / OV;
@@ -905,7 +906,11 @@ __device__ __forceinline__ void reduce_partials_block(const T* __restrict__ part
 		#pragma unroll
 		for (int j = 1; j < GR; ++j)
 			total += lds[j][threadIdx.x];
-		dst[o] += total;
+		if (!fresh)
+			total = dst[o] + total;
+		dst[o] = total;
+		if (copy != nullptr)
+			copy[o] = total;
 	}
 }
 
@@ -914,7 +919,7 @@ __device__ __forceinline__ void reduce_partials_block(const T* __restrict__ part
  * shuffle tree. With few outputs the form above is a handful of blocks walking hundreds of partials one after the other. */
 template<typename T>
 __device__ __forceinline__ void reduce_partials_wide_block(const T* __restrict__ partials, T* __restrict__ dst, size_t count, int blk,
-		int splits) {
+		int splits, bool fresh, T* __restrict__ copy) {
 	/* Neighbouring outputs share the cache lines of every slice: the blocks of one XCD take a contiguous range of outputs,
 	 * so that a line is fetched by one L2, not by all eight (the entry's blocks start at a multiple of 8 and are a
 	 * multiple of 8, see reduce_partials_many). */
@@ -942,8 +947,13 @@ __device__ __forceinline__ void reduce_partials_wide_block(const T* __restrict__
 	#pragma unroll
 	for (int off = 32; off > 0; off >>= 1)
 		s += __shfl_down(s, off, 64);
-	if (lane == 0)
-		dst[i] += s;
+	if (lane == 0) {
+		if (!fresh)
+			s = dst[i] + s;
+		dst[i] = s;
+		if (copy != nullptr)
+			copy[i] = s;
+	}
 }
 
 /* The partial sums of up to REDUCE_BATCH matrices (the weight and the bias gradients of several layers) added to their
@@ -959,11 +969,11 @@ void reduce_partials_many_kernel(const ReduceBatch<T> batch) {
 	const ReduceEntry<T>& q = batch.e[e];
 	const int blk = (int) blockIdx.x - q.first_block;
 	if (q.wide)
-		reduce_partials_wide_block<T>(q.partials, q.dst, q.count, blk, q.splits);
+		reduce_partials_wide_block<T>(q.partials, q.dst, q.count, blk, q.splits, q.fresh, q.copy);
 	else if (q.vec)
-		reduce_partials_block<T, 16 / (int) sizeof(T)>(q.partials, q.dst, q.count, blk, q.splits, lds);
+		reduce_partials_block<T, 16 / (int) sizeof(T)>(q.partials, q.dst, q.count, blk, q.splits, q.fresh, q.copy, lds);
 	else
-		reduce_partials_block<T, 1>(q.partials, q.dst, q.count, blk, q.splits, lds);
+		reduce_partials_block<T, 1>(q.partials, q.dst, q.count, blk, q.splits, q.fresh, q.copy, lds);
 }
 
 /* Forward weights: wt[k][f] = w[k + K*f], zero-padded to Kp rows x ldw columns. gate_block > 0: the columns in the
@@ -3131,22 +3141,22 @@ void conv_forward_static(const ConvShape& s, int N, const T* x, const T* w, cons
 
 template<typename T>
 void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* out_grad, T* wgrad, T* bgrad, T* partials,
-		const WgradAct<T>* act, ReduceBatch<T>* deferred, const std::function<bool(WgradRider<T>&)>* elsewhere);
+		const WgradAct<T>* act, ReduceBatch<T>* deferred, bool fresh, const std::function<bool(WgradRider<T>&)>* elsewhere);
 template<typename T>
 bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* out_grad, T* in_grad, T* wt_dgrad, bool wt_ready,
 		const LstmBackwardStep<T>* then, int og_batch, WgradRider<T>* rider);
 
 template<typename T>
 void conv_weight_gradient(const ConvShape& s, int N, const T* x, const T* out_grad, T* wgrad, T* bgrad, T* partials,
-		const WgradAct<T>* act, ReduceBatch<T>* deferred) {
-	conv_weight_gradient_with<T>(s, N, x, out_grad, wgrad, bgrad, partials, act, deferred, nullptr);
+		const WgradAct<T>* act, ReduceBatch<T>* deferred, bool fresh) {
+	conv_weight_gradient_with<T>(s, N, x, out_grad, wgrad, bgrad, partials, act, deferred, fresh, nullptr);
 }
 
 /* `elsewhere`, if given, is offered the kernel launch when it is one that can ride in another launch (WgradRider) and
  * says whether it ran it; the sums of the slices follow here either way. */
 template<typename T>
 void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* out_grad, T* wgrad, T* bgrad, T* partials,
-		const WgradAct<T>* act, ReduceBatch<T>* deferred, const std::function<bool(WgradRider<T>&)>* elsewhere) {
+		const WgradAct<T>* act, ReduceBatch<T>* deferred, bool fresh, const std::function<bool(WgradRider<T>&)>* elsewhere) {
 	check_sizes(s, N);
 	if (deferred)
 		deferred->count = 0;
@@ -3189,7 +3199,7 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 		if (!can_ride && !bf16x3 && small_weight_gradient_possible(g, vec, act)) {
 			T p0, p1;
 			negative_side(act, &p0, &p1);
-			small_weight_gradient(x, out_grad, wgrad, bgrad, g, act, p0, p1);
+			small_weight_gradient(x, out_grad, wgrad, bgrad, g, act, p0, p1, fresh);
 			return;
 		}
 	auto run = [&](T* to_w, T* to_b, const WgradSplit& how) {
@@ -3221,7 +3231,9 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 	};
 	if (p.splits == 1) {
 		/* one slice: every block owns its tile of the gradient and adds to it directly, no second launch */
-		const WgradSplit direct = { p.ktiles, p.ktiles * p.ftiles, 1, p.chunks_per_split, p.pixel_mode, 1 };
+		const WgradSplit direct = { p.ktiles, p.ktiles * p.ftiles, 1, p.chunks_per_split, p.pixel_mode, fresh ? 0 : 1 };
+		if (fresh)
+			b3.direct = 0;
 		run(wgrad, bgrad, direct);
 		return;
 	}
@@ -3235,9 +3247,9 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 	const bool vec_sum = count % V == 0 && g.F % V == 0 && (reinterpret_cast<uintptr_t>(partials) & 15) == 0;
 	ReduceBatch<T> both;
 	both.count = 0;
-	both.e[both.count++] = ReduceEntry<T>{ partials, wgrad, count, p.splits, 0, wide, vec_sum };
+	both.e[both.count++] = ReduceEntry<T>{ partials, wgrad, count, p.splits, 0, wide, vec_sum, fresh, nullptr };
 	if (bgrad)
-		both.e[both.count++] = ReduceEntry<T>{ bias_partials, bgrad, (size_t) g.F, p.splits, 0, wide, vec_sum };
+		both.e[both.count++] = ReduceEntry<T>{ bias_partials, bgrad, (size_t) g.F, p.splits, 0, wide, vec_sum, fresh, nullptr };
 	if (deferred) {
 		/* the caller adds the partial sums to the gradients later, together with those of other layers */
 		*deferred = both;
@@ -3354,7 +3366,7 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 
 template<typename T>
 void conv_backward(const ConvShape& s, int N, const T* x, const T* w, const T* out_grad, T* wgrad, T* bgrad,
-		T* in_grad, T* wt_dgrad, bool wt_ready, T* partials, const WgradAct<T>* act, ReduceBatch<T>* deferred) {
+		T* in_grad, T* wt_dgrad, bool wt_ready, T* partials, const WgradAct<T>* act, ReduceBatch<T>* deferred, bool fresh) {
 	CATTLE_HIP_REQUIRE(!act || !in_grad || act->dz != nullptr, "the input gradient needs the gradient before the activation");
 	/* Without an activation to undo, the two gradients wait for the same upstream gradient only: where the weight gradient
 	 * is a launch of one-wavefront tiles, the input-gradient launch takes its blocks along. */
@@ -3364,7 +3376,7 @@ void conv_backward(const ConvShape& s, int N, const T* x, const T* w, const T* o
 		in_grad_done = true;
 		return rider.done;
 	};
-	conv_weight_gradient_with<T>(s, N, x, out_grad, wgrad, bgrad, partials, act, deferred, in_grad && !act ? &with_input_gradient : nullptr);
+	conv_weight_gradient_with<T>(s, N, x, out_grad, wgrad, bgrad, partials, act, deferred, fresh, in_grad && !act ? &with_input_gradient : nullptr);
 	if (in_grad && !in_grad_done)
 		conv_input_gradient<T>(s, N, w, act ? (const T*) act->dz : out_grad, in_grad, wt_dgrad, wt_ready, nullptr, 0);
 }
@@ -3384,13 +3396,13 @@ template bool conv_forward_lstm<double>(const ConvShape&, int, const double*, in
 template void conv_forward_static<float>(const ConvShape&, int, const float*, const float*, const float*, float*);
 template void conv_forward_static<double>(const ConvShape&, int, const double*, const double*, const double*, double*);
 template void conv_backward<float>(const ConvShape&, int, const float*, const float*, const float*, float*, float*, float*,
-		float*, bool, float*, const WgradAct<float>*, ReduceBatch<float>*);
+		float*, bool, float*, const WgradAct<float>*, ReduceBatch<float>*, bool);
 template void conv_backward<double>(const ConvShape&, int, const double*, const double*, const double*, double*, double*,
-		double*, double*, bool, double*, const WgradAct<double>*, ReduceBatch<double>*);
+		double*, double*, bool, double*, const WgradAct<double>*, ReduceBatch<double>*, bool);
 template void conv_weight_gradient<float>(const ConvShape&, int, const float*, const float*, float*, float*, float*,
-		const WgradAct<float>*, ReduceBatch<float>*);
+		const WgradAct<float>*, ReduceBatch<float>*, bool);
 template void conv_weight_gradient<double>(const ConvShape&, int, const double*, const double*, double*, double*, double*,
-		const WgradAct<double>*, ReduceBatch<double>*);
+		const WgradAct<double>*, ReduceBatch<double>*, bool);
 template void reduce_partials_many<float>(ReduceBatch<float>);
 template void reduce_partials_many<double>(ReduceBatch<double>);
 template int dgrad_weight_layout<float>(const ConvShape&, int);

@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <set>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -267,6 +268,15 @@ struct Param {
 	 * optimizer step as a rule, in one launch for all layers - and until then `pending` lists them (see Deferred). */
 	DevBuf partials;
 	bool pending = false;
+	/* A gradient that has been reset need not be zeroed where the backward pass that comes next can overwrite it as well as add to it
+	 * (`overwritten`: weights and biases of convolution, dense and recurrent kernels). It is then `clear_due`: zero, whatever the
+	 * buffer holds. That backward pass takes the mark off by storing its gradient; whoever else needs the buffer calls
+	 * whole_grad(), which zeroes it first. Spares a launch per parameter and pass, and the optimizer and the weight gradient a write
+	 * and a read of it: a convolution of 64 x 32 x 32 x 3 with its gradients read and reset 26.8 -> 24 us a pass, a dense layer of
+	 * 512 x 4096 -> 1024 127.6 -> 115.9. Recordings know nothing of marks: they are settled before a recording begins and before a graph is launched, and none are set in between. */
+	bool overwritten = false, clear_due = false;
+	void* whole_grad();
+	void mark_clear();
 	DevBuf moments[3];                 /* the optimizer's state matrices, allocated (zeroed) on first use */
 	int moments_ready = 0;             /* how many of them are */
 	double reg_l1 = 0, reg_l2 = 0;     /* ParameterRegularization of the parameter: L1 and L2 lambdas (both 0: none) */
@@ -291,7 +301,8 @@ struct Param {
 	std::shared_ptr<Param> deep_copy() const {
 		std::shared_ptr<Param> c = std::make_shared<Param>(rows, cols, optimizable, esize);
 		copy_in(c->values.p, values.p, CATTLE_HIP_DEVICE, bytes());
-		copy_in(c->grad.p, grad.p, CATTLE_HIP_DEVICE, bytes());
+		copy_in(c->grad.p, const_cast<Param*>(this)->whole_grad(), CATTLE_HIP_DEVICE, bytes());
+		c->overwritten = overwritten;
 		c->reg_l1 = reg_l1;
 		c->reg_l2 = reg_l2;
 		std::memcpy(c->value_limits, value_limits, sizeof(value_limits));
@@ -322,9 +333,24 @@ struct Deferred {
 			owner->pending = true;
 	}
 	template<typename T> static ReduceEntry<T>& pick(Entry& e);
-	void settle() {
+	/* `read`, if given: a gradient that is about to be read into `into`, which receives it from the launch that sums it. Returns
+	 * whether it did. */
+	bool settle(const void* read = nullptr, void* into = nullptr) {
 		if (entries.empty())
-			return;
+			return false;
+		bool copied = false;
+		for (size_t i = 0; read && i < entries.size(); ++i) {
+			/* the last of its entries (each is a launch's, and complete after the ones before it) */
+			Entry& e = entries[entries.size() - 1 - i];
+			if (e.owner->esize == sizeof(float) ? e.f.dst == read : e.d.dst == read) {
+				if (e.owner->esize == sizeof(float))
+					e.f.copy = static_cast<float*>(into);
+				else
+					e.d.copy = static_cast<double*>(into);
+				copied = true;
+				break;
+			}
+		}
 		ReduceBatch<float> bf;
 		ReduceBatch<double> bd;
 		bf.count = bd.count = 0;
@@ -347,6 +373,7 @@ struct Deferred {
 		entries.clear();
 		reduce_partials_many<float>(bf);
 		reduce_partials_many<double>(bd);
+		return copied;
 	}
 	/* The one entry that waits to be added to `grad`, if it is few enough slices for the optimizer launch to add them on
 	 * its way (in the order reduce_partials_many would: for up to as many slices as it has groups of threads that is
@@ -387,9 +414,50 @@ template<> ReduceEntry<float>& Deferred::pick<float>(Entry& e) { return e.f; }
 template<> ReduceEntry<double>& Deferred::pick<double>(Entry& e) { return e.d; }
 Deferred g_deferred;
 
+/* The parameters whose gradients are Param::clear_due. */
+struct Clears {
+	std::set<Param*> due;
+	void settle() {
+		while (!due.empty())
+			(void) (*due.begin())->whole_grad();
+	}
+};
+Clears g_clears;
+
+void* Param::whole_grad() {
+	if (clear_due) {
+		fill_zero(grad.p, bytes());
+		clear_due = false;
+		g_clears.due.erase(this);
+	}
+	return grad.p;
+}
+void Param::mark_clear() {
+	if (!clear_due)
+		g_clears.due.insert(this);
+	clear_due = true;
+}
+/* Before a weight-gradient launch for a kernel's weights and bias: whether it may overwrite both gradients; if not, both are
+ * whole afterwards. `overwrote` follows the launch. */
+bool may_overwrite(Param& w, Param& b) {
+	if (w.clear_due && b.clear_due)
+		return true;
+	(void) w.whole_grad();
+	(void) b.whole_grad();
+	return false;
+}
+void overwrote(Param& w, Param& b) {
+	for (Param* p : { &w, &b }) {
+		p->clear_due = false;
+		g_clears.due.erase(p);
+	}
+}
+
 Param::~Param() {
 	if (pending)
 		g_deferred.forget(this);
+	if (clear_due)
+		g_clears.due.erase(this);
 }
 
 template<typename T>
@@ -403,7 +471,7 @@ void fill_constant(Param& p, T v) {
  * StandardParameters.hpp:105-112) or on the gradient (accumulate_grad, :114-123) */
 void constrain(Param& p, bool values) {
 	const double* lim = values ? p.value_limits : p.grad_limits;
-	void* m = values ? p.values.p : p.grad.p;
+	void* m = values ? p.values.p : p.whole_grad();
 	if (p.esize == sizeof(float))
 		constrain_matrix<float>(p.rows * p.cols, static_cast<float*>(m), lim[0], lim[1], lim[2]);
 	else
@@ -492,6 +560,7 @@ struct ConvLayer : LayerBase {
 		}
 		params.push_back(std::make_shared<Param>((size_t) s.K(), (size_t) s.F, true, sizeof(T)));
 		params.push_back(std::make_shared<Param>(1, (size_t) s.F, true, sizeof(T)));
+		params[0]->overwritten = params[1]->overwritten = true;
 	}
 	ConvLayer(const ConvLayer& o, bool share) : LayerBase(o.dtype), shape(o.shape) {
 		copy_base(o, share);
@@ -531,8 +600,11 @@ struct ConvLayer : LayerBase {
 			g_deferred.settle();
 		T* part = (T*) w.partials.ensure(ws.partials * sizeof(T));
 		ReduceBatch<T> later;
+		const bool fresh = may_overwrite(w, *params[1]);
 		conv_backward<T>(s, n, x_cache, (const T*) w.values.p, (const T*) out_grad, (T*) w.grad.p, (T*) params[1]->grad.p,
-				(T*) in_grad, wt, ready, part, act, &later);
+				(T*) in_grad, wt, ready, part, act, &later, fresh);
+		if (fresh)
+			overwrote(w, *params[1]);
 		g_deferred.add<T>(&w, later);
 		if (in_grad) {
 			w.derived_version[1] = w.version;
@@ -664,6 +736,8 @@ struct ConvLstm : LayerBase {
 		params.push_back(std::make_shared<Param>(1, (size_t) sx.F, true, sizeof(T)));
 		params.push_back(std::make_shared<Param>((size_t) sh.K(), (size_t) sh.F, true, sizeof(T)));
 		params.push_back(std::make_shared<Param>(1, (size_t) sh.F, true, sizeof(T)));
+		for (const ParamPtr& p : params)
+			p->overwritten = true;
 	}
 	ConvLstm(const ConvLstm& o, bool share) : LayerBase(o.dtype), sx(o.sx), sh(o.sh), hidden(o.hidden), acts(o.acts),
 			foremost(o.foremost), mul_int(o.mul_int) {
@@ -810,15 +884,21 @@ struct ConvLstm : LayerBase {
 		if (total > 1) {
 			ConvShape s = sh;
 			const ConvWorkspace ws = weight_gradient_workspace<T>(s, (int) (N * total), wh.partials);
+			const bool fresh = may_overwrite(wh, *params[3]);
 			conv_weight_gradient<T>(s, (int) (N * total), (const T*) hprev_all.p, (const T*) dzh_all.p, (T*) wh.grad.p,
-					(T*) params[3]->grad.p, (T*) wh.partials.ensure(ws.partials * e), nullptr, &later);
+					(T*) params[3]->grad.p, (T*) wh.partials.ensure(ws.partials * e), nullptr, &later, fresh);
+			if (fresh)
+				overwrote(wh, *params[3]);
 			g_deferred.add<T>(&wh, later);
 		}
 		{
 			ConvShape s = sx;
 			const ConvWorkspace ws = weight_gradient_workspace<T>(s, (int) (N * T_in), wx.partials);
+			const bool fresh = may_overwrite(wx, *params[1]);
 			conv_weight_gradient<T>(s, (int) (N * T_in), x_cache, (const T*) dzx_all.p, (T*) wx.grad.p, (T*) params[1]->grad.p,
-					(T*) wx.partials.ensure(ws.partials * e), nullptr, &later);
+					(T*) wx.partials.ensure(ws.partials * e), nullptr, &later, fresh);
+			if (fresh)
+				overwrote(wx, *params[1]);
 			g_deferred.add<T>(&wx, later);
 			if (in_grad) {
 				T* wt = (T*) wx.derived[1].ensure(ws.wt_dgrad * e);
@@ -1609,6 +1689,7 @@ void run_optimizer(cattle_hip_layer_t layer, size_t index, cattle_hip_optimizer 
 	Param& p = optimizable_param(layer, index);
 	CATTLE_HIP_REQUIRE(hyper != nullptr, "null hyper-parameter array");
 	g_deferred.settle();
+	(void) p.whole_grad();
 	const int states = optimizer_state_count((int) optimizer);
 	for (int i = p.moments_ready; i < states; ++i) {
 		fill_zero(p.moments[i].ensure(p.bytes()), p.bytes());
@@ -1650,10 +1731,12 @@ void run_optimizer_many(const cattle_hip_layer_t* layers, const size_t* indices,
 	 * others are added to their gradients first, in one launch for all layers. */
 	std::vector<Param*> seen, limited;
 	std::vector<std::pair<Param*, ReduceEntry<T>>> riding;
+	for (size_t i = 0; i < count; ++i)
+		CATTLE_HIP_REQUIRE(optimizable_param(layers[i], indices[i]).esize == sizeof(T), "parameters of one optimizer step must share a scalar type");
 	for (size_t i = 0; i < count; ++i) {
 		Param& p = optimizable_param(layers[i], indices[i]);
 		ReduceEntry<T> e;
-		if (p.esize == sizeof(T) && !p.constrains_grad() && g_deferred.take_for_optimizer<T>(static_cast<const T*>(p.grad.p), e))
+		if (!p.constrains_grad() && g_deferred.take_for_optimizer<T>(static_cast<const T*>(p.grad.p), e))
 			riding.push_back(std::make_pair(&p, e));
 	}
 	g_deferred.settle();
@@ -1665,7 +1748,6 @@ void run_optimizer_many(const cattle_hip_layer_t* layers, const size_t* indices,
 	};
 	for (size_t i = 0; i < count; ++i) {
 		Param& p = optimizable_param(layers[i], indices[i]);
-		CATTLE_HIP_REQUIRE(p.esize == sizeof(T), "parameters of one optimizer step must share a scalar type");
 		if (std::find(seen.begin(), seen.end(), &p) != seen.end())
 			continue;
 		seen.push_back(&p);
@@ -1684,16 +1766,23 @@ void run_optimizer_many(const cattle_hip_layer_t* layers, const size_t* indices,
 		q.l2 = (T) p.reg_l2;
 		q.parts = nullptr;
 		q.splits = 0;
+		if (p.constrains_grad())
+			(void) p.whole_grad();
+		q.has_grad = !p.clear_due;
 		for (const std::pair<Param*, ReduceEntry<T>>& r : riding)
 			if (r.first == &p) {
 				q.parts = r.second.partials;
 				q.splits = r.second.splits;
+				q.has_grad = !r.second.fresh;
 			}
 		if (p.constrains_grad() && (p.reg_l1 != 0 || p.reg_l2 != 0)) {
 			add_regularization<T>(p.rows * p.cols, static_cast<const T*>(p.values.p), static_cast<T*>(p.grad.p), q.l1, q.l2);
 			constrain(p, false);
 			q.l1 = q.l2 = (T) 0;
 		}
+		q.clear_grad = !p.overwritten || capturing();
+		if (!q.clear_grad)
+			p.mark_clear();
 		q.wt_fwd = q.wt_dgrad = nullptr;
 		q.K = q.RHW = 1;
 		q.ldw_fwd = q.ldw_dgrad = 0;
@@ -1931,6 +2020,7 @@ int cattle_hip_graph_begin_capture(void) {
 		if (g_capturing)
 			throw Error(ERR_STATE, "a graph is already being recorded");
 		g_deferred.settle();            /* nothing pending crosses into the recording ... */
+		g_clears.settle();
 		CATTLE_HIP_CHECK(hipStreamBeginCapture(stream(), hipStreamCaptureModeRelaxed));
 		g_capturing = true;
 	});
@@ -1981,7 +2071,8 @@ int cattle_hip_graph_launch(cattle_hip_graph_t graph) {
 	return guarded([&] {
 		CATTLE_HIP_REQUIRE(graph != nullptr, "null graph handle");
 		forbid_while_capturing("launching a graph");
-		g_deferred.settle();            /* the recorded calls did not know of sums that eager passes have left pending since */
+		g_deferred.settle();            /* the recorded calls did not know of sums that eager passes have left pending since, */
+		g_clears.settle();              /* nor of gradients that they have reset */
 		CATTLE_HIP_CHECK(hipGraphLaunch(reinterpret_cast<Graph*>(graph)->exec, stream()));
 	});
 }
@@ -2235,7 +2326,7 @@ int cattle_hip_convlstm_get_kernel_grad(cattle_hip_layer_t lstm, size_t kernel, 
 		size_t offset, bytes;
 		Param& p = lstm_kernel_param(lstm, kernel, bias, offset, bytes);
 		g_deferred.settle();
-		copy_out(grad, space, (const char*) p.grad.p + offset, bytes);
+		copy_out(grad, space, (const char*) p.whole_grad() + offset, bytes);
 	});
 }
 
@@ -2606,8 +2697,9 @@ int cattle_hip_layer_get_param_grad(cattle_hip_layer_t layer, size_t index, void
 		check_space(space);
 		CATTLE_HIP_REQUIRE(grad != nullptr, "null buffer");
 		Param& p = param_at(as_layer(layer), index);
-		g_deferred.settle();
-		copy_out(grad, space, p.grad.p, p.bytes());
+		if (space == CATTLE_HIP_DEVICE ? g_deferred.settle(p.grad.p, grad) : g_deferred.settle())
+			return;                     /* the launch that made the gradient whole wrote it there as well */
+		copy_out(grad, space, p.whole_grad(), p.bytes());
 	});
 }
 
@@ -2615,7 +2707,10 @@ int cattle_hip_layer_reset_param_grad(cattle_hip_layer_t layer, size_t index) {
 	return guarded([&] {
 		Param& p = param_at(as_layer(layer), index);
 		g_deferred.settle();
-		fill_zero(p.grad.p, p.bytes());
+		if (p.overwritten && !capturing())
+			p.mark_clear();
+		else
+			fill_zero(p.whole_grad(), p.bytes());
 	});
 }
 

@@ -265,7 +265,7 @@ template<bool ACT>
 __global__ __launch_bounds__(64 * GRAD_WAVES)
 void small_weight_gradient_kernel(const float* __restrict__ x, const float* __restrict__ og, float* __restrict__ wgrad, float* __restrict__ bgrad,
 		int M, int K, int F, int ktiles, int tiles, unsigned x_bytes, unsigned og_bytes, const float* __restrict__ act_y, float* __restrict__ act_dz,
-		float p0, float p1) {
+		float p0, float p1, bool fresh) {
 	constexpr int ROWS = 64 / UNITS, LOADS = GL / ROWS;             /* rows per load of a wavefront, loads per operand and half */
 	/* a wavefront's half shares of x and z; then its partial tile in the place of x and its column sums in that of z */
 	extern __shared__ f32x4 stage[];                                /* [wavefront][x, z][column][unit] */
@@ -298,7 +298,7 @@ void small_weight_gradient_kernel(const float* __restrict__ x, const float* __re
 	#pragma unroll
 	for (int i = 0; i < 4; ++i) {
 		const int o = tid + i * (int) blockDim.x, k = k0 + o % GL, f = f0 + o / GL;
-		before[i] = o < GL * GL && k < K && f < F ? wgrad[(size_t) k + (size_t) K * f] : 0.f;
+		before[i] = !fresh && o < GL * GL && k < K && f < F ? wgrad[(size_t) k + (size_t) K * f] : 0.f;
 	}
 	__builtin_amdgcn_sched_barrier(0);
 	typename Mfma<float>::acc_t acc;
@@ -370,7 +370,7 @@ void small_weight_gradient_kernel(const float* __restrict__ x, const float* __re
 		const int k = k0 + o % GL, f = f0 + o / GL;
 		if (k < K && f < F) {
 			float* dst = wgrad + ((size_t) k + (size_t) K * f);
-			*dst = (fetched ? old : *dst) + v;
+			*dst = (fetched ? old : fresh ? 0.f : *dst) + v;
 		}
 	};
 	#pragma unroll
@@ -383,7 +383,7 @@ void small_weight_gradient_kernel(const float* __restrict__ x, const float* __re
 		float v = red[GL * GL + tid];
 		for (int w = 1; w < waves; ++w)
 			v += red[w * STRIDE + GL * GL + tid];
-		bgrad[f0 + tid] += v;
+		bgrad[f0 + tid] = fresh ? v : bgrad[f0 + tid] + v;
 	}
 }
 
@@ -462,17 +462,17 @@ bool small_weight_gradient_possible(const GatherGeom& g, bool vec, const WgradAc
 }
 
 void small_weight_gradient(const float* x, const float* og, float* wgrad, float* bgrad, const GatherGeom& g, const WgradAct<float>* act,
-		float p0, float p1) {
+		float p0, float p1, bool fresh) {
 	const int ktiles = up(g.K, GL), tiles = ktiles * up(g.F, GL);
 	const dim3 grid((unsigned) up(tiles, 8) * 8), block(64u * (unsigned) up(g.M, WAVE_M));
 	const unsigned x_bytes = 4u * (unsigned) g.M * (unsigned) g.K, og_bytes = 4u * (unsigned) g.M * (unsigned) g.F;
 	const size_t lds = (block.x / 64) * 2 * GL * GL * sizeof(float);
 	if (act)
 		small_weight_gradient_kernel<true><<<grid, block, lds, stream()>>>(x, og, wgrad, bgrad, g.M, g.K, g.F, ktiles, tiles, x_bytes, og_bytes,
-				act->y, act->dz, p0, p1);
+				act->y, act->dz, p0, p1, fresh);
 	else
 		small_weight_gradient_kernel<false><<<grid, block, lds, stream()>>>(x, og, wgrad, bgrad, g.M, g.K, g.F, ktiles, tiles, x_bytes, og_bytes,
-				(const float*) nullptr, (float*) nullptr, 0.f, 0.f);
+				(const float*) nullptr, (float*) nullptr, 0.f, 0.f, fresh);
 	CATTLE_HIP_CHECK(hipGetLastError());
 }
 

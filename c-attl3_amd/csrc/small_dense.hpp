@@ -24,9 +24,9 @@ void small_product_ordered(const float* src, const float* wt, const float* bias,
  * what `act` holds lie on 16-byte boundaries and g.N is a multiple of four (`vec`). */
 bool small_weight_gradient_possible(const GatherGeom& g, bool vec, const WgradAct<float>* act);
 /* wgrad += x^T z, bgrad += column sums of z, with z the gradient og or, with `act`, what WgradAct says (p0 + p1 y: the derivative
- * on the negative side) */
+ * on the negative side); with `fresh` the gradients are overwritten, not added to */
 void small_weight_gradient(const float* x, const float* og, float* wgrad, float* bgrad, const GatherGeom& g, const WgradAct<float>* act,
-		float p0, float p1);
+		float p0, float p1, bool fresh);
 
 } /* namespace cattle_hip */
 

@@ -502,8 +502,8 @@ void add_regularization_kernel(size_t n, const T* __restrict__ values, T* __rest
  * 784 x 512, 512 x 256 and 256 x 10 weights, both prepared layouts rewritten, 7.8 -> 7.2 us; Adam on the 70 thousand parameters of a
  * small image classifier 5.8 -> 5.3, Nadam on 63 thousand with up to eight partial sums each 10.0 -> 6.2.
  * An element's gradient is what has been accumulated plus the partial sums that still wait, these added up first, in ascending
- * order from zero (the order and grouping of reduce_partials_many for so few of them). Writes the new value, state and a
- * gradient of zero, and returns the values. */
+ * order from zero (the order and grouping of reduce_partials_many for so few of them). Writes the new value and state and, if
+ * it is to be cleared here, a gradient of zero; returns the values. */
 template<typename T, int RULE>
 __device__ __forceinline__ void step_of_four(const OptParam<T>& q, const OptCoef<T>& k, const size_t (&at)[4], const bool (&in)[4], T (&values)[4]) {
 	constexpr int S = states_of(RULE);
@@ -511,7 +511,7 @@ __device__ __forceinline__ void step_of_four(const OptParam<T>& q, const OptCoef
 	#pragma unroll
 	for (int j = 0; j < 4; ++j) {
 		const size_t i = in[j] ? at[j] : 0;
-		g[j] = q.grad[i];
+		g[j] = q.has_grad ? q.grad[i] : (T) 0;
 		v[j] = q.values[i];
 		s0[j] = S > 0 ? q.s0[i] : (T) 0;
 		s1[j] = S > 1 ? q.s1[i] : (T) 0;
@@ -538,7 +538,8 @@ __device__ __forceinline__ void step_of_four(const OptParam<T>& q, const OptCoef
 	for (int j = 0; j < 4; ++j)
 		if (in[j]) {
 			q.values[at[j]] = values[j];
-			q.grad[at[j]] = (T) 0;
+			if (q.clear_grad)
+				q.grad[at[j]] = (T) 0;
 			if (S > 0)
 				q.s0[at[j]] = s0[j];
 			if (S > 1)
