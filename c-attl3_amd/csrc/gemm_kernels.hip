@@ -21,6 +21,7 @@
 #include "gemm_bf16x3.hpp"
 #include "lstm_steps.hpp"
 #include "small_dense.hpp"
+#include "few_weights.hpp"
 #include "gemm_tiles.hpp"
 #include "act_math.hpp"
 #include "lstm_math.hpp"
@@ -1345,6 +1346,20 @@ void few_columns_with_wgrad_kernel(const T* __restrict__ src, const T* __restric
 	}
 }
 
+/* The same with a weight gradient of few weights (few_weights.hpp): blocks of four wavefronts each, and 32 KB of dynamic LDS. */
+template<typename T, int VEC, int UNROLL, int NC, int GQ>
+__global__ __launch_bounds__(256)
+void few_columns_with_few_weights_kernel(const T* __restrict__ src, const T* __restrict__ wt, T* __restrict__ out, const GatherGeom g,
+		int gather_blocks, const few_weights::FewWeights W) {
+	extern __shared__ few_weights::f32x4 few_weights_stage[];
+	if ((int) blockIdx.x < gather_blocks) {
+		few_columns_body<T, VEC, false, UNROLL, NC>(src, wt, (const T*) nullptr, out, g, few_columns_block<VEC>(g, (int) blockIdx.x));
+	} else {
+		const int b = (int) blockIdx.x - gather_blocks, k_tile = b / W.slices;
+		few_weights::few_weights_body<GQ>(W, b - k_tile * W.slices, k_tile, few_weights_stage);
+	}
+}
+
 /* ------------------------------------------------------------------------------------------------
  * The weight gradient of a convolution with up to four filters (the last layer of an image decoder: many channels in, an
  * image out), dW[K x F] = patches(x)^T [K x M] * G[M x F], without matrix tiles: a 32 x 32 tile would be seven eighths
@@ -1752,6 +1767,7 @@ struct WgradRider {
 	GatherGeom g;
 	WgradSplit plan;
 	bool done;
+	const few_weights::FewWeights* few;     /* or null: the weight gradient is this one, and nothing above but `done` counts */
 };
 
 /* One instantiation of gather_gemm_kernel and what the tile chooser needs to know about it. */
@@ -2274,7 +2290,26 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 			return false;
 		if (epi == EPI_NONE && g.F <= FEW_COLUMNS && rider && wide && !divs && bias == nullptr) {
 			const unsigned w_blocks = (unsigned) round_up(rider->plan.tiles * rider->plan.splits, 8);
-			with_walk([&](auto w) {
+			bool rides = false;
+			if constexpr (std::is_same<T, float>::value)
+				if (rider->few) {
+					const unsigned few_blocks = (unsigned) (rider->few->slices * ((rider->few->g.K + 31) / 32));
+					with_walk([&](auto w) {
+						const auto launch = [&](auto c, auto gq) {
+							few_columns_with_few_weights_kernel<T, V, decltype(w)::value, decltype(c)::value, decltype(gq)::value>
+									<<<blocks + few_blocks, 256, 4 * 8192, stream()>>>(src, wt, out, g, (int) blocks, *rider->few);
+						};
+						typedef std::integral_constant<int, 1> one;
+						typedef std::integral_constant<int, 2> two;
+						if (g.F == 3)
+							rider->few->g.F <= 8 ? launch(std::integral_constant<int, 3>(), one()) : launch(std::integral_constant<int, 3>(), two());
+						else
+							rider->few->g.F <= 8 ? launch(std::integral_constant<int, FEW_COLUMNS>(), one()) :
+									launch(std::integral_constant<int, FEW_COLUMNS>(), two());
+					});
+					rides = true;
+				}
+			if (!rides) with_walk([&](auto w) {
 				if (g.F == 3)
 					few_columns_with_wgrad_kernel<T, V, decltype(w)::value, 3><<<blocks + w_blocks, 256, 0, stream()>>>(src, wt, out, g, (int) blocks,
 							rider->x, rider->og, rider->partials, rider->bias_partials, rider->g, rider->plan);
@@ -2387,7 +2422,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 	const GatherVariant<T>* chosen = &vars[best_v];
 	bool cuts = true;
 	if constexpr (std::is_same<T, float>::value)
-		if (epi != EPI_LSTM && !divs && then == nullptr && !(rider && chosen->launch_with_wgrad)) {
+		if (epi != EPI_LSTM && !divs && then == nullptr && !(rider && !rider->few && chosen->launch_with_wgrad)) {
 			const CutReductions fp32_cut = cut_reductions(*chosen, g, no_split, vec, divs, epi, 0);
 			const int resident = chosen->blocks_per_cu(0, vec, divs, epi);
 			/* (few tiles whose reductions the wavefronts of a block share are that launch either way) */
@@ -2512,7 +2547,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 		launch();
 		return true;
 	}
-	if (rider && v.launch_with_wgrad && epi == EPI_NONE && bias == nullptr && then == nullptr && vec && !divs && dyn == 0 &&
+	if (rider && !rider->few && v.launch_with_wgrad && epi == EPI_NONE && bias == nullptr && then == nullptr && vec && !divs && dyn == 0 &&
 			g.out_sa == 1 && g.out_sb == 1 && g.out_a0 == 0 && g.out_b0 == 0 && g.out_OA == g.OA && g.out_M == g.M) {
 		/* whole tiles only, and a small weight gradient that waits for the same upstream gradient: one launch for both */
 		const GatherLaunch L = { mtiles, tile_rows, mtiles, round_up(mtiles, 8), 0, 1, nchunks, sample_blocks, pos_b, sb_shift };
@@ -3192,11 +3227,20 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 	static_assert(WGRAD_MC == 32, "the chunk length gather_with_wgrad_kernel is built with");
 	/* (a larger one that stays on the fp32 instructions does not ride: it would hold the input gradient there too, 368 x 1549 x 442
 	 * backward 60 us against 36) */
-	const bool can_ride = elsewhere != nullptr && !bf16x3 && (g.fp32_products || 2.0 * g.M * g.K * g.F < BF16X3_WGRAD_FLOPS) &&
+	bool is_few_weights = false;
+	if constexpr (std::is_same<T, float>::value)
+		/* (a group with a max pool keeps the order of its sums: its first layer's gradient may be formed in another launch, from the
+		 * pooled gradient, and does not depend on which) */
+		if (!act && !few_filters && !bf16x3 && !g.fp32_products && p.splits > 1 && few_weights_possible(g, vec)) {
+			is_few_weights = true;
+			p.splits = few_weights_slices(g, p.splits);
+			bias_partials = partials + (size_t) p.splits * count;
+		}
+	const bool can_ride = elsewhere != nullptr && !bf16x3 && !is_few_weights && (g.fp32_products || 2.0 * g.M * g.K * g.F < BF16X3_WGRAD_FLOPS) &&
 			std::is_same<T, float>::value && !act && vec && v.bk == 32 && v.bf == 32 &&
 			v.waves == 1 && v.mc == WGRAD_MC;
 	if constexpr (std::is_same<T, float>::value)
-		if (!can_ride && !bf16x3 && small_weight_gradient_possible(g, vec, act)) {
+		if (!can_ride && !bf16x3 && !is_few_weights && small_weight_gradient_possible(g, vec, act)) {
 			T p0, p1;
 			negative_side(act, &p0, &p1);
 			small_weight_gradient(x, out_grad, wgrad, bgrad, g, act, p0, p1, fresh);
@@ -3218,18 +3262,26 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 			return;
 		}
 		if constexpr (std::is_same<T, float>::value)
+			if (is_few_weights) {
+				const few_weights::FewWeights problem = few_weights_problem(x, out_grad, to_w, to_b, g, how.splits);
+				WgradRider<T> rider = { x, out_grad, to_w, to_b, g, how, false, &problem };
+				if (!elsewhere || !(*elsewhere)(rider))
+					few_weights_gradient(problem);
+				return;
+			}
+		if constexpr (std::is_same<T, float>::value)
 			if (bf16x3) {
 				bf16x3_wgrad(b3, x, out_grad, to_w, to_b, g);
 				return;
 			}
 		if (can_ride) {
-			WgradRider<T> rider = { x, out_grad, to_w, to_b, g, how, false };
+			WgradRider<T> rider = { x, out_grad, to_w, to_b, g, how, false, nullptr };
 			if ((*elsewhere)(rider))
 				return;
 		}
 		v.launch(x, out_grad, to_w, to_b, g, how, vec, act);
 	};
-	if (p.splits == 1) {
+	if (p.splits == 1 && !is_few_weights) {
 		/* one slice: every block owns its tile of the gradient and adds to it directly, no second launch */
 		const WgradSplit direct = { p.ktiles, p.ktiles * p.ftiles, 1, p.chunks_per_split, p.pixel_mode, fresh ? 0 : 1 };
 		if (fresh)

@@ -273,7 +273,8 @@ struct Param {
 	 * buffer holds. That backward pass takes the mark off by storing its gradient; whoever else needs the buffer calls
 	 * whole_grad(), which zeroes it first. Spares a launch per parameter and pass, and the optimizer and the weight gradient a write
 	 * and a read of it: a convolution of 64 x 32 x 32 x 3 with its gradients read and reset 26.8 -> 24 us a pass, a dense layer of
-	 * 512 x 4096 -> 1024 127.6 -> 115.9. Recordings know nothing of marks: they are settled before a recording begins and before a graph is launched, and none are set in between. */
+	 * 512 x 4096 -> 1024 127.6 -> 115.9. Recordings know nothing of marks: they are settled before a recording begins and before a
+	 * graph is launched, and none are set in between. */
 	bool overwritten = false, clear_due = false;
 	void* whole_grad();
 	void mark_clear();
