@@ -87,6 +87,8 @@ struct ConvShape {
 	bool fp32_products = false;
 	/* The sums of the forward product in the order that the tiled launches take them (FusedLayer::shape says who asks for it). */
 	bool keeps_sums = false;
+	/* The weights are given as the F x K matrix, not the K x F one (the convolution that a transposed convolution's passes are). */
+	bool weights_transposed = false;
 	int OH() const { return (H - RH - (RH - 1) * dv + 2 * pv) / sv + 1; }
 	int OW() const { return (W - RW - (RW - 1) * dh + 2 * ph) / sh + 1; }
 	int K() const { return RH * RW * C; }
@@ -177,6 +179,14 @@ template<typename T> struct LstmBackwardStep;
  * be run (lstm_gates_backward). */
 template<typename T> bool conv_input_gradient(const ConvShape& s, int N, const T* w, const T* out_grad, T* in_grad,
 		T* wt_dgrad, bool wt_ready, const LstmBackwardStep<T>* then = nullptr, int og_batch = 0);
+/* The same as the forward pass of a transposed convolution, whose bias has an entry per output activation (position + H W channel):
+ * in_grad = input gradient + bias. Returns whether the launch added the bias; false: the caller adds it. */
+template<typename T> bool conv_input_gradient_biased(const ConvShape& s, int N, const T* w, const T* out_grad, const T* bias, T* in_grad,
+		T* wt_dgrad, bool wt_ready);
+/* The weight gradient as the F x K matrix, for a problem with few weights: its slices are left to the caller (`deferred`, one entry;
+ * `fresh`: see conv_weight_gradient). Returns false, having launched nothing, where there is no such launch. */
+template<typename T> bool conv_weight_gradient_transposed(const ConvShape& s, int N, const T* x, const T* out_grad, T* wgrad_t,
+		T* partials, ReduceBatch<T>* deferred, bool fresh);
 /* Which prepared layout conv_input_gradient builds in wt_dgrad at this batch size: 0 the plain one (all taps), 1 the
  * blocks of a strided convolution's residue classes. Prepared weights are current only for the layout they were built as. */
 template<typename T> int dgrad_weight_layout(const ConvShape& s, int N);

@@ -37,9 +37,10 @@ int few_weights_slices(const GatherGeom& g, int most) {
 	return (items + per - 1) / per;
 }
 
-few_weights::FewWeights few_weights_problem(const float* x, const float* og, float* partials, float* bias_partials, const GatherGeom& g, int slices) {
+few_weights::FewWeights few_weights_problem(const float* x, const float* og, float* partials, float* bias_partials, const GatherGeom& g, int slices,
+		bool transposed) {
 	const int items = items_of(g), per = (items + slices - 1) / slices;
-	return { x, og, partials, bias_partials, g, items, groups_of(g), per, slices, 4u * (unsigned) (g.NS * g.LH * g.LW) * (unsigned) g.LC,
+	return { x, og, partials, bias_partials, g, items, groups_of(g), per, slices, transposed, 4u * (unsigned) (g.NS * g.LH * g.LW) * (unsigned) g.LC,
 			4u * (unsigned) g.M * (unsigned) g.F };
 }
 

@@ -42,6 +42,7 @@ struct FewWeights {
 	float *partials, *bias_partials;
 	GatherGeom g;
 	int items, groups, per_slice, slices;
+	bool transposed;        /* a slice is F x K, not K x F */
 	unsigned x_bytes, og_bytes;
 };
 /* stage: 8 KB per wavefront of the block: [wavefront][x, og][row][unit], then partial tiles and column sums */
@@ -153,7 +154,7 @@ __device__ __forceinline__ void few_weights_body(const FewWeights& A, int slice,
 			v += red[w * STRIDE + o];
 		const int k = k0 + o % TL, f = o / TL;
 		if (k < g.K && f < g.F)
-			dst[(size_t) k + (size_t) g.K * f] = v;
+			dst[A.transposed ? (size_t) f + (size_t) g.F * k : (size_t) k + (size_t) g.K * f] = v;
 	}
 	if (sums_bias && tid < g.F) {
 		float v = red[TL * TL + tid];
@@ -171,7 +172,8 @@ bool few_weights_possible(const GatherGeom& g, bool vec);
 /* The slices it writes, at most `most`. */
 int few_weights_slices(const GatherGeom& g, int most);
 /* partials[slice][K x F], bias_partials[slice][F] (or null): the sums of x^T og and of og over the slice's rows */
-few_weights::FewWeights few_weights_problem(const float* x, const float* og, float* partials, float* bias_partials, const GatherGeom& g, int slices);
+few_weights::FewWeights few_weights_problem(const float* x, const float* og, float* partials, float* bias_partials, const GatherGeom& g, int slices,
+		bool transposed = false);
 void few_weights_gradient(const few_weights::FewWeights& problem);
 
 } /* namespace cattle_hip */

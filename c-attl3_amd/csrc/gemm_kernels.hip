@@ -978,35 +978,36 @@ void reduce_partials_many_kernel(const ReduceBatch<T> batch) {
 }
 
 /* Forward weights: wt[k][f] = w[k + K*f], zero-padded to Kp rows x ldw columns. gate_block > 0: the columns in the
- * order of lstm_gate_column (F = 4 * hidden). */
+ * order of lstm_gate_column (F = 4 * hidden). transposed, here and below: w is F x K (ConvShape::weights_transposed). */
 template<typename T>
 __global__ void prep_fwd_weights_kernel(const T* __restrict__ w, T* __restrict__ wt, int K, int F, int Kp, int ldw,
-		int gate_block = 0) {
+		int gate_block = 0, bool transposed = false) {
 	const size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= (size_t) Kp * ldw)
 		return;
 	const int f = (int) (i % ldw), k = (int) (i / ldw);
 	const int fs = gate_block > 0 && f < F ? lstm_gate_column(f, gate_block, F / 4) : f;
-	wt[i] = (k < K && f < F) ? w[(size_t) k + (size_t) K * fs] : (T) 0;
+	wt[i] = (k < K && f < F) ? w[transposed ? (size_t) fs + (size_t) F * k : (size_t) k + (size_t) K * fs] : (T) 0;
 }
 
 /* Input-gradient weights: wt[k' = rh + RH*(rw + RW*f)][c] = w[rh + RH*(rw + RW*c) + K*f]. */
 template<typename T>
 __global__ void prep_dgrad_weights_kernel(const T* __restrict__ w, T* __restrict__ wt, int RHW, int C, int F, int Kp,
-		int ldw) {
+		int ldw, bool transposed) {
 	const size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= (size_t) Kp * ldw)
 		return;
 	const int c = (int) (i % ldw), kp = (int) (i / ldw);
 	const int tap = kp % RHW, f = kp / RHW;
-	wt[i] = (f < F && c < C) ? w[(size_t) (tap + RHW * c) + (size_t) (RHW * C) * f] : (T) 0;
+	const size_t k = (size_t) (tap + RHW * c);
+	wt[i] = (f < F && c < C) ? w[transposed ? (size_t) f + (size_t) F * k : k + (size_t) (RHW * C) * f] : (T) 0;
 }
 
 /* Input-gradient weights of one residue class of a strided convolution (see StridedClasses): the receptor rows
  * r0, r0 + sv, ... and columns s0, s0 + sh, ... only, wt[k' = r' + Rc*(s' + Sc*f)][c] = w[(r0 + sv r') + RH*((s0 + sh s') + RW*c) + K*f]. */
 template<typename T>
 __global__ void prep_dgrad_class_weights_kernel(const T* __restrict__ w, T* __restrict__ wt, int RH, int RW, int C, int F,
-		int r0, int sv, int Rc, int s0, int sh, int Sc, int Kp, int ldw) {
+		int r0, int sv, int Rc, int s0, int sh, int Sc, int Kp, int ldw, bool transposed) {
 	const size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= (size_t) Kp * ldw)
 		return;
@@ -1014,7 +1015,8 @@ __global__ void prep_dgrad_class_weights_kernel(const T* __restrict__ w, T* __re
 	const int taps = Rc * Sc;
 	const int tap = kp % taps, f = kp / taps;
 	const int r = r0 + sv * (tap % Rc), sb = s0 + sh * (tap / Rc);
-	wt[i] = (f < F && c < C) ? w[(size_t) (r + RH * (sb + RW * c)) + (size_t) (RH * RW * C) * f] : (T) 0;
+	const size_t k = (size_t) (r + RH * (sb + RW * c));
+	wt[i] = (f < F && c < C) ? w[transposed ? (size_t) f + (size_t) F * k : k + (size_t) (RH * RW * C) * f] : (T) 0;
 }
 
 int round_up(int v, int to) {
@@ -1118,7 +1120,8 @@ void* g_scratch_ptr[MAX_DEVICES] = { nullptr };
 constexpr int FEW_COLUMNS = 4, SOME_COLUMNS = 8;
 template<typename T, int VEC, bool DIVS, int UNROLL, int NC = FEW_COLUMNS>
 __device__ __forceinline__ void few_columns_body(const T* __restrict__ src, const T* __restrict__ wt, const T* __restrict__ bias,
-		T* __restrict__ out, const GatherGeom& g, int block, int act_kind = -1, T act_p = (T) 0, T* __restrict__ act_pre = nullptr) {
+		T* __restrict__ out, const GatherGeom& g, int block, int act_kind = -1, T act_p = (T) 0, T* __restrict__ act_pre = nullptr,
+		int bias_stride = 0) {
 	constexpr int WAVES = 4, ROWS = 64 * VEC;
 	const int lane = threadIdx.x % 64;
 	const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x / 64);
@@ -1267,6 +1270,8 @@ __device__ __forceinline__ void few_columns_body(const T* __restrict__ src, cons
 	}
 	__syncthreads();
 	if (wave == 0 && mvalid) {
+		/* (bias_stride > 0: a bias per output position and column; a lane's rows are samples of one position where it has several) */
+		const int bias_pos = bias_stride > 0 ? m / g.N : 0;
 		#pragma unroll
 		for (int c = 0; c < NC; ++c) {
 			if (c < g.F) {
@@ -1278,7 +1283,7 @@ __device__ __forceinline__ void few_columns_body(const T* __restrict__ src, cons
 					for (int i = 0; i < VEC; ++i)
 						acc[c][i] += part[i];
 				}
-				const T bv = bias ? bias[c] : (T) 0;
+				const T bv = bias ? bias[bias_stride > 0 ? bias_pos + (size_t) bias_stride * c : (size_t) c] : (T) 0;
 				#pragma unroll
 				for (int i = 0; i < VEC; ++i)
 					acc[c][i] += bv;
@@ -1317,15 +1322,16 @@ __device__ __forceinline__ int few_columns_block(const GatherGeom& g, int bid) {
 template<typename T, int VEC, bool DIVS, int UNROLL>
 __global__ __launch_bounds__(256)
 void few_columns_gather_kernel(const T* __restrict__ src, const T* __restrict__ wt, const T* __restrict__ bias,
-		T* __restrict__ out, const GatherGeom g) {
-	few_columns_body<T, VEC, DIVS, UNROLL>(src, wt, bias, out, g, few_columns_block<VEC>(g, (int) blockIdx.x));
+		T* __restrict__ out, const GatherGeom g, int bias_stride) {
+	few_columns_body<T, VEC, DIVS, UNROLL>(src, wt, bias, out, g, few_columns_block<VEC>(g, (int) blockIdx.x), -1, (T) 0, nullptr, bias_stride);
 }
 
 template<typename T, int VEC, int UNROLL, int NC = FEW_COLUMNS>
 __global__ __launch_bounds__(256)
 void few_columns_plain_kernel(const T* __restrict__ src, const T* __restrict__ wt, const T* __restrict__ bias,
-		T* __restrict__ out, const GatherGeom g, int act_kind, T act_p, T* __restrict__ act_pre) {
-	few_columns_body<T, VEC, false, UNROLL, NC>(src, wt, bias, out, g, few_columns_block<VEC>(g, (int) blockIdx.x), act_kind, act_p, act_pre);
+		T* __restrict__ out, const GatherGeom g, int act_kind, T act_p, T* __restrict__ act_pre, int bias_stride) {
+	few_columns_body<T, VEC, false, UNROLL, NC>(src, wt, bias, out, g, few_columns_block<VEC>(g, (int) blockIdx.x), act_kind, act_p, act_pre,
+			bias_stride);
 }
 
 /* An input gradient of a few columns and the layer's weight gradient in one launch (see gather_with_wgrad_kernel: both
@@ -2240,7 +2246,8 @@ Bf16x3Choice bf16x3_for(const GatherProblem& g, long M, bool no_split, double fp
 template<typename T>
 bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const GatherProblem& g, ScratchArena* arena = nullptr,
 		int epi = EPI_NONE, const Epilogue<T>* E = nullptr, int* mtiles_out = nullptr, const LstmBackwardStep<T>* then = nullptr,
-		bool* then_done = nullptr, const std::function<void(int bf)>* before_launch = nullptr, WgradRider<T>* rider = nullptr) {
+		bool* then_done = nullptr, const std::function<void(int bf)>* before_launch = nullptr, WgradRider<T>* rider = nullptr,
+		const T* position_bias = nullptr, bool* position_bias_done = nullptr) {
 	g_last_products.product = 0;
 	const bool vec = g.N % GemmCfg<T>::VEC == 0 && g.NS % GemmCfg<T>::VEC == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
 	const bool divs = g.DA != 1 || g.DB != 1;
@@ -2264,6 +2271,13 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 		/* a handful of output columns: no matrix tiles (few_columns_gather_kernel); five to eight of them in the
 		 * vectorised forward form only */
 		constexpr int V = GemmCfg<T>::VEC;
+		/* a bias per output activation (a transposed convolution's), where a lane's rows are samples of one position */
+		int bias_stride = 0;
+		if (position_bias && bias == nullptr && g.out_OA == g.OA && g.out_M == g.M) {
+			bias = position_bias;
+			bias_stride = g.OA * g.OB;
+			*position_bias_done = true;
+		}
 		const unsigned blocks = (unsigned) round_up((g.M + (wide ? 64 * V : 64) - 1) / (wide ? 64 * V : 64), 8);   /* few_columns_block */
 		/* how a wave walks the reduction (few_columns_body): with up to eight source channels, steps of all taps in batches
 		 * (0); else tap by tap with a wave's share of the channels in whole batches of loads, eight to a batch if that
@@ -2319,18 +2333,18 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 			});
 			rider->done = true;
 		} else if (wide && divs)
-			few_columns_gather_kernel<T, V, true, 8><<<blocks, 256, 0, stream()>>>(src, wt, bias, out, g);
+			few_columns_gather_kernel<T, V, true, 8><<<blocks, 256, 0, stream()>>>(src, wt, bias, out, g, bias_stride);
 		else if (wide)
 			with_walk([&](auto w) {
 				with_columns([&](auto c) {
 					few_columns_plain_kernel<T, V, decltype(w)::value, decltype(c)::value><<<blocks, 256, 0, stream()>>>(src, wt, bias, out, g,
-							act_kind, act_p, act_pre);
+							act_kind, act_p, act_pre, bias_stride);
 				});
 			});
 		else if (divs)
-			few_columns_gather_kernel<T, 1, true, 8><<<blocks, 256, 0, stream()>>>(src, wt, bias, out, g);
+			few_columns_gather_kernel<T, 1, true, 8><<<blocks, 256, 0, stream()>>>(src, wt, bias, out, g, bias_stride);
 		else
-			few_columns_gather_kernel<T, 1, false, 8><<<blocks, 256, 0, stream()>>>(src, wt, bias, out, g);
+			few_columns_gather_kernel<T, 1, false, 8><<<blocks, 256, 0, stream()>>>(src, wt, bias, out, g, bias_stride);
 		CATTLE_HIP_CHECK(hipGetLastError());
 		if (mtiles_out)
 			*mtiles_out = 0;
@@ -3078,7 +3092,7 @@ void conv_forward(const ConvShape& s, int N, const T* x, const T* w, const T* b,
 	if (!wt_ready) {
 		const int Kp = round_up(g.K, WT_ROW_PAD);
 		const size_t count = (size_t) Kp * g.ldw;
-		prep_fwd_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, g.K, g.F, Kp, g.ldw);
+		prep_fwd_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, g.K, g.F, Kp, g.ldw, 0, s.weights_transposed);
 		CATTLE_HIP_CHECK(hipGetLastError());
 	}
 	launch_gather<T>(x, wt, b, out, g);
@@ -3179,7 +3193,8 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 		const WgradAct<T>* act, ReduceBatch<T>* deferred, bool fresh, const std::function<bool(WgradRider<T>&)>* elsewhere);
 template<typename T>
 bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* out_grad, T* in_grad, T* wt_dgrad, bool wt_ready,
-		const LstmBackwardStep<T>* then, int og_batch, WgradRider<T>* rider);
+		const LstmBackwardStep<T>* then, int og_batch, WgradRider<T>* rider, const T* position_bias = nullptr,
+		bool* position_bias_done = nullptr);
 
 template<typename T>
 void conv_weight_gradient(const ConvShape& s, int N, const T* x, const T* out_grad, T* wgrad, T* bgrad, T* partials,
@@ -3311,6 +3326,27 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 }
 
 template<typename T>
+bool conv_weight_gradient_transposed(const ConvShape& s, int N, const T* x, const T* out_grad, T* wgrad_t, T* partials,
+		ReduceBatch<T>* deferred, bool fresh) {
+	if constexpr (std::is_same<T, float>::value) {
+		check_sizes(s, N);
+		const GatherProblem g = forward_geom(s, N);
+		const bool vec = N % GemmCfg<T>::VEC == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(out_grad) & 15) == 0;
+		const WgradPlan p = wgrad_plan<T>(g.M, g.K, g.F, N, vec);
+		if (p.splits <= 1 || !few_weights_possible(g, vec))
+			return false;
+		const int slices = few_weights_slices(g, p.splits);
+		few_weights_gradient(few_weights_problem(x, out_grad, partials, nullptr, g, slices, true));
+		const size_t count = (size_t) g.K * g.F;
+		deferred->count = 1;
+		deferred->e[0] = ReduceEntry<T>{ partials, wgrad_t, count, slices, 0, count <= 8192 && slices >= 32,
+				count % 4 == 0 && (reinterpret_cast<uintptr_t>(partials) & 15) == 0, fresh, nullptr };
+		return true;
+	}
+	return false;
+}
+
+template<typename T>
 void reduce_partials_many(ReduceBatch<T> batch) {
 	if (batch.count == 0)
 		return;
@@ -3336,10 +3372,17 @@ bool conv_input_gradient(const ConvShape& s, int N, const T* w, const T* out_gra
 	return conv_input_gradient_with<T>(s, N, w, out_grad, in_grad, wt_dgrad, wt_ready, then, og_batch, nullptr);
 }
 
+template<typename T>
+bool conv_input_gradient_biased(const ConvShape& s, int N, const T* w, const T* out_grad, const T* bias, T* in_grad, T* wt_dgrad, bool wt_ready) {
+	bool done = false;
+	conv_input_gradient_with<T>(s, N, w, out_grad, in_grad, wt_dgrad, wt_ready, nullptr, 0, nullptr, bias, &done);
+	return done;
+}
+
 /* (`rider`: a small weight-gradient launch that may run inside this one, see WgradRider) */
 template<typename T>
 bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* out_grad, T* in_grad, T* wt_dgrad, bool wt_ready,
-		const LstmBackwardStep<T>* then, int og_batch, WgradRider<T>* rider) {
+		const LstmBackwardStep<T>* then, int og_batch, WgradRider<T>* rider, const T* position_bias, bool* position_bias_done) {
 	check_sizes(s, std::max(N, og_batch));
 	if (then == nullptr && use_strided_classes<T>(s, N)) {
 		std::vector<StridedClass> classes;
@@ -3360,7 +3403,7 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 			if (!wt_ready) {
 				const size_t count = (size_t) Kp * ldw;
 				prep_dgrad_class_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wtc, s.RH, s.RW, s.C, s.F,
-						c.r0, s.sv, c.Rc, c.s0, s.sh, c.Sc, Kp, ldw);
+						c.r0, s.sv, c.Rc, c.s0, s.sh, c.Sc, Kp, ldw, s.weights_transposed);
 				CATTLE_HIP_CHECK(hipGetLastError());
 			}
 			GatherProblem g;
@@ -3403,7 +3446,7 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 		const int Kp = round_up(d.K, WT_ROW_PAD);
 		const size_t count = (size_t) Kp * d.ldw;
 		prep_dgrad_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt_dgrad, s.RH * s.RW, s.C, s.F,
-				Kp, d.ldw);
+				Kp, d.ldw, s.weights_transposed);
 		CATTLE_HIP_CHECK(hipGetLastError());
 	}
 	if constexpr (std::is_same<T, float>::value)
@@ -3412,7 +3455,7 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 			return true;
 		}
 	bool then_done = false;
-	launch_gather<T>(out_grad, wt_dgrad, (const T*) nullptr, in_grad, d, nullptr, EPI_NONE, nullptr, nullptr, then, &then_done, nullptr, rider);
+	launch_gather<T>(out_grad, wt_dgrad, (const T*) nullptr, in_grad, d, nullptr, EPI_NONE, nullptr, nullptr, then, &then_done, nullptr, rider, position_bias, position_bias_done);
 	return then_done;
 }
 
@@ -3455,6 +3498,11 @@ template void conv_weight_gradient<float>(const ConvShape&, int, const float*, c
 		const WgradAct<float>*, ReduceBatch<float>*, bool);
 template void conv_weight_gradient<double>(const ConvShape&, int, const double*, const double*, double*, double*, double*,
 		const WgradAct<double>*, ReduceBatch<double>*, bool);
+template bool conv_input_gradient_biased<float>(const ConvShape&, int, const float*, const float*, const float*, float*, float*, bool);
+template bool conv_input_gradient_biased<double>(const ConvShape&, int, const double*, const double*, const double*, double*, double*, bool);
+template bool conv_weight_gradient_transposed<float>(const ConvShape&, int, const float*, const float*, float*, float*, ReduceBatch<float>*, bool);
+template bool conv_weight_gradient_transposed<double>(const ConvShape&, int, const double*, const double*, double*, double*, ReduceBatch<double>*,
+		bool);
 template void reduce_partials_many<float>(ReduceBatch<float>);
 template void reduce_partials_many<double>(ReduceBatch<double>);
 template int dgrad_weight_layout<float>(const ConvShape&, int);

@@ -624,21 +624,23 @@ struct ConvLayer : LayerBase {
 /* TransConvKernelLayer (layer/kernel/TransConvKernelLayer.hpp:143-216). Its forward pass scatters
  * in * W into the output, which is the input gradient of the convolution that maps the output back
  * to the input (same receptor, padding, stride, dilation; channels and filters exchanged) with
- * weights W^T; its backward pass is that convolution's forward pass (input gradient) and weight
+ * weights W^T (ConvShape::weights_transposed); its backward pass is that convolution's forward pass (input gradient) and weight
  * gradient (transposed). So the three GEMM kernels are reused as they are:
  *   weights W [C x RH*RW*F], column rh + RH*(rw + RW*f)   ->   Wc = W^T, the convolution's [K x C]
  *   bias    [1 x OH*OW*F], one entry per output activation (:52-56). */
 template<typename T>
 struct TransConvLayer : LayerBase {
-	ConvShape conv;                   /* the equivalent convolution: output dims -> input dims */
+	ConvShape conv;                   /* the equivalent convolution: output dims -> input dims, its weights W^T given as W */
 	const T* x_cache = nullptr;
-	DevBuf partials, wgrad_t;
+	DevBuf wgrad_t;
 
 	TransConvLayer(int dtype, const ConvShape& c) : LayerBase(dtype), conv(c) {
+		conv.weights_transposed = true;
 		in_dims[0] = (size_t) c.OH(); in_dims[1] = (size_t) c.OW(); in_dims[2] = (size_t) c.F;
 		out_dims[0] = (size_t) c.H; out_dims[1] = (size_t) c.W; out_dims[2] = (size_t) c.C;
 		params.push_back(std::make_shared<Param>((size_t) c.F, (size_t) c.K(), true, sizeof(T)));
 		params.push_back(std::make_shared<Param>(1, out_volume(), true, sizeof(T)));
+		params[0]->overwritten = true;
 	}
 	TransConvLayer(const TransConvLayer& o, bool share) : LayerBase(o.dtype), conv(o.conv) {
 		copy_base(o, share);
@@ -646,47 +648,46 @@ struct TransConvLayer : LayerBase {
 	LayerBase* clone(bool share) const override {
 		return new TransConvLayer(*this, share);
 	}
-	/* Wc = W^T, rebuilt when the weights change */
-	const T* conv_weights() {
-		Param& w = *params[0];
-		T* wc = (T*) w.derived[2].ensure(w.bytes());
-		if (w.derived_version[2] != w.version) {
-			transpose_matrix<T>((int) w.rows, (int) w.cols, (const T*) w.values.p, wc, false);
-			w.derived_version[2] = w.version;
-		}
-		return wc;
-	}
 	void forward(const void* in, size_t N, bool, void* out) override {
 		const int n = checked_int(N, "batch size");
 		const ConvWorkspace ws = conv_workspace<T>(conv, n);
 		Param& w = *params[0];
-		const T* wc = conv_weights();
 		T* wt = (T*) w.derived[1].ensure(ws.wt_dgrad * sizeof(T));
 		const int layout = dgrad_weight_layout<T>(conv, n);
-		conv_input_gradient<T>(conv, n, wc, (const T*) in, (T*) out, wt, w.derived_version[1] == w.version && w.dgrad_layout == layout);
+		const bool biased = conv_input_gradient_biased<T>(conv, n, (const T*) w.values.p, (const T*) in, (const T*) params[1]->values.p, (T*) out,
+				wt, w.derived_version[1] == w.version && w.dgrad_layout == layout);
 		w.derived_version[1] = w.version;
 		w.dgrad_layout = layout;
-		add_row_vector<T>(n, out_volume(), (const T*) params[1]->values.p, (T*) out);
+		if (!biased)
+			add_row_vector<T>(n, out_volume(), (const T*) params[1]->values.p, (T*) out);
 		x_cache = (const T*) in;       /* in_mat_cache (:147) */
 	}
 	void backward(const void* out_grad, size_t N, void* in_grad) override {
 		CATTLE_HIP_REQUIRE(x_cache != nullptr, "pass_back without a cached forward input");
 		const int n = checked_int(N, "batch size");
 		ConvShape s = conv;
-		const ConvWorkspace ws = weight_gradient_workspace<T>(s, n, partials);
 		Param& w = *params[0];
-		accumulate_column_sums<T>(n, out_volume(), (const T*) out_grad, (T*) params[1]->grad.p);      /* :184-185 */
-		/* in_mat^T * patches(out_grad) (:208) is the transpose of the convolution's weight gradient */
-		T* part = (T*) partials.ensure(ws.partials * sizeof(T));
-		T* gt = (T*) wgrad_t.ensure(w.bytes());
-		fill_zero(gt, w.bytes());
-		conv_weight_gradient<T>(s, n, (const T*) out_grad, x_cache, gt, (T*) nullptr, part);
-		transpose_matrix<T>((int) w.cols, (int) w.rows, gt, (T*) w.grad.p, true);
+		const ConvWorkspace ws = weight_gradient_workspace<T>(s, n, w.partials);
+		if (w.pending)
+			g_deferred.settle();
+		accumulate_column_sums<T>(n, out_volume(), (const T*) out_grad, (T*) params[1]->whole_grad());      /* :184-185 */
+		/* in_mat^T * patches(out_grad) (:208) is the transpose of the convolution's weight gradient: slices of it where the launch
+		 * writes them transposed, to be added like any layer's; else the whole of it, transposed */
+		T* part = (T*) w.partials.ensure(ws.partials * sizeof(T));
+		const bool fresh = w.clear_due;
+		ReduceBatch<T> later;
+		if (conv_weight_gradient_transposed<T>(s, n, (const T*) out_grad, x_cache, (T*) w.grad.p, part, &later, fresh)) {
+			g_deferred.add<T>(&w, later);
+		} else {
+			T* gt = (T*) wgrad_t.ensure(w.bytes());
+			conv_weight_gradient<T>(s, n, (const T*) out_grad, x_cache, gt, (T*) nullptr, part, nullptr, nullptr, true);
+			transpose_matrix<T>((int) w.cols, (int) w.rows, gt, (T*) w.grad.p, !fresh);
+		}
+		overwrote(w, w);
 		if (!in_grad)
 			return;
-		const T* wc = conv_weights();
 		T* wt = (T*) w.derived[0].ensure(ws.wt_fwd * sizeof(T));
-		conv_forward<T>(conv, n, (const T*) out_grad, wc, (const T*) nullptr, (T*) in_grad, wt, w.derived_version[0] == w.version);
+		conv_forward<T>(conv, n, (const T*) out_grad, (const T*) w.values.p, (const T*) nullptr, (T*) in_grad, wt, w.derived_version[0] == w.version);
 		w.derived_version[0] = w.version;
 	}
 	void empty_cache() override {

@@ -141,3 +141,34 @@ def test_transconv_rejects_bad_geometry():
     layer = ch.TransConvKernelLayer(np.float32, (4, 4, 2), 3)
     with pytest.raises(ch.CattleHipError):
         layer.pass_back(np.zeros((2, 4, 4, 3), np.float32, order="F"))          # pass_back before pass_forward
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N", [60, 64, 130])
+@pytest.mark.parametrize("case", [(10, 10, 3, 3, 4, 4, 0, 0, 1, 1, 0, 0), (13, 13, 3, 1, 4, 4, 0, 0, 2, 2, 0, 0), (9, 7, 5, 4, 3, 3, 1, 1, 1, 1, 0, 0),
+                                  (8, 8, 9, 7, 2, 2, 0, 0, 1, 1, 0, 0), (5, 6, 4, 12, 2, 2, 0, 0, 2, 2, 0, 0)])
+def test_transconv_into_few_filters(case, N, dtype):
+    """The layers of an image decoder: the bias, one value per output activation, is added by the launch of the few output columns,
+    and the weight gradient is left in slices, transposed as the weights are, for later; two passes, of which the second adds, a
+    reset that the next pass overwrites, and an optimizer step that takes the slices along."""
+    layer, (x, w, b, go), (_, _, dw_ref, db_ref) = _check(case, N, dtype)
+    wp, bp = layer.get_params()
+    once = wp.get_grad()
+    layer.pass_forward(x, True)
+    layer.pass_back(go)
+    tol = TOL[np.dtype(dtype)]
+    assert hp.rel_err(wp.get_grad(), 2 * dw_ref) < tol and hp.rel_err(bp.get_grad(), 2 * db_ref) < tol
+    for p in (wp, bp):
+        p.reset_grad()
+    layer.pass_forward(x, True)
+    layer.pass_back(go)
+    assert np.array_equal(wp.get_grad(), once)
+    wp.reset_grad()
+    layer.pass_back(go)
+    ch.ParameterList([wp]).optimizer_step("vanilla_sgd", (0.25,))
+    assert hp.rel_err(wp.get_values(), np.asarray(w, np.float64) - 0.25 * dw_ref) < tol
+    assert np.all(wp.get_grad() == 0)
+    # the prepared weights follow the new values
+    out = layer.pass_forward(x, False)
+    w64 = np.asarray(wp.get_values(), np.float64)
+    assert hp.rel_err(out, oracle.transconv_forward(np.asarray(x, np.float64), w64, np.asarray(b, np.float64), case[3], **_geom(case))) < tol
