@@ -1788,12 +1788,18 @@ void run_optimizer_many(const cattle_hip_layer_t* layers, const size_t* indices,
 		q.wt_fwd = q.wt_dgrad = nullptr;
 		q.K = q.RHW = 1;
 		q.ldw_fwd = q.ldw_dgrad = 0;
-		const ConvLayer<T>* conv = dynamic_cast<const ConvLayer<T>*>(as_layer(layers[i]));
+		/* the kernel that a weight matrix belongs to, whose prepared layouts follow the update (not the forward layout that the steps of
+		 * a recurrent network read, whose columns are in another order) */
+		const ConvShape* weights_of = nullptr;
+		if (const ConvLayer<T>* conv = dynamic_cast<const ConvLayer<T>*>(as_layer(layers[i])))
+			weights_of = indices[i] == 0 ? &conv->shape : nullptr;
+		else if (const ConvLstm<T>* lstm = dynamic_cast<const ConvLstm<T>*>(as_layer(layers[i])))
+			weights_of = indices[i] == 0 ? &lstm->sx : indices[i] == 2 ? &lstm->sh : nullptr;
 		bool fwd_current = false, dgrad_current = false;
 		if (p.constrains_values()) {
 			limited.push_back(&p);         /* constrained after the update; the prepared layouts are rebuilt from the result */
-		} else if (conv && indices[i] == 0) {
-			const ConvShape& cs = conv->shape;
+		} else if (weights_of) {
+			const ConvShape& cs = *weights_of;
 			fwd_current = p.derived[0].p && p.derived_version[0] == p.version;
 			dgrad_current = p.derived[1].p && p.derived_version[1] == p.version && p.dgrad_layout == 0;
 			q.K = cs.K();
