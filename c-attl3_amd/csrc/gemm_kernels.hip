@@ -22,6 +22,7 @@
 #include "lstm_steps.hpp"
 #include "small_dense.hpp"
 #include "few_weights.hpp"
+#include "few_channels.hpp"
 #include "gemm_tiles.hpp"
 #include "act_math.hpp"
 #include "lstm_math.hpp"
@@ -2461,6 +2462,14 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 						(void) split_workspace(0, fp32_bytes);
 				}
 			}
+		}
+	/* a handful of channels whose products stay on the fp32 instructions */
+	if constexpr (std::is_same<T, float>::value)
+		if (chosen == &vars[best_v] && !rider && epi == EPI_NONE && then == nullptr && !g.keeps_sums && !g.fp32_products && few_channels_possible(g)) {
+			few_channels_product(src, wt, bias, out, g);
+			if (mtiles_out)
+				*mtiles_out = 0;
+			return true;
 		}
 	const GatherVariant<T>& v = *chosen;
 	if (epi == EPI_LSTM) {
