@@ -248,20 +248,21 @@ void small_product_ordered_kernel(const float* __restrict__ src, const float* __
 
 /* ------------------------------------------------------------------------------------------------
  * wgrad[K x F] += x^T z, bgrad[F] += column sums of z, z = og or slope(y) * og. A block owns a 32 x 32 tile and each of its
- * wavefronts 64 samples: all its loads are issued at once, the operands change places through LDS (a lane of the instruction holds
- * a column, a line of memory 32 samples of one: 256 x 784 x 512 with the lanes reading their own columns 11.2 us, 8.6 this way),
+ * wavefronts 32 or 64 samples: all its loads are issued at once, the operands change places through LDS (a lane of the instruction holds
+ * a column, a line of memory 32 samples of one: 256 x 784 x 512 with the lanes reading their own columns 11.2 us, 7.7 this way),
  * and the wavefronts' sums meet in LDS and are added to the gradient in ascending order. No slices of M in memory: wgrad_kernel took
  * 9.3 us there and left four slices for the optimizer to add (11.6 us, 7.8 without them). A batch of up to eight wavefronts'
  * shares; with 32 columns or more, so that no tile is mostly padding (a layer of few outputs has a launch
  * that its input gradient takes along).
  * ---------------------------------------------------------------------------------------------- */
-constexpr int GL = 32, WAVE_M = 64, HALF_M = 32, GRAD_WAVES = 8, UNITS = HALF_M / 4;
+constexpr int GL = 32, HALF_M = 32, GRAD_WAVES = 8, UNITS = HALF_M / 4;
 /* Where 16-byte unit c (four samples) of row r of an operand's half share lies: shifted by the row, so that the eight rows that a
  * read of 64 lanes takes at a time lie on different banks. */
 __device__ __forceinline__ int unit_of(int r, int c) {
 	return r * UNITS + (c ^ (r % UNITS));
 }
-template<bool ACT>
+/* HALVES: 32 samples each that a wavefront takes */
+template<bool ACT, int HALVES>
 __global__ __launch_bounds__(64 * GRAD_WAVES)
 void small_weight_gradient_kernel(const float* __restrict__ x, const float* __restrict__ og, float* __restrict__ wgrad, float* __restrict__ bgrad,
 		int M, int K, int F, int ktiles, int tiles, unsigned x_bytes, unsigned og_bytes, const float* __restrict__ act_y, float* __restrict__ act_dz,
@@ -278,11 +279,11 @@ void small_weight_gradient_kernel(const float* __restrict__ x, const float* __re
 	const int lc = lane % GL, lk = lane / GL;
 	const __amdgpu_buffer_rsrc_t x_buf = buffer_of(x, x_bytes), og_buf = buffer_of(og, og_bytes), y_buf = buffer_of(ACT ? act_y : og, og_bytes);
 	/* loads: eight lanes read 32 samples of a column, whole lines */
-	const int row = lane / UNITS, unit = lane % UNITS, m0 = wave * WAVE_M + 4 * unit;
+	const int row = lane / UNITS, unit = lane % UNITS, m0 = wave * HALVES * HALF_M + 4 * unit;
 	const unsigned x_lane = 4u * (unsigned) (M * (k0 + row) + m0), g_lane = 4u * (unsigned) (M * (f0 + row) + m0), rows = 4u * ROWS * (unsigned) M;
-	f32x4 xv[2][LOADS], gv[2][LOADS], yv[ACT ? 2 : 1][LOADS];
+	f32x4 xv[HALVES][LOADS], gv[HALVES][LOADS], yv[ACT ? HALVES : 1][LOADS];
 	#pragma unroll
-	for (int h = 0; h < 2; ++h) {
+	for (int h = 0; h < HALVES; ++h) {
 		const bool in = m0 + h * HALF_M < M;            /* (columns past K or F lie beyond the buffers) */
 		const unsigned xo = in ? x_lane : OUTSIDE, go = in ? g_lane : OUTSIDE, half = 4u * HALF_M * (unsigned) h;
 		#pragma unroll
@@ -313,7 +314,7 @@ void small_weight_gradient_kernel(const float* __restrict__ x, const float* __re
 	f32x4* const xs = stage + wave * 2 * GL * UNITS;
 	f32x4* const zs = xs + GL * UNITS;
 	#pragma unroll
-	for (int h = 0; h < 2; ++h) {
+	for (int h = 0; h < HALVES; ++h) {
 		if constexpr (ACT) {
 			#pragma unroll
 			for (int q = 0; q < LOADS; ++q)
@@ -457,22 +458,30 @@ void small_product(const float* src, const float* wt, const float* bias, float* 
 }
 
 bool small_weight_gradient_possible(const GatherGeom& g, bool vec, const WgradAct<float>* act) {
-	return is_dense(g) && vec && (act == nullptr || act->pool_inds == nullptr) && g.M <= WAVE_M * GRAD_WAVES && g.F >= GL &&
+	return is_dense(g) && vec && (act == nullptr || act->pool_inds == nullptr) && g.M <= 2 * HALF_M * GRAD_WAVES && g.F >= GL &&
 			4.0 * g.M * std::max(g.K, g.F) < 1073741824.0;
 }
 
 void small_weight_gradient(const float* x, const float* og, float* wgrad, float* bgrad, const GatherGeom& g, const WgradAct<float>* act,
 		float p0, float p1, bool fresh) {
 	const int ktiles = up(g.K, GL), tiles = ktiles * up(g.F, GL);
-	const dim3 grid((unsigned) up(tiles, 8) * 8), block(64u * (unsigned) up(g.M, WAVE_M));
+	/* 32 samples a wavefront where eight wavefronts hold the batch and the tiles are few, else 64: 256 x 784 x 512 (400 tiles) 8.1 -> 7.7 us,
+	 * a pass of that MLP 427 -> 422; but the pass of one with 3072 tiles 403 -> 427, whose blocks fill the chip either way and have twice
+	 * as many partial tiles to add. */
+	const int halves = g.M <= HALF_M * GRAD_WAVES && tiles <= 512 ? 1 : 2;
+	const dim3 grid((unsigned) up(tiles, 8) * 8), block(64u * (unsigned) up(g.M, halves * HALF_M));
 	const unsigned x_bytes = 4u * (unsigned) g.M * (unsigned) g.K, og_bytes = 4u * (unsigned) g.M * (unsigned) g.F;
 	const size_t lds = (block.x / 64) * 2 * GL * GL * sizeof(float);
+	const auto launch = [&](auto undoes, auto h) {
+		small_weight_gradient_kernel<decltype(undoes)::value, decltype(h)::value><<<grid, block, lds, stream()>>>(x, og, wgrad, bgrad, g.M, g.K, g.F,
+				ktiles, tiles, x_bytes, og_bytes, act ? act->y : nullptr, act ? act->dz : nullptr, p0, p1, fresh);
+	};
+	typedef std::integral_constant<int, 1> one;
+	typedef std::integral_constant<int, 2> two;
 	if (act)
-		small_weight_gradient_kernel<true><<<grid, block, lds, stream()>>>(x, og, wgrad, bgrad, g.M, g.K, g.F, ktiles, tiles, x_bytes, og_bytes,
-				act->y, act->dz, p0, p1, fresh);
+		halves == 1 ? launch(std::true_type(), one()) : launch(std::true_type(), two());
 	else
-		small_weight_gradient_kernel<false><<<grid, block, lds, stream()>>>(x, og, wgrad, bgrad, g.M, g.K, g.F, ktiles, tiles, x_bytes, og_bytes,
-				(const float*) nullptr, (float*) nullptr, 0.f, 0.f, fresh);
+		halves == 1 ? launch(std::false_type(), one()) : launch(std::false_type(), two());
 	CATTLE_HIP_CHECK(hipGetLastError());
 }
 
