@@ -890,7 +890,14 @@ __device__ __forceinline__ void reduce_partials_block(const T* __restrict__ part
 	#pragma unroll
 	for (int e = 0; e < V; ++e)
 		s[e] = (T) 0;
-	if (i < count)
+	/* The old gradient is fetched before it is needed, and so are eight slices at a time where a thread adds several (one after the
+	 * other they are a chain of round trips to memory: 59 slices of 216 x 44 6.9 -> 4.8 us); the additions keep their order. With one
+	 * or two to a thread, as large gradients have them, the plain loop: the other made a pass of 6272 x 2304 -> 512 266 -> 270 us. */
+	const size_t o = (size_t) blk * 64 + threadIdx.x;
+	const bool writes = threadIdx.x < 64 && o < count;
+	const T old = writes && !fresh ? dst[o] : (T) 0;
+	constexpr int AHEAD = 8;
+	if (i < count && splits <= 2 * GR) {
 		for (int p = grp; p < splits; p += GR) {
 			T v[V];
 			vec_load<T, V>(v, partials + (size_t) p * count + i);
@@ -898,18 +905,32 @@ __device__ __forceinline__ void reduce_partials_block(const T* __restrict__ part
 			for (int e = 0; e < V; ++e)
 				s[e] += v[e];
 		}
+	} else if (i < count) {
+		for (int p0 = grp; p0 < splits; p0 += GR * AHEAD) {
+			T v[AHEAD][V];
+			#pragma unroll
+			for (int j = 0; j < AHEAD; ++j)
+				vec_load<T, V>(v[j], partials + (size_t) min(p0 + GR * j, splits - 1) * count + i);
+			#pragma unroll
+			for (int j = 0; j < AHEAD; ++j)
+				if (p0 + GR * j < splits) {
+					#pragma unroll
+					for (int e = 0; e < V; ++e)
+						s[e] += v[j][e];
+				}
+		}
+	}
 	#pragma unroll
 	for (int e = 0; e < V; ++e)
 		lds[grp][ox + e] = s[e];
 	__syncthreads();
-	const size_t o = (size_t) blk * 64 + threadIdx.x;
-	if (threadIdx.x < 64 && o < count) {
+	if (writes) {
 		T total = lds[0][threadIdx.x];
 		#pragma unroll
 		for (int j = 1; j < GR; ++j)
 			total += lds[j][threadIdx.x];
 		if (!fresh)
-			total = dst[o] + total;
+			total = old + total;
 		dst[o] = total;
 		if (copy != nullptr)
 			copy[o] = total;
