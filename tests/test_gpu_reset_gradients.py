@@ -114,6 +114,42 @@ def test_resets_and_recorded_passes():
     assert all(np.allclose(q.get_grad(), 2 * o, rtol=1e-5, atol=1e-5 * np.abs(o).max()) for q, o in zip(p, once))
 
 
+@pytest.mark.parametrize("kind", [DENSE, SLICES, WHOLE])
+def test_recorded_passes_with_the_optimizer_outside(kind):
+    """Marked before the recording, zeroed by the optimizer while the graph lives, marked again once it is destroyed: each step
+    starts from zero gradients, as the same steps without a recording do (sums of parts may be rounded in another order: 1e-5)."""
+    layer, p, x, g = _layer(kind, np.float32)
+    twin, tp, tx, tg = _layer(kind, np.float32)
+    params, tparams = ch.ParameterList(p), ch.ParameterList(tp)
+
+    def same():
+        for q, t in zip(p, tp):
+            v = t.get_values()
+            assert np.allclose(q.get_values(), v, rtol=1e-5, atol=1e-5 * np.abs(v).max())
+
+    def eager(n):
+        for _ in range(n):
+            _pass(layer, x, g)
+            params.optimizer_step("vanilla_sgd", [1e-3])
+    eager(2)
+    with ch.Graph() as graph:
+        _pass(layer, x, g)
+    for _ in range(3):
+        graph.launch()
+        params.optimizer_step("vanilla_sgd", [1e-3])
+    assert all(np.all(q.get_grad() == 0) for q in p)
+    eager(1)
+    graph.launch()
+    params.optimizer_step("vanilla_sgd", [1e-3])
+    graph.destroy()
+    eager(2)
+    assert all(np.all(q.get_grad() == 0) for q in p)
+    for _ in range(9):
+        _pass(twin, tx, tg)
+        tparams.optimizer_step("vanilla_sgd", [1e-3])
+    same()
+
+
 def test_a_recurrent_network():
     net = ch.ConvLSTMNetwork(np.float32, (4, 4, 2), 8)
     gen = hp.rng(9)
