@@ -190,6 +190,12 @@ template<typename T> bool conv_weight_gradient_transposed(const ConvShape& s, in
 /* Which prepared layout conv_input_gradient builds in wt_dgrad at this batch size: 0 the plain one (all taps), 1 the
  * blocks of a strided convolution's residue classes. Prepared weights are current only for the layout they were built as. */
 template<typename T> int dgrad_weight_layout(const ConvShape& s, int N);
+/* The layouts of a kernel's weights that its passes keep between calls, and the orders (`kind`) that a slot may be in: the forward
+ * product's (0), the input gradient's (dgrad_weight_layout) and that of a recurrent step with its gates in blocks (the block).
+ * prepare_weights makes one of them in wt, which has the elements that conv_workspace gives for it, as the passes make it themselves
+ * when they are told that it is not ready. */
+enum { PREPARED_FORWARD = 0, PREPARED_DGRAD = 1, PREPARED_GATES = 2, PREPARED_SLOTS = 3 };
+template<typename T> void prepare_weights(const ConvShape& s, int slot, int kind, const T* w, T* wt);
 
 /* Element-wise / reduction kernels (pointwise_kernels.hip). */
 template<typename T> void act_forward(int kind, size_t n, T p, const T* x, T* y);

@@ -3113,18 +3113,61 @@ ConvWorkspace conv_workspace(const ConvShape& s, int N) {
 	return ws;
 }
 
+namespace {
+
+/* the launches that make the prepared layouts */
+template<typename T>
+void prepare_forward_weights(const ConvShape& s, const T* w, T* wt, int gate_block = 0) {
+	const int Kp = round_up(s.K(), WT_ROW_PAD), ldw = round_up(s.F, WT_COL_PAD);
+	const size_t count = (size_t) Kp * ldw;
+	prep_fwd_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, s.K(), s.F, Kp, ldw, gate_block, s.weights_transposed);
+	CATTLE_HIP_CHECK(hipGetLastError());
+}
+template<typename T>
+void prepare_dgrad_weights(const ConvShape& s, const T* w, T* wt) {
+	const int Kp = round_up(s.RH * s.RW * s.F, WT_ROW_PAD), ldw = round_up(s.C, WT_COL_PAD);
+	const size_t count = (size_t) Kp * ldw;
+	prep_dgrad_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, s.RH * s.RW, s.C, s.F, Kp, ldw, s.weights_transposed);
+	CATTLE_HIP_CHECK(hipGetLastError());
+}
+/* (nothing for a class without positions or taps, which has no launch) */
+template<typename T>
+void prepare_class_weights(const ConvShape& s, const StridedClass& c, const T* w, T* wt) {
+	if (c.OAc * c.OBc == 0 || c.Rc * c.Sc == 0)
+		return;
+	const int Kp = round_up(c.Rc * c.Sc * s.F, WT_ROW_PAD), ldw = round_up(s.C, WT_COL_PAD);
+	const size_t count = (size_t) Kp * ldw;
+	prep_dgrad_class_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt + c.wt_offset, s.RH, s.RW, s.C, s.F,
+			c.r0, s.sv, c.Rc, c.s0, s.sh, c.Sc, Kp, ldw, s.weights_transposed);
+	CATTLE_HIP_CHECK(hipGetLastError());
+}
+
+} /* namespace */
+
+template<typename T>
+void prepare_weights(const ConvShape& s, int slot, int kind, const T* w, T* wt) {
+	if (slot == PREPARED_FORWARD) {
+		prepare_forward_weights<T>(s, w, wt);
+	} else if (slot == PREPARED_GATES) {
+		prepare_forward_weights<T>(s, w, wt, kind);
+	} else if (kind == 0) {
+		prepare_dgrad_weights<T>(s, w, wt);
+	} else {
+		std::vector<StridedClass> classes;
+		strided_classes(s, &classes, nullptr);
+		for (const StridedClass& c : classes)
+			prepare_class_weights<T>(s, c, w, wt);
+	}
+}
+
 template<typename T>
 void conv_forward(const ConvShape& s, int N, const T* x, const T* w, const T* b, T* out, T* wt, bool wt_ready, int x_batch) {
 	check_sizes(s, std::max(N, x_batch));
 	GatherProblem g = forward_geom(s, N);
 	if (x_batch > 0)
 		g.NS = x_batch;
-	if (!wt_ready) {
-		const int Kp = round_up(g.K, WT_ROW_PAD);
-		const size_t count = (size_t) Kp * g.ldw;
-		prep_fwd_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, g.K, g.F, Kp, g.ldw, 0, s.weights_transposed);
-		CATTLE_HIP_CHECK(hipGetLastError());
-	}
+	if (!wt_ready)
+		prepare_forward_weights<T>(s, w, wt);
 	launch_gather<T>(x, wt, b, out, g);
 }
 
@@ -3140,10 +3183,7 @@ bool conv_forward_lstm(const ConvShape& s, int N, const T* x, int x_batch, const
 	const std::function<void(int)> prepare = [&](int bf) {
 		if (*gate_block == bf / 4)
 			return;
-		const int Kp = round_up(g.K, WT_ROW_PAD);
-		const size_t count = (size_t) Kp * g.ldw;
-		prep_fwd_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, g.K, g.F, Kp, g.ldw, bf / 4);
-		CATTLE_HIP_CHECK(hipGetLastError());
+		prepare_forward_weights<T>(s, w, wt, bf / 4);
 		*gate_block = bf / 4;
 	};
 	if constexpr (std::is_same<T, float>::value)
@@ -3167,12 +3207,8 @@ bool conv_forward_fused(const ConvShape& s, int N, const T* x, const T* w, const
 	if (epi == EPI_STATS)
 		CATTLE_HIP_REQUIRE(E.stats != nullptr, "the moments epilogue needs a buffer for its partials");
 	/* the prepared weights come first: they are valid afterwards whatever the answer is */
-	if (!wt_ready) {
-		const int Kp = round_up(g.K, WT_ROW_PAD);
-		const size_t count = (size_t) Kp * g.ldw;
-		prep_fwd_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, g.K, g.F, Kp, g.ldw);
-		CATTLE_HIP_CHECK(hipGetLastError());
-	}
+	if (!wt_ready)
+		prepare_forward_weights<T>(s, w, wt);
 	/* the staging pass deals threads over windows of at most a tile's positions */
 	if (epi == EPI_POOL && E.prh * E.prw > 64)
 		return false;
@@ -3213,8 +3249,7 @@ void conv_forward_static(const ConvShape& s, int N, const T* x, const T* w, cons
 	const int Kp = round_up(g.K, WT_ROW_PAD);
 	const size_t count = (size_t) Kp * g.ldw;
 	T* wt = static_cast<T*>(arena.take(count * sizeof(T), "prepared weights"));
-	prep_fwd_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt, g.K, g.F, Kp, g.ldw);
-	CATTLE_HIP_CHECK(hipGetLastError());
+	prepare_forward_weights<T>(s, w, wt);
 	launch_gather<T>(x, wt, b, out, g, &arena);
 }
 
@@ -3429,13 +3464,9 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 			if (c.OAc * c.OBc == 0 || c.Rc * c.Sc == 0)
 				continue;
 			T* wtc = wt_dgrad + c.wt_offset;
-			const int Kc = c.Rc * c.Sc * s.F, Kp = round_up(Kc, WT_ROW_PAD);
-			if (!wt_ready) {
-				const size_t count = (size_t) Kp * ldw;
-				prep_dgrad_class_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wtc, s.RH, s.RW, s.C, s.F,
-						c.r0, s.sv, c.Rc, c.s0, s.sh, c.Sc, Kp, ldw, s.weights_transposed);
-				CATTLE_HIP_CHECK(hipGetLastError());
-			}
+			const int Kc = c.Rc * c.Sc * s.F;
+			if (!wt_ready)
+				prepare_class_weights<T>(s, c, w, wt_dgrad);
 			GatherProblem g;
 			g.N = N; g.NS = og_batch > 0 ? og_batch : N; g.LH = s.OH(); g.LW = s.OW(); g.LC = s.F;
 			g.OA = c.OAc; g.OB = c.OBc;
@@ -3472,13 +3503,8 @@ bool conv_input_gradient_with(const ConvShape& s, int N, const T* w, const T* ou
 	GatherProblem d = dgrad_geom(s, N);
 	if (og_batch > 0)
 		d.NS = og_batch;
-	if (!wt_ready) {
-		const int Kp = round_up(d.K, WT_ROW_PAD);
-		const size_t count = (size_t) Kp * d.ldw;
-		prep_dgrad_weights_kernel<T><<<(unsigned) ((count + 255) / 256), 256, 0, stream()>>>(w, wt_dgrad, s.RH * s.RW, s.C, s.F,
-				Kp, d.ldw, s.weights_transposed);
-		CATTLE_HIP_CHECK(hipGetLastError());
-	}
+	if (!wt_ready)
+		prepare_dgrad_weights<T>(s, w, wt_dgrad);
 	if constexpr (std::is_same<T, float>::value)
 		if (then != nullptr && lstm_step_backward_possible(d, *then, device_shape().cus)) {
 			lstm_step_backward(out_grad, wt_dgrad, d, *then);
@@ -3506,6 +3532,8 @@ void conv_backward(const ConvShape& s, int N, const T* x, const T* w, const T* o
 		conv_input_gradient<T>(s, N, w, act ? (const T*) act->dz : out_grad, in_grad, wt_dgrad, wt_ready, nullptr, 0);
 }
 
+template void prepare_weights<float>(const ConvShape&, int, int, const float*, float*);
+template void prepare_weights<double>(const ConvShape&, int, int, const double*, double*);
 template ConvWorkspace conv_workspace<float>(const ConvShape&, int);
 template ConvWorkspace conv_workspace<double>(const ConvShape&, int);
 template void conv_forward<float>(const ConvShape&, int, const float*, const float*, const float*, float*, float*, bool, int);

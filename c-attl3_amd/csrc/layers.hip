@@ -252,17 +252,29 @@ struct DevicePool {
 DevicePool g_pool;
 
 /* Device twin of a Parameters object (core/Parameters.hpp:15-95): values plus accumulated gradient.
- * `derived` holds kernel-friendly re-layouts of the values, rebuilt when `version` moves on. */
-struct Param {
+ * `prepared` holds kernel-friendly re-layouts of a kernel's weights (PreparedSlot), rebuilt when `version` has moved on or when
+ * another order of the same slot is wanted. What a recording does with them takes effect at its launches: see Recording. */
+struct Param : std::enable_shared_from_this<Param> {
 	size_t rows, cols;
 	bool optimizable;
 	size_t esize;
 	DevBuf values, grad;
 	uint64_t version = 1;
-	DevBuf derived[3];
-	uint64_t derived_version[3] = { 0, 0, 0 };
-	int dgrad_layout = 0;              /* which layout derived[1] holds (dgrad_weight_layout) */
-	int gate_block = 0;                /* and derived[2] of a recurrent kernel (conv_forward_lstm) */
+	struct Prepared {
+		DevBuf buf;
+		uint64_t version = 0;          /* of the values it was made from */
+		int kind = 0;                  /* the order it is in (prepare_weights) */
+	};
+	Prepared prepared[PREPARED_SLOTS];
+	ConvShape kernel = {};             /* the problem whose weights these are, where they have prepared layouts */
+	bool holds(int slot, int kind) const {
+		return prepared[slot].version == version && prepared[slot].kind == kind;
+	}
+	/* Whether the layout can be read as it lies. A caller that is told so reads it, one that is not builds it and says built(). */
+	bool ready(int slot, int kind);
+	void built(int slot, int kind);
+	/* after every write to the values */
+	void values_changed();
 	/* A weight matrix: the partial sums of the last weight-gradient launch that was cut into slices (its own and, behind
 	 * them, those of the bias gradient). They are added to the gradients when a gradient is first needed - by the
 	 * optimizer step as a rule, in one launch for all layers - and until then `pending` lists them (see Deferred). */
@@ -310,6 +322,7 @@ struct Param {
 		copy_in(c->values.p, values.p, CATTLE_HIP_DEVICE, bytes());
 		copy_in(c->grad.p, const_cast<Param*>(this)->whole_grad(), CATTLE_HIP_DEVICE, bytes());
 		c->overwritten = overwritten;
+		c->kernel = kernel;
 		c->reg_l1 = reg_l1;
 		c->reg_l2 = reg_l2;
 		std::memcpy(c->value_limits, value_limits, sizeof(value_limits));
@@ -319,6 +332,111 @@ struct Param {
 };
 
 typedef std::shared_ptr<Param> ParamPtr;
+
+/* What the recording of a graph does to the values and the prepared layouts of the parameters that it touches. While it is made the
+ * parameters are kept as if its calls ran, so that a pass that needs a layout twice records its making once; at its end they are put
+ * back, since nothing has run. A launch makes the layouts that the recorded passes read as they found them (`needs`) where the values
+ * have changed, or the slot has been taken for another order, since they were last made, and afterwards notes what the recorded
+ * calls have left: recorded and eager passes may follow each other in any order, whoever changes the values in between. */
+struct Recording {
+	struct Entry {
+		ParamPtr param;
+		uint64_t version_before = 0;
+		struct Slot {
+			uint64_t version_before = 0;
+			int kind_before = 0;
+			int needs = -1;                /* kind that a launch has to find, -1 none */
+			bool made = false;             /* by the recorded calls */
+			bool current_after = false;    /* of the values as a launch leaves them, */
+			int kind_after = 0;            /* in this order */
+		} slots[PREPARED_SLOTS];
+		bool changes_values = false;
+	};
+	std::map<Param*, Entry> entries;
+
+	Entry& touch(Param& p) {
+		std::map<Param*, Entry>::iterator it = entries.find(&p);
+		if (it != entries.end())
+			return it->second;
+		Entry& e = entries[&p];
+		e.param = p.shared_from_this();
+		e.version_before = p.version;
+		for (int i = 0; i < PREPARED_SLOTS; ++i) {
+			e.slots[i].version_before = p.prepared[i].version;
+			e.slots[i].kind_before = p.prepared[i].kind;
+		}
+		return e;
+	}
+	void read(Param& p, int slot) {
+		Entry::Slot& s = touch(p).slots[slot];
+		if (!s.made && s.needs < 0)
+			s.needs = p.prepared[slot].kind;
+	}
+	/* the end of the recording */
+	void put_back() {
+		for (std::pair<Param* const, Entry>& pe : entries) {
+			Param& p = *pe.first;
+			Entry& e = pe.second;
+			e.changes_values = p.version != e.version_before;
+			for (int i = 0; i < PREPARED_SLOTS; ++i) {
+				Entry::Slot& s = e.slots[i];
+				s.current_after = p.prepared[i].version == p.version;
+				s.kind_after = p.prepared[i].kind;
+				p.prepared[i].version = s.version_before;
+				p.prepared[i].kind = s.kind_before;
+			}
+			p.version = e.version_before;
+		}
+	}
+	void before_launch() {
+		for (std::pair<Param* const, Entry>& pe : entries)
+			for (int i = 0; i < PREPARED_SLOTS; ++i) {
+				const int kind = pe.second.slots[i].needs;
+				Param& p = *pe.first;
+				if (kind < 0 || p.holds(i, kind))
+					continue;
+				if (p.esize == sizeof(float))
+					prepare_weights<float>(p.kernel, i, kind, static_cast<const float*>(p.values.p), static_cast<float*>(p.prepared[i].buf.p));
+				else
+					prepare_weights<double>(p.kernel, i, kind, static_cast<const double*>(p.values.p), static_cast<double*>(p.prepared[i].buf.p));
+				p.built(i, kind);
+			}
+	}
+	void after_launch() {
+		for (std::pair<Param* const, Entry>& pe : entries) {
+			Param& p = *pe.first;
+			if (pe.second.changes_values)
+				++p.version;
+			for (int i = 0; i < PREPARED_SLOTS; ++i) {
+				const Entry::Slot& s = pe.second.slots[i];
+				if (s.needs < 0 && !s.made)
+					continue;
+				p.prepared[i].version = s.current_after ? p.version : 0;
+				p.prepared[i].kind = s.kind_after;
+			}
+		}
+	}
+};
+Recording g_recording;                  /* of the graph that is being recorded */
+
+bool Param::ready(int slot, int kind) {
+	if (!holds(slot, kind))
+		return false;
+	if (capturing())
+		g_recording.read(*this, slot);
+	return true;
+}
+void Param::built(int slot, int kind) {
+	if (capturing())
+		g_recording.touch(*this).slots[slot].made = true;
+	prepared[slot].version = version;
+	prepared[slot].kind = kind;
+}
+void Param::values_changed() {
+	if (capturing())
+		g_recording.touch(*this);
+	++version;
+}
 
 /* Sums of weight-gradient slices that have not been added to their gradients yet. Nothing reads a gradient between the
  * backward pass of its layer and the optimizer step (FeedforwardNeuralNetwork.hpp:129-141 runs the layers back to front,
@@ -471,7 +589,7 @@ template<typename T>
 void fill_constant(Param& p, T v) {
 	std::vector<T> host(p.rows * p.cols, v);
 	copy_in(p.values.p, host.data(), CATTLE_HIP_HOST, p.bytes());
-	++p.version;
+	p.values_changed();
 }
 
 /* enforce_clip_constraint, enforce_l1_norm_constraint, enforce_l2_norm_constraint on the values (set_values,
@@ -567,6 +685,7 @@ struct ConvLayer : LayerBase {
 		}
 		params.push_back(std::make_shared<Param>((size_t) s.K(), (size_t) s.F, true, sizeof(T)));
 		params.push_back(std::make_shared<Param>(1, (size_t) s.F, true, sizeof(T)));
+		params[0]->kernel = s;
 		params[0]->overwritten = params[1]->overwritten = true;
 	}
 	ConvLayer(const ConvLayer& o, bool share) : LayerBase(o.dtype), shape(o.shape) {
@@ -586,10 +705,11 @@ struct ConvLayer : LayerBase {
 		const int n = checked_int(N, "batch size");
 		const ConvWorkspace ws = conv_workspace<T>(s, n);
 		Param& w = *params[0];
-		T* wt = (T*) w.derived[0].ensure(ws.wt_fwd * sizeof(T));
-		const bool ready = w.derived_version[0] == w.version;
+		T* wt = (T*) w.prepared[PREPARED_FORWARD].buf.ensure(ws.wt_fwd * sizeof(T));
+		const bool ready = w.ready(PREPARED_FORWARD, 0);
 		conv_forward<T>(s, n, (const T*) in, (const T*) w.values.p, (const T*) params[1]->values.p, (T*) out, wt, ready);
-		w.derived_version[0] = w.version;
+		if (!ready)
+			w.built(PREPARED_FORWARD, 0);
 		x_cache = (const T*) in;       /* the reference caches the patch matrix (ConvKernelLayer.hpp:127); the input suffices */
 	}
 	/* `act`: out_grad is the gradient behind an element-wise activation whose derivative the weight-gradient launch
@@ -599,9 +719,9 @@ struct ConvLayer : LayerBase {
 		const int n = checked_int(N, "batch size");
 		Param& w = *params[0];
 		const ConvWorkspace ws = weight_gradient_workspace<T>(s, n, w.partials);
-		T* wt = (T*) w.derived[1].ensure(ws.wt_dgrad * sizeof(T));
+		T* wt = (T*) w.prepared[PREPARED_DGRAD].buf.ensure(ws.wt_dgrad * sizeof(T));
 		const int layout = dgrad_weight_layout<T>(s, n);
-		const bool ready = w.derived_version[1] == w.version && w.dgrad_layout == layout;
+		const bool ready = in_grad && w.ready(PREPARED_DGRAD, layout);
 		/* the partial sums of the launch before, if they still wait, would be overwritten */
 		if (w.pending)
 			g_deferred.settle();
@@ -613,10 +733,8 @@ struct ConvLayer : LayerBase {
 		if (fresh)
 			overwrote(w, *params[1]);
 		g_deferred.add<T>(&w, later);
-		if (in_grad) {
-			w.derived_version[1] = w.version;
-			w.dgrad_layout = layout;
-		}
+		if (in_grad && !ready)
+			w.built(PREPARED_DGRAD, layout);
 	}
 	void empty_cache() override {
 		LayerBase::empty_cache();
@@ -646,6 +764,7 @@ struct TransConvLayer : LayerBase {
 		out_dims[0] = (size_t) c.H; out_dims[1] = (size_t) c.W; out_dims[2] = (size_t) c.C;
 		params.push_back(std::make_shared<Param>((size_t) c.F, (size_t) c.K(), true, sizeof(T)));
 		params.push_back(std::make_shared<Param>(1, out_volume(), true, sizeof(T)));
+		params[0]->kernel = conv;
 		params[0]->overwritten = true;
 	}
 	TransConvLayer(const TransConvLayer& o, bool share) : LayerBase(o.dtype), conv(o.conv) {
@@ -658,12 +777,13 @@ struct TransConvLayer : LayerBase {
 		const int n = checked_int(N, "batch size");
 		const ConvWorkspace ws = conv_workspace<T>(conv, n);
 		Param& w = *params[0];
-		T* wt = (T*) w.derived[1].ensure(ws.wt_dgrad * sizeof(T));
+		T* wt = (T*) w.prepared[PREPARED_DGRAD].buf.ensure(ws.wt_dgrad * sizeof(T));
 		const int layout = dgrad_weight_layout<T>(conv, n);
+		const bool ready = w.ready(PREPARED_DGRAD, layout);
 		const bool biased = conv_input_gradient_biased<T>(conv, n, (const T*) w.values.p, (const T*) in, (const T*) params[1]->values.p, (T*) out,
-				wt, w.derived_version[1] == w.version && w.dgrad_layout == layout);
-		w.derived_version[1] = w.version;
-		w.dgrad_layout = layout;
+				wt, ready);
+		if (!ready)
+			w.built(PREPARED_DGRAD, layout);
 		if (!biased)
 			add_row_vector<T>(n, out_volume(), (const T*) params[1]->values.p, (T*) out);
 		x_cache = (const T*) in;       /* in_mat_cache (:147) */
@@ -692,9 +812,11 @@ struct TransConvLayer : LayerBase {
 		overwrote(w, w);
 		if (!in_grad)
 			return;
-		T* wt = (T*) w.derived[0].ensure(ws.wt_fwd * sizeof(T));
-		conv_forward<T>(conv, n, (const T*) out_grad, (const T*) w.values.p, (const T*) nullptr, (T*) in_grad, wt, w.derived_version[0] == w.version);
-		w.derived_version[0] = w.version;
+		T* wt = (T*) w.prepared[PREPARED_FORWARD].buf.ensure(ws.wt_fwd * sizeof(T));
+		const bool ready = w.ready(PREPARED_FORWARD, 0);
+		conv_forward<T>(conv, n, (const T*) out_grad, (const T*) w.values.p, (const T*) nullptr, (T*) in_grad, wt, ready);
+		if (!ready)
+			w.built(PREPARED_FORWARD, 0);
 	}
 	void empty_cache() override {
 		LayerBase::empty_cache();
@@ -744,6 +866,8 @@ struct ConvLstm : LayerBase {
 		params.push_back(std::make_shared<Param>(1, (size_t) sx.F, true, sizeof(T)));
 		params.push_back(std::make_shared<Param>((size_t) sh.K(), (size_t) sh.F, true, sizeof(T)));
 		params.push_back(std::make_shared<Param>(1, (size_t) sh.F, true, sizeof(T)));
+		params[0]->kernel = sx;
+		params[2]->kernel = sh;
 		for (const ParamPtr& p : params)
 			p->overwritten = true;
 	}
@@ -785,10 +909,12 @@ struct ConvLstm : LayerBase {
 		Param& wh = *params[2];
 		{
 			const ConvWorkspace ws = conv_workspace<T>(sx, (int) (N * in_len));
-			T* wt = (T*) wx.derived[0].ensure(ws.wt_fwd * e);
+			T* wt = (T*) wx.prepared[PREPARED_FORWARD].buf.ensure(ws.wt_fwd * e);
+			const bool ready = wx.ready(PREPARED_FORWARD, 0);
 			conv_forward<T>(sx, (int) (N * in_len), input, (const T*) wx.values.p, (const T*) params[1]->values.p,
-					(T*) zx_all.ensure(4 * p * in_len * e), wt, wx.derived_version[0] == wx.version);
-			wx.derived_version[0] = wx.version;
+					(T*) zx_all.ensure(4 * p * in_len * e), wt, ready);
+			if (!ready)
+				wx.built(PREPARED_FORWARD, 0);
 		}
 		CATTLE_HIP_REQUIRE((double) (4 * p) * (double) std::max(total, in_len) <= 2147483647.0, "sequence tensor exceeds 2^31-1 elements");
 		if (keeps_z())
@@ -802,7 +928,7 @@ struct ConvLstm : LayerBase {
 		 * output); every slab is written once per pass. The last step's hidden output goes to `out` only. */
 		hprev_all.ensure(p * total * e);
 		const ConvWorkspace wsh = conv_workspace<T>(sh, n);
-		T* wth = (T*) wh.derived[0].ensure(wsh.wt_fwd * e);
+		T* wth = (T*) wh.prepared[PREPARED_FORWARD].buf.ensure(wsh.wt_fwd * e);
 		bool fused_steps = fuse_steps;
 		fused_forward_steps = 0;
 		T* wth_gates = nullptr;             /* the prepared layout of the kernel that runs the step itself */
@@ -820,12 +946,16 @@ struct ConvLstm : LayerBase {
 				 * the weighted previous output then exists only inside that kernel (with multiplicative integration
 				 * the backward pass reads it, so it has to be stored) */
 				if (!wth_gates)
-					wth_gates = (T*) wh.derived[2].ensure(wsh.wt_fwd * e);
-				int block = wh.derived_version[2] == wh.version ? wh.gate_block : 0;
+					wth_gates = (T*) wh.prepared[PREPARED_GATES].buf.ensure(wsh.wt_fwd * e);
+				int block = wh.prepared[PREPARED_GATES].kind;
+				if (!wh.holds(PREPARED_GATES, block))
+					block = 0;
+				const int held = block;
 				if (conv_forward_lstm<T>(sh, n, hprev, (int) (N * total), (const T*) wh.values.p, (const T*) params[3]->values.p,
 						wth_gates, &block, fs)) {
-					wh.gate_block = block;
-					wh.derived_version[2] = wh.version;
+					/* (the launcher chooses the block; it has read the layout as it lay if it is still the same) */
+					if (block != held || !wh.ready(PREPARED_GATES, block))
+						wh.built(PREPARED_GATES, block);
 					++fused_forward_steps;
 					continue;
 				}
@@ -833,9 +963,10 @@ struct ConvLstm : LayerBase {
 			}
 			T* zh_t = step(zh, mul_int ? t : 0, 4 * p);
 			if (has_prev) {
-				conv_forward<T>(sh, n, hprev, (const T*) wh.values.p, (const T*) params[3]->values.p, zh_t,
-						wth, wh.derived_version[0] == wh.version, (int) (N * total));
-				wh.derived_version[0] = wh.version;
+				const bool ready = wh.ready(PREPARED_FORWARD, 0);
+				conv_forward<T>(sh, n, hprev, (const T*) wh.values.p, (const T*) params[3]->values.p, zh_t, wth, ready, (int) (N * total));
+				if (!ready)
+					wh.built(PREPARED_FORWARD, 0);
 			}
 			lstm_gates_forward<T>(fs, has_prev ? (const T*) zh_t : nullptr);
 		}
@@ -855,7 +986,7 @@ struct ConvLstm : LayerBase {
 		dzx_all.ensure(4 * p * T_in * e);
 		dzh_all.ensure(4 * p * total * e);                               /* every slab is written; step 0 writes zeros */
 		const ConvWorkspace wsh = conv_workspace<T>(sh, n);
-		T* wtd = (T*) wh.derived[1].ensure(wsh.wt_dgrad * e);
+		T* wtd = (T*) wh.prepared[PREPARED_DGRAD].buf.ensure(wsh.wt_dgrad * e);
 		auto backward_step = [&](size_t t) {
 			const bool has_in = t < T_in, has_prev = t > 0;
 			const bool emitted = t >= delay && t < delay + T_out;
@@ -876,9 +1007,11 @@ struct ConvLstm : LayerBase {
 			 * parts of that launch's reductions when the launch has such a kernel */
 			const bool no_fusion = !fuse_steps;
 			const LstmBackwardStep<T> before = backward_step(t - 1);
-			const bool done = conv_input_gradient<T>(sh, n, (const T*) wh.values.p, (const T*) dzh_all.p + N * t, (T*) dh.p, wtd,
-					wh.derived_version[1] == wh.version, no_fusion ? nullptr : &before, (int) (N * total));
-			wh.derived_version[1] = wh.version;
+			const bool ready = wh.ready(PREPARED_DGRAD, 0);
+			const bool done = conv_input_gradient<T>(sh, n, (const T*) wh.values.p, (const T*) dzh_all.p + N * t, (T*) dh.p, wtd, ready,
+					no_fusion ? nullptr : &before, (int) (N * total));
+			if (!ready)
+				wh.built(PREPARED_DGRAD, 0);
 			if (done)
 				++fused_backward_steps;
 			else
@@ -909,10 +1042,11 @@ struct ConvLstm : LayerBase {
 				overwrote(wx, *params[1]);
 			g_deferred.add<T>(&wx, later);
 			if (in_grad) {
-				T* wt = (T*) wx.derived[1].ensure(ws.wt_dgrad * e);
-				conv_input_gradient<T>(sx, (int) (N * T_in), (const T*) wx.values.p, (const T*) dzx_all.p, in_grad, wt,
-						wx.derived_version[1] == wx.version);
-				wx.derived_version[1] = wx.version;
+				T* wt = (T*) wx.prepared[PREPARED_DGRAD].buf.ensure(ws.wt_dgrad * e);
+				const bool ready = wx.ready(PREPARED_DGRAD, 0);
+				conv_input_gradient<T>(sx, (int) (N * T_in), (const T*) wx.values.p, (const T*) dzx_all.p, in_grad, wt, ready);
+				if (!ready)
+					wx.built(PREPARED_DGRAD, 0);
 			}
 		}
 	}
@@ -973,8 +1107,8 @@ struct BatchNormLayer : LayerBase {
 			stats_init = true;
 			cache_valid = true;
 			cache_batch = N;
-			++params[0]->version;
-			++params[1]->version;
+			params[0]->values_changed();
+			params[1]->values_changed();
 		}
 	}
 	void backward(const void* out_grad, size_t N, void* in_grad) override {
@@ -1229,12 +1363,14 @@ struct FusedLayer : LayerBase {
 	T* prepared_weights(int n, bool& ready) {
 		const ConvWorkspace ws = conv_workspace<T>(shape(), n);
 		Param& w = *conv->params[0];
-		ready = w.derived_version[0] == w.version;
-		return (T*) w.derived[0].ensure(ws.wt_fwd * sizeof(T));
+		ready = w.ready(PREPARED_FORWARD, 0);
+		return (T*) w.prepared[PREPARED_FORWARD].buf.ensure(ws.wt_fwd * sizeof(T));
 	}
-	void weights_prepared() {
-		Param& w = *conv->params[0];
-		w.derived_version[0] = w.version;
+	/* after a launch that builds them unless it was told that they are ready */
+	void weights_prepared(bool& ready) {
+		if (!ready)
+			conv->params[0]->built(PREPARED_FORWARD, 0);
+		ready = true;
 	}
 
 	void forward(const void* in, size_t N, bool training, void* out) override {
@@ -1264,7 +1400,7 @@ struct FusedLayer : LayerBase {
 			if (training) {
 				E.stats = (T*) stats_buf.ensure(conv_stats_rows(conv->shape, n) * F() * 3 * sizeof(T));
 				ok = conv_forward_fused<T>(shape(training), n, x, wv, bv, z, wt, ready, EPI_STATS, E, &mtiles);
-				weights_prepared();
+				weights_prepared(ready);
 			}
 			if (!ok) {
 				forward_unfused(in, N, training, out);
@@ -1272,7 +1408,7 @@ struct FusedLayer : LayerBase {
 			}
 			if (!training) {
 				conv_forward<T>(shape(training), n, x, wv, bv, z, wt, ready);
-				weights_prepared();
+				weights_prepared(ready);
 			}
 			pool_in_chain = pool_tiles();
 			const ChainShape cs = chain_shape(pool_in_chain);
@@ -1292,8 +1428,8 @@ struct FusedLayer : LayerBase {
 			if (training) {
 				bn->stats_init = true;
 				bn->cache_valid = false;        /* the member's own backward pass has nothing to work from */
-				++bn->params[0]->version;
-				++bn->params[1]->version;
+				bn->params[0]->values_changed();
+				bn->params[1]->values_changed();
 			}
 			if (pool && !pool_in_chain)
 				pool->forward(dst, N, training, out);
@@ -1321,8 +1457,7 @@ struct FusedLayer : LayerBase {
 				E.pre = needs_pre ? (T*) pre_buf.ensure(pcount * sizeof(T)) : nullptr;
 			}
 			const bool ok = conv_forward_fused<T>(shape(training), n, x, wv, bv, (T*) out, wt, ready, EPI_POOL, E, nullptr);
-			weights_prepared();
-			ready = true;
+			weights_prepared(ready);
 			if (ok) {
 				if (!mean)
 					pool->inds_count = pcount;
@@ -1343,7 +1478,7 @@ struct FusedLayer : LayerBase {
 			T* y = pool ? (T*) z_buf.ensure(zcount * sizeof(T)) : (T*) out;
 			E.pre = needs_pre ? (T*) pre_buf.ensure(zcount * sizeof(T)) : nullptr;
 			const bool ok = conv_forward_fused<T>(shape(training), n, x, wv, bv, y, wt, ready, EPI_ACT, E, nullptr);
-			weights_prepared();
+			weights_prepared(ready);
 			if (ok) {
 				if (pool)
 					pool->forward(y, N, training, out);
@@ -1592,6 +1727,7 @@ struct Graph {
 	hipGraph_t graph = nullptr;
 	hipGraphExec_t exec = nullptr;
 	std::vector<void*> blocks;
+	Recording uses;                    /* (it keeps the parameters that it lists) */
 	uint64_t recorded_at = 0;          /* on the allocation clock: older allocations are pinned while the graph lives */
 };
 
@@ -1725,7 +1861,7 @@ void run_optimizer(cattle_hip_layer_t layer, size_t index, cattle_hip_optimizer 
 				static_cast<double*>(p.moments[2].p), static_cast<double*>(p.values.p), reset_grad, l1, l2);
 	if (p.constrains_values())
 		constrain(p, true);              /* the optimizers hand the new values to set_values */
-	++p.version;
+	p.values_changed();
 }
 
 /* The update + gradient reset of many parameters, OPT_BATCH per launch. A parameter shared by several of the listed
@@ -1806,22 +1942,22 @@ void run_optimizer_many(const cattle_hip_layer_t* layers, const size_t* indices,
 			limited.push_back(&p);         /* constrained after the update; the prepared layouts are rebuilt from the result */
 		} else if (weights_of) {
 			const ConvShape& cs = *weights_of;
-			fwd_current = p.derived[0].p && p.derived_version[0] == p.version;
-			dgrad_current = p.derived[1].p && p.derived_version[1] == p.version && p.dgrad_layout == 0;
+			fwd_current = p.ready(PREPARED_FORWARD, 0);
+			dgrad_current = p.ready(PREPARED_DGRAD, 0);
 			q.K = cs.K();
 			q.RHW = cs.RH * cs.RW;
 			q.ldw_fwd = prepared_weight_row_length(cs.F);
 			q.ldw_dgrad = prepared_weight_row_length(cs.C);
 			if (fwd_current)
-				q.wt_fwd = static_cast<T*>(p.derived[0].p);
+				q.wt_fwd = static_cast<T*>(p.prepared[PREPARED_FORWARD].buf.p);
 			if (dgrad_current)
-				q.wt_dgrad = static_cast<T*>(p.derived[1].p);
+				q.wt_dgrad = static_cast<T*>(p.prepared[PREPARED_DGRAD].buf.p);
 		}
-		++p.version;
+		p.values_changed();
 		if (fwd_current)
-			p.derived_version[0] = p.version;
+			p.built(PREPARED_FORWARD, 0);
 		if (dgrad_current)
-			p.derived_version[1] = p.version;
+			p.built(PREPARED_DGRAD, 0);
 		if (batch.count == OPT_BATCH)
 			flush();
 	}
@@ -2054,6 +2190,8 @@ int cattle_hip_graph_end_capture(cattle_hip_graph_t* graph) {
 		}
 		g_capturing = false;
 		std::unique_ptr<Graph> gr(new Graph());
+		g_recording.put_back();
+		gr->uses.entries.swap(g_recording.entries);
 		/* blocks freed during the recording stay out of circulation, whatever becomes of the graph */
 		gr->blocks.swap(g_pool.held);
 		for (void* b : g_pool.taken)
@@ -2087,7 +2225,10 @@ int cattle_hip_graph_launch(cattle_hip_graph_t graph) {
 		forbid_while_capturing("launching a graph");
 		g_deferred.settle();            /* the recorded calls did not know of sums that eager passes have left pending since, */
 		g_clears.settle();              /* nor of gradients that they have reset */
-		CATTLE_HIP_CHECK(hipGraphLaunch(reinterpret_cast<Graph*>(graph)->exec, stream()));
+		Graph* gr = reinterpret_cast<Graph*>(graph);
+		gr->uses.before_launch();
+		CATTLE_HIP_CHECK(hipGraphLaunch(gr->exec, stream()));
+		gr->uses.after_launch();
 	});
 }
 
@@ -2318,7 +2459,7 @@ int cattle_hip_convlstm_set_kernel_values(cattle_hip_layer_t lstm, size_t kernel
 		size_t offset, bytes;
 		Param& p = lstm_kernel_param(lstm, kernel, bias, offset, bytes);
 		copy_in((char*) p.values.p + offset, values, space, bytes);
-		++p.version;
+		p.values_changed();
 	});
 }
 
@@ -2693,7 +2834,7 @@ int cattle_hip_layer_set_param_values(cattle_hip_layer_t layer, size_t index, co
 		copy_in(p.values.p, values, space, p.bytes());
 		if (p.constrains_values())
 			constrain(p, true);
-		++p.version;
+		p.values_changed();
 	});
 }
 
@@ -2779,7 +2920,7 @@ int cattle_hip_layer_param_set_constraints(cattle_hip_layer_t layer, size_t inde
 		std::memcpy(p.grad_limits, v + 3, sizeof(p.grad_limits));
 		if (p.constrains_values()) {
 			constrain(p, true);
-			++p.version;
+			p.values_changed();
 		}
 	});
 }

@@ -102,6 +102,8 @@ int cattle_hip_timer_stop(cattle_hip_timer_t timer, float* elapsed_ms);   /* syn
  *    cattle_hip_alloc returned during the recording; cattle_hip_free on them takes effect when the graph is destroyed),
  *    the same batch size, and the same scalars - an optimizer whose update depends on the time step or epoch (Adam,
  *    Nadam, AMSGrad, ...) is therefore called outside the recording, as is anything whose result the host must see;
+ *  - values of parameters may change between launches by any call, on or off the graph (set_values, optimizer calls, constraints, other
+ *    passes of the layer at the same or another batch size); a launch works on the values as they are;
  *  - a training pass of a dropout layer cannot be recorded (CATTLE_HIP_ERR_STATE): its mask is a function of the number
  *    of the pass, which a replay would not advance; record the layers on either side of it;
  *  - a graph holds the device addresses it was recorded with. As long as it exists, a buffer of the library that was
