@@ -14,7 +14,7 @@ using namespace tap_product;
  * waits. The wavefronts of a block are the column tiles of the same rows, or neighbouring rows: what they share comes from the
  * caches. gather_gemm_kernel takes such a reduction in two to seven chunks with a barrier and a round trip to memory each:
  * 65,536 x 27 x 16 7.7 -> 6.2 us. Bound by latency. */
-template<int SPC>
+template<int SPC, bool ODD>
 __global__ __launch_bounds__(256)
 void few_channels_kernel(const float* __restrict__ src, const float* __restrict__ wt, const float* __restrict__ bias, float* __restrict__ out,
 		const GatherGeom g, const StepGeom G, int ftiles, int tiles, int blocks) {
@@ -31,7 +31,7 @@ void few_channels_kernel(const float* __restrict__ src, const float* __restrict_
 	#pragma unroll
 	for (int r = 0; r < 16; ++r)
 		bv[r] = bias != nullptr ? bias[min(f0 + acc_row<float>(r, lk), g.F - 1)] : 0.f;
-	const acc_t acc = share_of_product<SPC>(src, wt, g, G, row, valid, lk, f0 + lc, 0);
+	const acc_t acc = share_of_product<SPC, ODD>(src, wt, g, G, row, valid, lk, f0 + lc, 0);
 	if (!valid)
 		return;
 	#pragma unroll
@@ -57,10 +57,10 @@ void few_channels_product(const float* src, const float* wt, const float* bias, 
 	const int ftiles = tiles_of(g.F), tiles = tiles_of(g.M) * ftiles, blocks = (tiles + 3) / 4;
 	const StepGeom G = step_geom(g);
 	const dim3 grid((unsigned) ((blocks + 7) / 8 * 8));
-	switch ((g.LC + 1) / 2) {
-#define CATTLE_HIP_STEPS(n) case n: few_channels_kernel<n><<<grid, 256, 0, stream()>>>(src, wt, bias, out, g, G, ftiles, tiles, blocks); break;
-	CATTLE_HIP_STEPS(1) CATTLE_HIP_STEPS(2) CATTLE_HIP_STEPS(3)
-#undef CATTLE_HIP_STEPS
+	switch (g.LC) {
+#define CATTLE_HIP_CHANNELS(n) case n: few_channels_kernel<(n + 1) / 2, n % 2 != 0><<<grid, 256, 0, stream()>>>(src, wt, bias, out, g, G, ftiles, tiles, blocks); break;
+	CATTLE_HIP_CHANNELS(1) CATTLE_HIP_CHANNELS(2) CATTLE_HIP_CHANNELS(3) CATTLE_HIP_CHANNELS(4) CATTLE_HIP_CHANNELS(5) CATTLE_HIP_CHANNELS(6)
+#undef CATTLE_HIP_CHANNELS
 	}
 	CATTLE_HIP_CHECK(hipGetLastError());
 }

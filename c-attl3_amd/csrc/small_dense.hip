@@ -8,7 +8,9 @@
 namespace cattle_hip {
 namespace {
 
-constexpr unsigned OUTSIDE = 0x80000000u;       /* a byte offset beyond any buffer: such a load returns zero */
+/* A byte offset beyond any buffer: such a load returns zero. Every load below is in range by the lane's own choice between its offset and
+ * this one; none counts on the range check for a sum of its two offsets, and the wavefront's alone lies inside the buffer. */
+constexpr unsigned OUTSIDE = 0x80000000u;
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -56,22 +58,24 @@ __device__ __forceinline__ void finish_product(const ProductArgs& A, float* __re
 	__builtin_nontemporal_store(v, out + at);
 }
 
-/* PAIRS: rows 2 l and 2 l + 1 of a tile belong to lane l, one load of eight bytes; else rows l and l + 16. */
+/* PAIRS: rows 2 l and 2 l + 1 of a tile belong to lane l, one load of eight bytes; else rows l and l + 16. x_last: the offsets of the last
+ * of the steps, past whose reduction indices there may be none. */
 template<int MB, bool PAIRS, int STEPS>
 __device__ __forceinline__ void product_steps(f32x4 (&acc)[chains(MB)][MB], __amdgpu_buffer_rsrc_t x_buf, __amdgpu_buffer_rsrc_t wt_buf,
-		unsigned x_lane, unsigned w_lane, unsigned x_wave, unsigned w_wave, unsigned x_step, unsigned w_step) {
+		const unsigned (&x_lane)[MB], const unsigned (&x_last)[MB], unsigned w_lane, unsigned x_wave, unsigned w_wave, unsigned x_step,
+		unsigned w_step) {
 	float x[STEPS][MB], w[STEPS];
 	#pragma unroll
 	for (int s = 0; s < STEPS; ++s) {
 		w[s] = load_1(wt_buf, w_lane, w_wave + (unsigned) s * w_step);
 		if constexpr (PAIRS) {
-			const f32x2 v = load_2(x_buf, x_lane, x_wave + (unsigned) s * x_step);
+			const f32x2 v = load_2(x_buf, s == STEPS - 1 ? x_last[0] : x_lane[0], x_wave + (unsigned) s * x_step);
 			x[s][0] = v[0];
 			x[s][MB - 1] = v[1];
 		} else {
 			#pragma unroll
 			for (int j = 0; j < MB; ++j)
-				x[s][j] = load_1(x_buf, x_lane, x_wave + (unsigned) s * x_step + 64u * (unsigned) j);
+				x[s][j] = load_1(x_buf, s == STEPS - 1 ? x_last[j] : x_lane[j], x_wave + (unsigned) s * x_step);
 		}
 	}
 	__builtin_amdgcn_sched_barrier(0);
@@ -106,9 +110,15 @@ void small_product_kernel(const float* __restrict__ src, const float* __restrict
 	int s = wave * A.per;
 	const int end = min(total, s + A.per);
 	const unsigned x_step = 4u * PK * (unsigned) A.M, w_step = 4u * PK * (unsigned) A.ldw;
-	/* (rows past M are rows of the next reduction index, or beyond the buffer: they end up in rows of the tile that nobody stores;
-	 * reduction indices past K lie beyond the buffer and meet zero weights) */
-	const unsigned x_lane = 4u * (unsigned) (m0 + (PAIRS ? 2 * lc : lc) + lk * A.M), w_lane = 4u * (unsigned) (f0 + lc + lk * A.ldw);
+	/* (rows past M and reduction indices past K are zeros; the weights have rows for all steps and columns for all tiles) */
+	unsigned x_lane[MB], x_last[MB];
+	#pragma unroll
+	for (int j = 0; j < MB; ++j) {
+		const int row = m0 + (PAIRS ? 2 * lc + j : lc + PL * j);
+		x_lane[j] = row < A.M ? 4u * (unsigned) (row + lk * A.M) : OUTSIDE;
+	}
+	const bool past_K = PK * (total - 1) + lk >= A.K;
+	const unsigned w_lane = 4u * (unsigned) (f0 + lc + lk * A.ldw);
 	/* Every fourth (eighth) step goes to an accumulator of its own, so that a sum is rounded as often as one of a fraction of the
 	 * length. Error of the output against 64 bits in the 2-norm, with one, and with these: 256 x 784 -> 512 1.5e-7, 1.0e-7; 128 x 3000 ->
 	 * 128 2.6e-7, 1.2e-7 (1.2e-7 on the bf16 instructions). */
@@ -122,12 +132,15 @@ void small_product_kernel(const float* __restrict__ src, const float* __restrict
 	while (s < end) {
 		const int steps = min(end - s, MAX_STEPS);
 		const unsigned x_wave = (unsigned) s * x_step, w_wave = (unsigned) s * w_step;
+		#pragma unroll
+		for (int j = 0; j < MB; ++j)
+			x_last[j] = s + steps == total && past_K ? OUTSIDE : x_lane[j];
 		switch (steps) {
-#define CATTLE_HIP_STEPS(n) case n: product_steps<MB, PAIRS, n>(sums, x_buf, wt_buf, x_lane, w_lane, x_wave, w_wave, x_step, w_step); break;
+#define CATTLE_HIP_STEPS(n) case n: product_steps<MB, PAIRS, n>(sums, x_buf, wt_buf, x_lane, x_last, w_lane, x_wave, w_wave, x_step, w_step); break;
 		CATTLE_HIP_STEPS(1) CATTLE_HIP_STEPS(2) CATTLE_HIP_STEPS(3) CATTLE_HIP_STEPS(4) CATTLE_HIP_STEPS(5) CATTLE_HIP_STEPS(6)
 		CATTLE_HIP_STEPS(7) CATTLE_HIP_STEPS(8) CATTLE_HIP_STEPS(9) CATTLE_HIP_STEPS(10) CATTLE_HIP_STEPS(11) CATTLE_HIP_STEPS(12)
 		CATTLE_HIP_STEPS(13) CATTLE_HIP_STEPS(14) CATTLE_HIP_STEPS(15)
-		default: product_steps<MB, PAIRS, MAX_STEPS>(sums, x_buf, wt_buf, x_lane, w_lane, x_wave, w_wave, x_step, w_step);
+		default: product_steps<MB, PAIRS, MAX_STEPS>(sums, x_buf, wt_buf, x_lane, x_last, w_lane, x_wave, w_wave, x_step, w_step);
 #undef CATTLE_HIP_STEPS
 		}
 		s += steps;
@@ -212,7 +225,7 @@ void small_product_ordered_kernel(const float* __restrict__ src, const float* __
 	int s = wave * A.per;
 	const int end = min(A.K / OK, s + A.per);
 	const unsigned x_step = 4u * OK * (unsigned) A.M, w_step = 4u * OK * (unsigned) A.ldw;
-	const unsigned x_lane = 4u * (unsigned) (m0 + lc + lk * A.M), w_lane = 4u * (unsigned) (f0 + lc + lk * A.ldw);
+	const unsigned x_lane = m0 + lc < A.M ? 4u * (unsigned) (m0 + lc + lk * A.M) : OUTSIDE, w_lane = 4u * (unsigned) (f0 + lc + lk * A.ldw);
 	Mfma<float>::acc_t acc;
 	#pragma unroll
 	for (int r = 0; r < 16; ++r)
@@ -284,14 +297,16 @@ void small_weight_gradient_kernel(const float* __restrict__ x, const float* __re
 	f32x4 xv[HALVES][LOADS], gv[HALVES][LOADS], yv[ACT ? HALVES : 1][LOADS];
 	#pragma unroll
 	for (int h = 0; h < HALVES; ++h) {
-		const bool in = m0 + h * HALF_M < M;            /* (columns past K or F lie beyond the buffers) */
-		const unsigned xo = in ? x_lane : OUTSIDE, go = in ? g_lane : OUTSIDE, half = 4u * HALF_M * (unsigned) h;
+		const bool in = m0 + h * HALF_M < M;
+		const unsigned half = 4u * HALF_M * (unsigned) h;
 		#pragma unroll
 		for (int q = 0; q < LOADS; ++q) {
-			gv[h][q] = load_4(og_buf, go, half + rows * (unsigned) q);
+			const unsigned at = half + rows * (unsigned) q;
+			const unsigned xo = in && k0 + row + ROWS * q < K ? x_lane + at : OUTSIDE, go = in && f0 + row + ROWS * q < F ? g_lane + at : OUTSIDE;
+			gv[h][q] = load_4(og_buf, go, 0u);
 			if constexpr (ACT)
-				yv[h][q] = load_4(y_buf, go, half + rows * (unsigned) q);
-			xv[h][q] = load_4(x_buf, xo, half + rows * (unsigned) q);
+				yv[h][q] = load_4(y_buf, go, 0u);
+			xv[h][q] = load_4(x_buf, xo, 0u);
 		}
 	}
 	/* the gradient that the sums are added to, fetched with the operands: up to four values a thread, all of them from 256 threads on */
