@@ -34,7 +34,7 @@ EXPORTS = [
     "cattle_hip_batchnorm_set_stats_initialized", "cattle_hip_activation_create", "cattle_hip_pool_create",
     "cattle_hip_convlstm_set_multiplicative_integration", "cattle_hip_convlstm_fused_steps", "cattle_hip_last_products", "cattle_hip_layer_param_set_regularization",
     "cattle_hip_layer_param_regularization_penalty", "cattle_hip_dropout_create", "cattle_hip_reshape_create", "cattle_hip_broadcast_create",
-    "cattle_hip_layer_clone", "cattle_hip_layer_destroy", "cattle_hip_layer_input_dims",
+    "cattle_hip_layer_keep_sum_order", "cattle_hip_layer_clone", "cattle_hip_layer_destroy", "cattle_hip_layer_input_dims",
     "cattle_hip_layer_output_dims", "cattle_hip_layer_is_input_layer", "cattle_hip_layer_set_input_layer",
     "cattle_hip_layer_empty_cache", "cattle_hip_layer_forward", "cattle_hip_layer_backward",
     "cattle_hip_layer_num_params", "cattle_hip_layer_param_shape", "cattle_hip_layer_set_param_values",
@@ -459,6 +459,11 @@ class Layer(object):
             _check(rc)
         return bool(v.value)
 
+    def keep_sum_order(self, enabled=True):
+        """The forward products of a convolutional or dense layer in the order of sums of the tiled launches, whichever is the
+        fastest (cattle_hip_layer_keep_sum_order); for layers behind a max pool."""
+        _check(lib().cattle_hip_layer_keep_sum_order(self._h, ctypes.c_int(int(bool(enabled)))))
+
     def set_input_layer(self, flag):
         _check(lib().cattle_hip_layer_set_input_layer(self._h, ctypes.c_int(int(bool(flag)))))
 
@@ -882,8 +887,14 @@ class FusedKernelLayer(Layer):
 def fuse_layers(layers):
     """The layer list of a feed-forward network with every convolutional or dense layer and the batch norm, activation
     and pool layers right behind it (in this order, each optional) replaced by one FusedKernelLayer over them; the other
-    layers stay as they are. Calling the result in order equals calling `layers` in order."""
+    layers stay as they are. Calling the result in order equals calling `layers` in order. The kernel layers behind a max pool
+    keep the order of their sums from here on (Layer.keep_sum_order)."""
     out, i = [], 0
+    pooled = False
+    for l in layers:
+        if pooled and isinstance(l, (ConvKernelLayer, DenseKernelLayer)):
+            l.keep_sum_order()
+        pooled = pooled or isinstance(l, MaxPoolLayer)
     while i < len(layers):
         group = [layers[i]]
         if isinstance(layers[i], (ConvKernelLayer, DenseKernelLayer)):

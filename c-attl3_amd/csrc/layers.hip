@@ -1327,11 +1327,13 @@ struct FusedLayer : LayerBase {
 	 * value falls on decides whether its gradient passes, and of the million values of a few batches of an MLP (784-512-256-10, eight
 	 * batches of 256) another order of the sums moves one across now and then: the trained parameters are then 1.5e-4 from where
 	 * they were (2e-7 without such a value), with neither side the more accurate.
-	 * The member layer itself is not touched: called alone it chooses like any other. */
+	 * A kernel layer behind max pools, the head of an image classifier for one, asks for the same through its own shape
+	 * (cattle_hip_layer_keep_sum_order), since it does not see what lies in front of it. The member layer itself is not touched: called
+	 * alone, or with a rectifier behind it that is not part of the group, it chooses like any other. */
 	ConvShape shape(bool training = false) const {
 		ConvShape s = conv->shape;
 		s.fp32_products = pool && pool->kind == CATTLE_HIP_POOL_MAX;
-		s.keeps_sums = s.fp32_products || (training && act && (act_sign_coded(act->kind) || act->kind == CATTLE_HIP_ACT_BINARY_STEP));
+		s.keeps_sums = s.keeps_sums || s.fp32_products || (training && act && (act_sign_coded(act->kind) || act->kind == CATTLE_HIP_ACT_BINARY_STEP));
 		return s;
 	}
 	int OH() const { return conv->shape.OH(); }
@@ -2634,6 +2636,16 @@ int cattle_hip_fused_last_mode(cattle_hip_layer_t fused, int* mode) {
 			*mode = f->mode;
 		else
 			throw Error(ERR_INVALID, "not a fused layer");
+	});
+}
+
+int cattle_hip_layer_keep_sum_order(cattle_hip_layer_t layer, int enabled) {
+	return guarded([&] {
+		LayerBase* l = as_layer(layer);
+		if (ConvLayer<float>* c = dynamic_cast<ConvLayer<float>*>(l))
+			c->shape.keeps_sums = enabled != 0;
+		else if (FusedLayer<float>* f = dynamic_cast<FusedLayer<float>*>(l))
+			f->conv->shape.keeps_sums = enabled != 0;
 	});
 }
 

@@ -422,12 +422,10 @@ bool small_product_possible(const GatherGeom& g, int cus) {
 	/* Up to two tiles per CU, three where the reduction is short; more tiles, and reductions of more than three batches of loads a
 	 * wavefront, go to the tiled launches. Whole passes, this kernel against those: 256 x 3072 -> 128 32.6 us against 45.4, 512 x 600
 	 * x 600 (608 tiles) 41.6 / 48.1, 256 x 512 x 1500 (752) 33.7 / 36.1; but 128 x 2048 x 3000 (752) 89.4 / 86.3, 2048 x 500 x 200 (832) 44.1 /
-	 * 43.0, and 128 x 8192 -> 256 66.3 / 57.6 (at 5000 inputs as fast). Below 32 reduction indices there is nothing to deal out. */
+	 * 43.0, and 128 x 8192 -> 256 66.3 / 57.6 (at 5000 inputs as fast). Below 32 reduction indices there is nothing to deal out. Forward
+	 * launches of few columns, this kernel against those: 128 x 1100 -> 10 4.8 / 7.3, 128 x 3072 -> 10 8.3 / 10.4, 1 x 2000 -> 10 7.0 / 12.4,
+	 * 128 x 2000 -> 2 6.2 / 53.9 (few_columns_plain_kernel). */
 	const long tiles = (long) up(g.M, 2 * PL) * up(g.F, PL);
-	/* A long reduction for one tile of columns is the head of an image classifier. Its products stay as they were: what they are
-	 * rounded to moves the arg-max picks of the pools in front of it, a step later (FusedLayer::shape). */
-	if (g.F <= PL && g.K > 1024)
-		return false;
 	return g.K >= 32 && g.K <= 3072 && tiles <= (g.K <= 1024 ? 3 : 2) * (long) cus;
 }
 

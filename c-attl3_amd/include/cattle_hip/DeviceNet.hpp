@@ -276,7 +276,9 @@ public:
 		cattle_hip_layer_t h = nullptr;
 		check(cattle_hip_pool_create(Code<Scalar>::value, kind, input_dims[0], input_dims[1], input_dims[2], receptor_height,
 				receptor_width, vertical_stride, horizontal_stride, &h));
-		return DeviceLayer(h);
+		DeviceLayer layer(h);
+		layer.max_pool = kind == CATTLE_HIP_POOL_MAX;
+		return layer;
 	}
 	/* layer/DropoutLayer.hpp:33-42; `seed` keys the generator of the masks (give every dropout layer its own) */
 	inline static DeviceLayer dropout(const Dims& dims, Scalar dropout_prob, unsigned long long seed = 0, Scalar epsilon = 1e-5) {
@@ -319,7 +321,7 @@ public:
 	}
 	inline DeviceLayer(DeviceLayer&& other) : handle(other.handle), in_dims(other.in_dims), out_dims(other.out_dims),
 			cached_in(std::move(other.cached_in)), cached_out(std::move(other.cached_out)),
-			params_per_column(other.params_per_column), kernel_layer(other.kernel_layer) {
+			params_per_column(other.params_per_column), kernel_layer(other.kernel_layer), max_pool(other.max_pool) {
 		other.handle = nullptr;
 	}
 	DeviceLayer(const DeviceLayer&) = delete;
@@ -411,6 +413,13 @@ public:
 	/** Whether the layer is a kernel layer: parameter 0 its weight matrix, parameter 1 its bias. */
 	inline bool is_kernel_layer() const {
 		return kernel_layer;
+	}
+	inline bool is_max_pool() const {
+		return max_pool;
+	}
+	/** The order of a kernel layer's sums stays that of the tiled launches (cattle_hip_layer_keep_sum_order). */
+	inline void keep_sum_order(bool enabled = true) {
+		check(cattle_hip_layer_keep_sum_order(handle, enabled ? 1 : 0));
 	}
 	/**
 	 * Parameters::init_values (parameters/StandardParameters.hpp:91-95) for parameter `index`: the initialization applied
@@ -561,7 +570,7 @@ public:
 		}
 	}
 private:
-	inline explicit DeviceLayer(cattle_hip_layer_t handle) : handle(handle), params_per_column(false), kernel_layer(false) {
+	inline explicit DeviceLayer(cattle_hip_layer_t handle) : handle(handle), params_per_column(false), kernel_layer(false), max_pool(false) {
 		std::size_t d[3];
 		check(cattle_hip_layer_input_dims(handle, d));
 		in_dims = Dims{ { d[0], d[1], d[2] } };
@@ -573,7 +582,7 @@ private:
 		in_dims = in;
 	}
 	inline DeviceLayer(cattle_hip_layer_t handle, const Dims& in, const Dims& out) : handle(handle), in_dims(in),
-			out_dims(out), params_per_column(false), kernel_layer(false) { }
+			out_dims(out), params_per_column(false), kernel_layer(false), max_pool(false) { }
 	template<typename Fn>
 	inline void for_each_optimizable(Fn fn) {
 		const std::size_t n = num_params();
@@ -598,6 +607,7 @@ private:
 	DeviceTensor<Scalar> cached_in, cached_out;
 	bool params_per_column;
 	bool kernel_layer;          /* a weight matrix (parameter 0) and a bias (parameter 1): conv, transposed conv, dense */
+	bool max_pool;
 };
 
 /**
@@ -685,8 +695,13 @@ public:
 			frozen(false) {
 		assert(!this->layers.empty());
 		this->layers[0].set_input_layer(foremost);
-		for (std::size_t i = 0; i < this->layers.size(); ++i)
+		bool pooled = false;
+		for (std::size_t i = 0; i < this->layers.size(); ++i) {
 			units.push_back(Unit{ i, 1, NO_FUSED });
+			if (pooled)
+				this->layers[i].keep_sum_order();
+			pooled = pooled || this->layers[i].is_max_pool();
+		}
 	}
 	inline std::vector<DeviceLayer<Scalar>>& get_layers() {
 		return layers;

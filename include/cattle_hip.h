@@ -211,6 +211,12 @@ int cattle_hip_fused_create(const cattle_hip_layer_t* layers, size_t count, catt
 /* How the last forward pass of a fused handle ran: 0 none yet, 1 member by member, 2 activation in the GEMM epilogue,
  * 3 activation and max or mean pooling in the GEMM epilogue, 4 batch-norm moments from the GEMM epilogue + one chain pass. */
 int cattle_hip_fused_last_mode(cattle_hip_layer_t fused, int* mode);
+/* Whether the forward products of a convolutional or dense layer (or of a fused handle's) take their sums in the order of the tiled
+ * launches even where a launch for small products is faster (no counterpart in the reference; off when a layer is created; other
+ * layers take no notice; fp32 only, the fp64 launches have one order). For the kernel layers of a network behind a max pool: what their
+ * products are rounded to decides, a training step later, which of two nearly equal values the pool picks, and with it results far
+ * above rounding, whichever order is the more accurate. */
+int cattle_hip_layer_keep_sum_order(cattle_hip_layer_t layer, int enabled);
 
 /* DropoutLayer<Scalar,Rank>(dims, dropout_prob, epsilon) - layer/DropoutLayer.hpp:33-42, passes :74-96: a training
  * pass multiplies by the inverted-dropout mask (0 where u <= dropout_prob, else 1 / (1 - dropout_prob + epsilon)), an

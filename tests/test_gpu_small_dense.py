@@ -78,3 +78,31 @@ def test_non_finite_operands_stay_in_their_rows():
     bad = np.zeros(N, bool)
     bad[[3, 17]] = True
     assert np.all(np.isfinite(y[~bad])) and not np.any(np.isfinite(y[bad]))
+
+
+@pytest.mark.parametrize("inputs", [900, 2000])
+def test_layers_behind_a_max_pool_keep_the_order_of_their_sums(inputs):
+    """The order is asked for, not guessed from sizes: a dense layer alone takes the small launch, one behind a pool the sums of the
+    tiled launches, which a training pass in front of a rectifier takes too."""
+    N, F = 64, 10
+    gen = hp.rng(inputs)
+    x = ch.DeviceTensor.from_host(hp.normal(gen, (N, inputs), np.float32))
+    w, b = hp.normal(gen, (inputs, F), np.float32), hp.normal(gen, (1, F), np.float32)
+    dense = ch.DenseKernelLayer(np.float32, (inputs,), F)
+    dense.get_params()[0].set_values(w)
+    dense.get_params()[1].set_values(b)
+    alone = dense.pass_forward(x, True).to_host()
+    (rectified,) = ch.fuse_layers([dense, ch.ActivationLayer(np.float32, "relu", (F,))])
+    tiled = rectified.pass_forward(x, True).to_host()
+    assert np.array_equal(dense.pass_forward(x, True).to_host(), alone)
+    pool = ch.MaxPoolLayer(np.float32, (4, inputs // 4, 4))
+    assert ch.fuse_layers([pool, dense])[1] is dense
+    behind = dense.pass_forward(x, True).to_host()
+    positive = behind > 0
+    assert np.array_equal(behind[positive], tiled[positive]) and not np.array_equal(behind, alone)
+    ref = np.asarray(x.to_host(), np.float64) @ w.astype(np.float64) + b
+    size = np.abs(x.to_host()) @ np.abs(w) + np.abs(b)
+    for got in (alone, behind):
+        assert np.all(np.abs(got - ref) <= _bound(inputs + 1) * size)
+    dense.keep_sum_order(False)
+    assert np.array_equal(dense.pass_forward(x, True).to_host(), alone)
