@@ -430,7 +430,7 @@ def loss_d_function(kind, out, obj, epsilon=1e-5, scale=1.0, sequential=False, n
     else:
         grad = np.empty(out.shape, dtype=out.dtype, order="F")
     rc = _step.loss_d_function(_dtype_code(out.dtype), LOSS[kind] | (LOSS_NEGATED if negated else 0), ptr(out), space, ptr(obj), space,
-                               batch, steps, size, float(epsilon), float(scale), ptr(grad), space)
+                               batch, steps, size, _D(epsilon), _D(scale), ptr(grad), space)
     if rc:
         _check(rc)
     return grad

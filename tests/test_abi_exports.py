@@ -71,3 +71,19 @@ def test_noalloc_wrapper_refuses_mismatched_buffers(monkeypatch, what, kw):
         (args if k in args else geom)[k] = v
     with pytest.raises(ValueError):
         binding.conv_forward_noalloc(args["x"], args["weights"], args["bias"], args["out"], **geom)
+
+
+@pytest.mark.parametrize("kw", [dict(epsilon="1e-5"), dict(scale="2")], ids=str)
+def test_loss_gradient_takes_numbers_only(monkeypatch, kw):
+    import numpy as np
+    binding = importlib.import_module("c-attl3_amd.binding")
+
+    class Library(object):
+        def loss_d_function(self, *args):
+            return 0
+
+    monkeypatch.setattr(binding, "_step", Library())
+    a = np.zeros((2, 3), np.float32, order="F")
+    with pytest.raises(TypeError):
+        binding.loss_d_function("squared", a, a, **kw)
+    binding.loss_d_function("squared", a, a, epsilon=np.float32(1), scale=2)
