@@ -241,7 +241,8 @@ def conv_forward_noalloc(x, weights, bias, out, receptor_height=3, receptor_widt
 
 def last_products():
     """(product, weight gradient): rows * 1000 + columns of the tile that the last forward or input-gradient product and the
-    last weight gradient of a kernel layer took on the bf16 matrix instructions, 0 where they ran on others."""
+    last weight gradient of a kernel layer took on the bf16 matrix instructions, a negative number for the fp32 launches without tiles
+    (-1 small dense, -2 small dense in the tiled order of sums, -3 few channels, -4 few weights), 0 for all others."""
     p, w = ctypes.c_int(), ctypes.c_int()
     _check(lib().cattle_hip_last_products(ctypes.byref(p), ctypes.byref(w)))
     return int(p.value), int(w.value)

@@ -48,7 +48,7 @@ def _within(got, ref, mag, terms):
 
 # batch, inputs, outputs: fewer inputs than a tile of the weight gradient has; a remainder of the reduction's steps; fewer rows than a
 # block, of one and of two row blocks; the kernel that keeps the order of the sums (training, behind a rectifier)
-DENSE = [(4, 1, 32), (4, 3, 40), (36, 20, 33), (512, 23, 64), (256, 5, 40), (7, 33, 40), (5, 35, 4100), (33, 50, 4000), (1, 97, 10), (30, 66, 48)]
+DENSE = [(4, 1, 32), (4, 3, 40), (36, 20, 33), (512, 23, 64), (256, 5, 40), (7, 33, 40), (5, 35, 4100), (33, 50, 4000), (1, 97, 10), (30, 66, 48), (17, 100, 130)]
 
 
 @pytest.mark.gpu
@@ -64,8 +64,12 @@ def test_dense_layers(case, act):
     (layer,) = ch.fuse_layers([dense] + ([ch.ActivationLayer(np.float32, "relu", (F,))] if act else []))
     out, dx = ch.DeviceTensor((N, F), np.float32), ch.DeviceTensor((N, K), np.float32)
     xd, gd = _Between(x), _Between(g)
+    # (ch.last_products(): the launches that these cases are meant for)
     layer.forward_into(xd, out)
+    assert ch.last_products()[0] == ((-2 if case == (17, 100, 130) else 0) if act else -1 if K >= 32 else 0)
     layer.backward_into(gd, dx)
+    if act:
+        assert ch.last_products() == (-1 if 32 <= F <= 3072 else 0, -1 if F >= 32 and N % 4 == 0 else 0)
     y = out.to_host()
     x64, w64, g64 = (np.asarray(a, np.float64) for a in (x, w, g))
     z, size = x64 @ w64 + b, np.abs(x64) @ np.abs(w64) + np.abs(b)
@@ -81,6 +85,8 @@ def test_dense_layers(case, act):
 CONV = [(33, 9, 1, 1, 16, 1, 1, 0, 0), (32, 1, 9, 1, 16, 1, 1, 0, 0), (16, 1, 1, 5, 12, 1, 1, 0, 0), (16, 1, 1, 4, 12, 1, 1, 0, 0), (12, 2, 2, 3, 24, 2, 2, 1, 1),
         (12, 2, 2, 3, 24, 1, 1, 0, 0), (8, 30, 1, 3, 9, 2, 1, 1, 0), (21, 7, 5, 3, 33, 1, 1, 0, 0), (64, 12, 12, 1, 10, 1, 1, 0, 0), (5, 9, 8, 5, 16, 2, 0, 0, 0),
         (16, 9, 1, 12, 5, 1, 1, 0, 0)]
+# the last tap of a lone last channel reaches past the image
+TILED = [(33, 9, 1, 1, 16, 1, 1, 0, 0), (16, 1, 1, 5, 12, 1, 1, 0, 0), (12, 2, 2, 3, 24, 2, 2, 1, 1), (8, 30, 1, 3, 9, 2, 1, 1, 0)]
 
 
 @pytest.mark.gpu
@@ -97,6 +103,7 @@ def test_convolutions(case):
     out, dx = ch.DeviceTensor(g.shape, np.float32), ch.DeviceTensor(x.shape, np.float32)
     xd, gd = _Between(x), _Between(g)
     layer.forward_into(xd, out)
+    assert (ch.last_products()[0] == -3) == (C <= 6 and case not in TILED)
     layer.backward_into(gd, dx)
     x64, w64, b64, g64 = (np.asarray(a, np.float64) for a in (x, w, b, g))
     ref, cache = oracle.conv_forward(x64, w64, b64, return_cache=True, **geom)
