@@ -44,12 +44,12 @@ void few_channels_kernel(const float* __restrict__ src, const float* __restrict_
 
 } /* namespace */
 
-bool few_channels_possible(const GatherGeom& g) {
-	/* Up to eight wavefronts of 32 x 32 per CU of a chip of 256. More of them are better served by tiles that are fetched once for
+bool few_channels_possible(const GatherGeom& g, int cus) {
+	/* Up to eight wavefronts of 32 x 32 per CU. More of them are better served by tiles that are fetched once for
 	 * several: a pass of 524,288 x 27 x 16 85 us against 74.5, one of 81,920 x 72 x 128 42 us against 27; and longer reductions by the
 	 * chunks that overlap the products (3200 x 108 x 64 28.0 against 27.1). 25,088 x 54 x 10 27.2 against 31.9. */
 	const double tiles = (double) tiles_of(g.M) * tiles_of(g.F);
-	return addressable(g) && g.LC <= 6 && tiles <= 2048 && g.F > 8 && g.out_M == g.M && g.out_a0 == 0 && g.out_b0 == 0 && g.out_sa == 1 && g.out_sb == 1 &&
+	return addressable(g) && g.LC <= 6 && tiles <= 8.0 * cus && g.F > 8 && g.out_M == g.M && g.out_a0 == 0 && g.out_b0 == 0 && g.out_sa == 1 && g.out_sb == 1 &&
 			g.out_OA == g.OA;
 }
 

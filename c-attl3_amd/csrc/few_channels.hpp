@@ -9,8 +9,8 @@
 namespace cattle_hip {
 
 /* Whether the product of this gather is one of few_channels_product's: 3 x 3 taps without divisors, a handful of channels, the plain
- * output map. */
-bool few_channels_possible(const GatherGeom& g);
+ * output map, on a chip of `cus` CUs. */
+bool few_channels_possible(const GatherGeom& g, int cus);
 /* out = gather(src) wt + bias; any batch size and alignment */
 void few_channels_product(const float* src, const float* wt, const float* bias, float* out, const GatherGeom& g);
 

@@ -2487,7 +2487,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 		}
 	/* a handful of channels whose products stay on the fp32 instructions */
 	if constexpr (std::is_same<T, float>::value)
-		if (chosen == &vars[best_v] && !rider && epi == EPI_NONE && then == nullptr && !g.keeps_sums && !g.fp32_products && few_channels_possible(g)) {
+		if (chosen == &vars[best_v] && !rider && epi == EPI_NONE && then == nullptr && !g.keeps_sums && !g.fp32_products && few_channels_possible(g, device_shape().cus)) {
 			few_channels_product(src, wt, bias, out, g);
 			g_last_products.product = RAN_FEW_CHANNELS;
 			if (mtiles_out)
