@@ -47,7 +47,8 @@ SHAPE = dict(H=56, W=56, C=64, F=128, RH=3, RW=3)
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "conv_cfg4_hbm_traffic.json")
 KERNEL_SOURCES = ("c-attl3_amd/csrc/gemm_kernels.hip", "c-attl3_amd/csrc/gemm_bf16x3.hip", "c-attl3_amd/csrc/gemm_bf16x3.hpp",
                   "c-attl3_amd/csrc/gemm_tiles.hpp", "c-attl3_amd/csrc/gather_epilogue.hpp", "c-attl3_amd/csrc/common.hpp",
-                  "c-attl3_amd/csrc/act_math.hpp", "c-attl3_amd/csrc/lstm_math.hpp", "c-attl3_amd/csrc/few_weights.hpp")
+                  "c-attl3_amd/csrc/act_math.hpp", "c-attl3_amd/csrc/lstm_math.hpp", "c-attl3_amd/csrc/few_weights.hpp",
+                  "c-attl3_amd/csrc/buffer_loads.hpp")
 
 
 def kernel_sources_hash():

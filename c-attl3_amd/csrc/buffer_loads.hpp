@@ -8,7 +8,7 @@
 #include <hip/hip_runtime.h>
 
 namespace cattle_hip {
-namespace loads {
+namespace buffer_loads {
 
 /* A byte offset beyond any buffer (below 2 GiB): such a load returns zero. Loads are to be in range by the lane's own choice between its
  * offset and this one; none counts on the range check for a sum of its two offsets, and the wavefront's alone lies inside the buffer. */
@@ -36,7 +36,7 @@ __device__ __forceinline__ int unit_of(int r, int c) {
 	return r * UNITS + (c ^ (r % UNITS));
 }
 
-} /* namespace loads */
+} /* namespace buffer_loads */
 } /* namespace cattle_hip */
 
 #endif /* CATTLE_HIP_BUFFER_LOADS_HPP_ */

@@ -6,27 +6,17 @@
 #ifndef CATTLE_HIP_FEW_WEIGHTS_HPP_
 #define CATTLE_HIP_FEW_WEIGHTS_HPP_
 
+#include "buffer_loads.hpp"
 #include "gemm_tiles.hpp"
 
 namespace cattle_hip {
 namespace few_weights {
 
-constexpr unsigned OUTSIDE = 0x80000000u;       /* a byte offset beyond any buffer: such a load returns zero */
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int TL = 32, ITEM = 64, HALF = 32, UNITS = HALF / 4, ROWS = 64 / UNITS;
-constexpr int WAVES = 4;        /* of a block, alone and riding: the order of the sums does not depend on which */
+using namespace buffer_loads;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
-	return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int) bytes, 0x00020000);
-}
-__device__ __forceinline__ f32x4 load_4(__amdgpu_buffer_rsrc_t b, unsigned lane_off, unsigned wave_off) {
-	return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, (int) lane_off, (int) wave_off, 0));
-}
-/* Where 16-byte unit c (four samples) of row r lies: shifted by the row, so that the eight rows that a read of 64 lanes takes at a
- * time lie on different banks. */
-__device__ __forceinline__ int unit_of(int r, int c) {
-	return r * UNITS + (c ^ (r % UNITS));
-}
+constexpr int TL = 32, ITEM = 64, HALF = 32, ROWS = 64 / UNITS;
+constexpr int WAVES = 4;        /* of a block, alone and riding: the order of the sums does not depend on which */
+static_assert(UNITS == HALF / 4, "rows of 32 samples");
 
 /* ------------------------------------------------------------------------------------------------
  * partials[slice][K x F] = sum over the slice of x^T og. An item is 64 samples of one output position; a slice is a block, its

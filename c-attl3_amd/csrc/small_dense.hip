@@ -4,28 +4,12 @@
  */
 #include "small_dense.hpp"
 #include "act_math.hpp"
+#include "buffer_loads.hpp"
 
 namespace cattle_hip {
 namespace {
 
-/* A byte offset beyond any buffer: such a load returns zero. Every load below is in range by the lane's own choice between its offset and
- * this one; none counts on the range check for a sum of its two offsets, and the wavefront's alone lies inside the buffer. */
-constexpr unsigned OUTSIDE = 0x80000000u;
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
-	return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int) bytes, 0x00020000);
-}
-__device__ __forceinline__ float load_1(__amdgpu_buffer_rsrc_t b, unsigned lane_off, unsigned wave_off) {
-	return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, (int) lane_off, (int) wave_off, 0));
-}
-__device__ __forceinline__ f32x2 load_2(__amdgpu_buffer_rsrc_t b, unsigned lane_off, unsigned wave_off) {
-	return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(b, (int) lane_off, (int) wave_off, 0));
-}
-__device__ __forceinline__ f32x4 load_4(__amdgpu_buffer_rsrc_t b, unsigned lane_off, unsigned wave_off) {
-	return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, (int) lane_off, (int) wave_off, 0));
-}
+using namespace buffer_loads;
 
 /* ------------------------------------------------------------------------------------------------
  * out[M x F] = x[M x K] wt[K x F] (+ bias, activation). A block owns 16 MB rows and 16 columns, and its wavefronts a contiguous
@@ -268,12 +252,8 @@ void small_product_ordered_kernel(const float* __restrict__ src, const float* __
  * shares; with 32 columns or more, so that no tile is mostly padding (a layer of few outputs has a launch
  * that its input gradient takes along).
  * ---------------------------------------------------------------------------------------------- */
-constexpr int GL = 32, HALF_M = 32, GRAD_WAVES = 8, UNITS = HALF_M / 4;
-/* Where 16-byte unit c (four samples) of row r of an operand's half share lies: shifted by the row, so that the eight rows that a
- * read of 64 lanes takes at a time lie on different banks. */
-__device__ __forceinline__ int unit_of(int r, int c) {
-	return r * UNITS + (c ^ (r % UNITS));
-}
+constexpr int GL = 32, HALF_M = 32, GRAD_WAVES = 8;
+static_assert(UNITS == HALF_M / 4, "rows of 32 samples");
 /* HALVES: 32 samples each that a wavefront takes */
 template<bool ACT, int HALVES>
 __global__ __launch_bounds__(64 * GRAD_WAVES)

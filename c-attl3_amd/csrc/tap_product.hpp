@@ -5,6 +5,7 @@
 #ifndef CATTLE_HIP_TAP_PRODUCT_HPP_
 #define CATTLE_HIP_TAP_PRODUCT_HPP_
 
+#include "buffer_loads.hpp"
 #include "gemm_tiles.hpp"
 
 #include <algorithm>
@@ -13,10 +14,11 @@
 namespace cattle_hip {
 namespace tap_product {
 
+using namespace buffer_loads;
+
 typedef Mfma<float>::acc_t acc_t;
 constexpr int TAPS = 9;
 constexpr int TL = Mfma<float>::TL;
-constexpr unsigned OUTSIDE = 0x80000000u;       /* a byte offset beyond any buffer: such a load returns zero */
 
 /* n / d for n < 2^31: the host's multiplier in place of a division's two dozen instructions (Granlund and Montgomery, 1994) */
 struct Divisor { unsigned mul, shift; };
@@ -69,13 +71,6 @@ __host__ __device__ __forceinline__ bool row_inside(const GatherGeom& g, int a, 
 }
 __host__ __device__ __forceinline__ bool column_inside(const GatherGeom& g, int b, int s) {
 	return (unsigned) (b + g.PB + s * g.RB) < (unsigned) g.LW;
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
-	return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int) bytes, 0x00020000);
-}
-__device__ __forceinline__ float load_f32(__amdgpu_buffer_rsrc_t b, unsigned lane_off, unsigned wave_off) {
-	return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, (int) lane_off, (int) wave_off, 0));
 }
 
 /* The row m of this lane as sample and position. */
@@ -131,8 +126,8 @@ __device__ __forceinline__ acc_t share_of_product(const float* __restrict__ src,
 				#pragma unroll
 				for (int i = 0; i < SPC; ++i) {
 					const bool last = ODD && i == SPC - 1;
-					x[j * SPC + i] = load_f32(src_buf, last && missing ? OUTSIDE : lane_off, a_tap + (unsigned) i * a_pair);
-					w[j * SPC + i] = load_f32(wt_buf, last && missing ? OUTSIDE : b_lane, b_wave + wt_tap(g, t) + (unsigned) i * b_pair);
+					x[j * SPC + i] = load_1(src_buf, last && missing ? OUTSIDE : lane_off, a_tap + (unsigned) i * a_pair);
+					w[j * SPC + i] = load_1(wt_buf, last && missing ? OUTSIDE : b_lane, b_wave + wt_tap(g, t) + (unsigned) i * b_pair);
 				}
 			}
 		}
