@@ -129,6 +129,10 @@ __device__ __forceinline__ acc_t share_of_product(const float* __restrict__ src,
 					x[j * SPC + i] = load_1(src_buf, last && missing ? OUTSIDE : lane_off, a_tap + (unsigned) i * a_pair);
 					w[j * SPC + i] = load_1(wt_buf, last && missing ? OUTSIDE : b_lane, b_wave + wt_tap(g, t) + (unsigned) i * b_pair);
 				}
+				/* in the order of the products: left alone, the compiler issues the last channel's loads behind all others (both passes of
+				 * 65,536 x 27 x 16 20.5 us, 19.7 this way) */
+				if constexpr (ODD)
+					__builtin_amdgcn_sched_barrier(0);
 			}
 		}
 		__builtin_amdgcn_sched_barrier(0);
