@@ -32,7 +32,7 @@ EXPORTS = [
     "cattle_hip_timer_destroy", "cattle_hip_timer_start", "cattle_hip_timer_stop", "cattle_hip_conv_create",
     "cattle_hip_transconv_create", "cattle_hip_dense_create", "cattle_hip_batchnorm_create", "cattle_hip_batchnorm_get_stats_initialized",
     "cattle_hip_batchnorm_set_stats_initialized", "cattle_hip_activation_create", "cattle_hip_pool_create",
-    "cattle_hip_convlstm_set_multiplicative_integration", "cattle_hip_convlstm_fused_steps", "cattle_hip_last_products", "cattle_hip_layer_param_set_regularization",
+    "cattle_hip_convlstm_set_multiplicative_integration", "cattle_hip_convlstm_fused_steps", "cattle_hip_last_products", "cattle_hip_last_launches", "cattle_hip_layer_param_set_regularization",
     "cattle_hip_layer_param_regularization_penalty", "cattle_hip_dropout_create", "cattle_hip_reshape_create", "cattle_hip_broadcast_create",
     "cattle_hip_layer_keep_sum_order", "cattle_hip_layer_clone", "cattle_hip_layer_destroy", "cattle_hip_layer_input_dims",
     "cattle_hip_layer_output_dims", "cattle_hip_layer_is_input_layer", "cattle_hip_layer_set_input_layer",
@@ -241,10 +241,17 @@ def conv_forward_noalloc(x, weights, bias, out, receptor_height=3, receptor_widt
 
 def last_products():
     """(product, weight gradient): rows * 1000 + columns of the tile that the last forward or input-gradient product and the
-    last weight gradient of a kernel layer took on the bf16 matrix instructions, a negative number for the fp32 launches without tiles
-    (-1 small dense, -2 small dense in the tiled order of sums, -3 few channels, -4 few weights), 0 for all others."""
+    last weight gradient of a kernel layer took on the bf16 matrix instructions, 0 where they ran on others."""
     p, w = ctypes.c_int(), ctypes.c_int()
     _check(lib().cattle_hip_last_products(ctypes.byref(p), ctypes.byref(w)))
+    return int(p.value), int(w.value)
+
+
+def last_launches():
+    """(product, weight gradient): which of the fp32 launches without tiles the same two were: 1 small dense, 2 small dense in the
+    tiled order of sums, 3 few channels, 4 few weights, 0 any other launch."""
+    p, w = ctypes.c_int(), ctypes.c_int()
+    _check(lib().cattle_hip_last_launches(ctypes.byref(p), ctypes.byref(w)))
     return int(p.value), int(w.value)
 
 

@@ -94,9 +94,10 @@ struct ConvShape {
 	int K() const { return RH * RW * C; }
 };
 
-/* What the last launches of a kernel layer ran on (cattle_hip_last_products): rows * 1000 + columns of the tile on the bf16
- * instructions, one of these where it was one of the fp32 launches without tiles, 0 for all others. */
-enum { RAN_SMALL_DENSE = -1, RAN_SMALL_DENSE_ORDERED = -2, RAN_FEW_CHANNELS = -3, RAN_FEW_WEIGHTS = -4 };
+/* What the last launches of a kernel layer ran on: rows * 1000 + columns of the tile on the bf16 instructions
+ * (cattle_hip_last_products), one of these, negative, where it was one of the fp32 launches without tiles (cattle_hip_last_launches),
+ * 0 for all others. */
+enum { RAN_SMALL_DENSE = 1, RAN_SMALL_DENSE_ORDERED = 2, RAN_FEW_CHANNELS = 3, RAN_FEW_WEIGHTS = 4 };
 struct LastProducts { int product = 0, weight_gradient = 0; };
 extern LastProducts g_last_products;
 

@@ -2278,7 +2278,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 		if constexpr (std::is_same<T, float>::value)
 			if ((epi == EPI_NONE || epi == EPI_ACT) && then == nullptr && !g.keeps_sums && small_product_possible(g, device_shape().cus)) {
 				small_product(src, wt, bias, out, g, round_up(g.K, WT_ROW_PAD), epi == EPI_ACT ? E : nullptr, device_shape().cus);
-				g_last_products.product = RAN_SMALL_DENSE;
+				g_last_products.product = -RAN_SMALL_DENSE;
 				return true;
 			}
 		return false;
@@ -2489,7 +2489,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 	if constexpr (std::is_same<T, float>::value)
 		if (chosen == &vars[best_v] && !rider && epi == EPI_NONE && then == nullptr && !g.keeps_sums && !g.fp32_products && few_channels_possible(g, device_shape().cus)) {
 			few_channels_product(src, wt, bias, out, g);
-			g_last_products.product = RAN_FEW_CHANNELS;
+			g_last_products.product = -RAN_FEW_CHANNELS;
 			if (mtiles_out)
 				*mtiles_out = 0;
 			return true;
@@ -2576,7 +2576,7 @@ bool launch_gather(const T* src, const T* wt, const T* bias, T* out, const Gathe
 			if constexpr (std::is_same<T, float>::value)
 				if (tail != WS_LSTM_BACKWARD && addressable_product(g)) {
 					small_product_ordered(src, wt, bias, out, g, round_up(g.K, WT_ROW_PAD), epi == EPI_ACT ? E : nullptr, waves);
-					g_last_products.product = RAN_SMALL_DENSE_ORDERED;
+					g_last_products.product = -RAN_SMALL_DENSE_ORDERED;
 					return true;
 				}
 			if (waves == 16)
@@ -3327,7 +3327,7 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 			T p0, p1;
 			negative_side(act, &p0, &p1);
 			small_weight_gradient(x, out_grad, wgrad, bgrad, g, act, p0, p1, fresh);
-			g_last_products.weight_gradient = RAN_SMALL_DENSE;
+			g_last_products.weight_gradient = -RAN_SMALL_DENSE;
 			return;
 		}
 	auto run = [&](T* to_w, T* to_b, const WgradSplit& how) {
@@ -3351,7 +3351,7 @@ void conv_weight_gradient_with(const ConvShape& s, int N, const T* x, const T* o
 				WgradRider<T> rider = { x, out_grad, to_w, to_b, g, how, false, &problem };
 				if (!elsewhere || !(*elsewhere)(rider))
 					few_weights_gradient(problem);
-				g_last_products.weight_gradient = RAN_FEW_WEIGHTS;
+				g_last_products.weight_gradient = -RAN_FEW_WEIGHTS;
 				return;
 			}
 		if constexpr (std::is_same<T, float>::value)
@@ -3407,7 +3407,7 @@ bool conv_weight_gradient_transposed(const ConvShape& s, int N, const T* x, cons
 			return false;
 		const int slices = few_weights_slices(g, p.splits);
 		few_weights_gradient(few_weights_problem(x, out_grad, partials, nullptr, g, slices, true));
-		g_last_products.weight_gradient = RAN_FEW_WEIGHTS;
+		g_last_products.weight_gradient = -RAN_FEW_WEIGHTS;
 		const size_t count = (size_t) g.K * g.F;
 		deferred->count = 1;
 		deferred->e[0] = ReduceEntry<T>{ partials, wgrad_t, count, slices, 0, count <= 8192 && slices >= 32,

@@ -2513,8 +2513,16 @@ int cattle_hip_convlstm_fused_steps(cattle_hip_layer_t lstm, int* forward_steps,
 int cattle_hip_last_products(int* product, int* weight_gradient) {
 	return guarded([&] {
 		CATTLE_HIP_REQUIRE(product != nullptr && weight_gradient != nullptr, "null output pointer");
-		*product = g_last_products.product;
-		*weight_gradient = g_last_products.weight_gradient;
+		*product = std::max(0, g_last_products.product);
+		*weight_gradient = std::max(0, g_last_products.weight_gradient);
+	});
+}
+
+int cattle_hip_last_launches(int* product, int* weight_gradient) {
+	return guarded([&] {
+		CATTLE_HIP_REQUIRE(product != nullptr && weight_gradient != nullptr, "null output pointer");
+		*product = std::max(0, -g_last_products.product);
+		*weight_gradient = std::max(0, -g_last_products.weight_gradient);
 	});
 }
 

@@ -449,10 +449,11 @@ int cattle_hip_convlstm_set_multiplicative_integration(cattle_hip_layer_t lstm, 
 int cattle_hip_convlstm_fused_steps(cattle_hip_layer_t lstm, int* forward_steps, int* backward_steps);
 /* Which matrix instructions the last kernel layer's launches ran on (no counterpart in the reference; for tests and profiles):
  * *product for the last forward or input-gradient product, *weight_gradient for the last weight gradient - the tile's rows *
- * 1000 + its columns where it multiplied on the bf16 instructions, a negative number where it was one of the fp32 launches without
- * tiles (-1 a small dense layer's, -2 the same in the tiled launches' order of sums, -3 a 3 x 3 convolution of few channels, -4 a weight
- * gradient of few weights), 0 where anything else. */
+ * 1000 + its columns where it multiplied on the bf16 instructions, 0 where on others. */
 int cattle_hip_last_products(int* product, int* weight_gradient);
+/* Which of the fp32 launches without tiles the same two were: 1 a small dense layer's, 2 the same in the tiled launches' order of sums,
+ * 3 a 3 x 3 convolution of few channels, 4 a weight gradient of few weights, 0 any other launch. */
+int cattle_hip_last_launches(int* product, int* weight_gradient);
 
 #ifdef __cplusplus
 }

@@ -16,7 +16,7 @@ ch = importlib.import_module("c-attl3_amd")
 # N, H, W, C, F, pv, ph, dv, dh
 CASES = [(64, 32, 32, 3, 16, 1, 1, 0, 0), (1, 5, 6, 1, 9, 1, 1, 0, 0), (33, 9, 7, 2, 33, 0, 0, 0, 0), (7, 12, 10, 5, 40, 2, 1, 1, 0), (32, 8, 8, 6, 64, 3, 4, 2, 3),
          (40, 10, 9, 12, 4, 1, 1, 0, 0), (5, 11, 8, 17, 6, 0, 2, 0, 1), (33, 10, 9, 12, 4, 1, 1, 0, 0)]
-FEW_CHANNELS = -3       # ch.last_products(): the launch that these cases are meant for
+FEW_CHANNELS = 3        # ch.last_launches(): the launch that these cases are meant for
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(str(v) for v in c))
@@ -33,10 +33,10 @@ def test_convolutions_of_few_channels(case):
     wp.set_values(w)
     bp.set_values(b)
     out = layer.pass_forward(ch.DeviceTensor.from_host(x), True).to_host()
-    assert (ch.last_products()[0] == FEW_CHANNELS) == (C <= 6)
+    assert (ch.last_launches()[0] == FEW_CHANNELS) == (C <= 6)
     dx = layer.pass_back(ch.DeviceTensor.from_host(g)).to_host()
     # the input gradients of few filters, where no weight gradient rides in their launch (it does at a multiple of four samples)
-    assert (ch.last_products()[0] == FEW_CHANNELS) == (F <= 6 and N % 4 != 0)
+    assert (ch.last_launches()[0] == FEW_CHANNELS) == (F <= 6 and N % 4 != 0)
     geom = dict(RH=3, RW=3, pv=pv, ph=ph, sv=1, sh=1, dv=dv, dh=dh)
     x64, w64, b64, g64 = (np.asarray(a, np.float64) for a in (x, w, b, g))
     ref, cache = oracle.conv_forward(x64, w64, b64, return_cache=True, **geom)

@@ -32,7 +32,7 @@ def test_gradients_of_few_weights(case):
     wp.set_values(w)
     layer.pass_forward(ch.DeviceTensor.from_host(x), True)
     layer.pass_back(ch.DeviceTensor.from_host(g))
-    assert ch.last_products()[1] == -4          # the launch that these cases are meant for, alone or in that of the input gradient
+    assert ch.last_launches()[1] == 4          # the launch that these cases are meant for, alone or in that of the input gradient
     geom = dict(RH=RH, RW=RW, pv=pv, ph=ph, sv=sv, sh=sh, dv=dv, dh=dh)
     x64, w64, g64, b64 = (np.asarray(a, np.float64) for a in (x, w, g, np.zeros((1, F))))
     _, cache = oracle.conv_forward(x64, w64, b64, return_cache=True, **geom)

@@ -19,7 +19,7 @@ CASES = [(1, 32, 1000), (2, 33, 17), (15, 61, 40), (16, 64, 16), (17, 100, 130),
          (255, 500, 513), (4, 3072, 48), (60, 35, 32), (64, 31, 64), (68, 96, 100), (508, 40, 36), (512, 33, 700), (512, 600, 96)]
 
 
-SMALL, SMALL_ORDERED = -1, -2       # ch.last_products(): the launches that these cases are meant for
+SMALL, SMALL_ORDERED = 1, 2       # ch.last_launches(): the launches that these cases are meant for
 # in front of a rectifier (the sums keep the order of the tiled launches): the others are few tiles of few reduction indices, or whole tiles
 ORDERED = [(17, 100, 130), (31, 1000, 9), (256, 784, 512), (255, 500, 513), (512, 600, 96)]
 
@@ -44,12 +44,12 @@ def test_small_dense_layers(case, act):
     bp.set_values(b)
     (layer,) = ch.fuse_layers([dense] + ([ch.ActivationLayer(np.float32, act, (F,), 0.5)] if act else []))
     y = layer.pass_forward(ch.DeviceTensor.from_host(x), True).to_host()
-    assert (ch.last_products()[0] == SMALL_ORDERED) == bool(act and case in ORDERED)
-    assert (ch.last_products()[0] == SMALL) == bool(not act and K >= 32)
+    assert (ch.last_launches()[0] == SMALL_ORDERED) == bool(act and case in ORDERED)
+    assert (ch.last_launches()[0] == SMALL) == bool(not act and K >= 32)
     dx = layer.pass_back(ch.DeviceTensor.from_host(g)).to_host()
     if act or case == (256, 784, 512):      # (the others' weight gradients are one-wavefront tiles that ride with the input gradient)
-        assert (ch.last_products()[0] == SMALL) == (F >= 32)
-        assert (ch.last_products()[1] == SMALL) == (F >= 32 and N % 4 == 0)
+        assert (ch.last_launches()[0] == SMALL) == (F >= 32)
+        assert (ch.last_launches()[1] == SMALL) == (F >= 32 and N % 4 == 0)
     dw, db = wp.get_grad(), bp.get_grad()
     x64, w64, g64 = (np.asarray(a, np.float64) for a in (x, w, g))
     z = x64 @ w64 + b
